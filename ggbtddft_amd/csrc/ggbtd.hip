@@ -14,8 +14,9 @@
 //
 // Kernels, launch order per step:
 //   k_angular<mode 0>   Vh, Le, Lo                       grid (N / 8 NT, C)
-//   k_kin_fwd(_tiled)   Y = e^{-i lam dt} Q^T psi        grid (nk/16, 2C/16, n_l) or 64 x 128 tiles
-//   k_kin_bwd(_tiled)   psi = Q Y                        grid (N/16,  2C/16, n_l) or 64 x 128 tiles
+//   k_kin64<0>          Y = e^{-i lam dt} Q^T psi (FP64) grid (nk/32, 2C/32, n_l)
+//   k_kin64<1>          psi = Q Y                        grid (N/32,  2C/32, n_l)
+//   (mixed form: k_kin_fwd / k_kin_bwd, 16-wide tiles, or k_kin_*_dma / _tiled, 64 x 128 tiles)
 //   k_angular<mode 1>   Lo, Le, Vh, |B psi|^2, observable partials
 //   k_rho               rho_u = sum occ |Psi|^2, v_xc; observable sums
 //   k_tile_gemm<Qmom>   multipole moments q_L = P_L^T rho_u
@@ -147,12 +148,12 @@ struct KinRef {
 
 // whether any instance with a column among real columns [n0, n0 + nreal) is
 // in use (work-group-uniform; idle serving slots skip their kinetic tiles)
-static __device__ __forceinline__ bool kin_cols_active(const KinRef &kr, int n0, int nreal, int C,
+static __device__ __forceinline__ bool kin_cols_active(const int32_t *active, int n0, int nreal, int C,
                                                        int n_orb) {
-    if (!kr.active) return true;
+    if (!active) return true;
     const int c0 = n0 >> 1, c1 = min(C, (n0 + nreal + 1) >> 1);
     for (int q = c0 / n_orb; q * n_orb < c1; ++q)
-        if (kr.active[q]) return true;
+        if (active[q]) return true;
     return false;
 }
 __global__ __launch_bounds__(WG) void k_kin_ref(const double *__restrict__ psi,
@@ -228,78 +229,70 @@ static __device__ __forceinline__ const double *kin_ref_row(const KinRef &kr, in
 }
 
 // ---------------------------------------------------------------------------
-// Kinetic propagator, pass 1: Y[l][c][p][a] = (e^{-i lam_a dt} sum_i Q[l][i][a] psi[l][c][i])_p
+// Mixed form, narrow passes (few columns).
+// Pass 1: Y[l][c][p][a] = (e^{-i lam_a dt} sum_i Q[l][i][a] psi[l][c][i])_p
 // M = eigen index a, N = real column (c, p = re/im), K = radial node i.
 // One work-group computes 16 TA x 16 outputs; its NW waves take equal shares
 // of K (more loads in flight per CU than one wave per tile), then the partial
 // tiles are added in fixed order through LDS.  Y is planar in (re, im)
-// so that pass 2 reads contiguous runs of a.  T is the compute type (tables
-// and Y in T, state in FP64, phase in FP64).
+// so that pass 2 reads contiguous runs of a (tables and Y in FP32, state and
+// phase in FP64).
 // ---------------------------------------------------------------------------
 #ifndef KIN_KU
 #define KIN_KU 2
 #endif
 #define KU KIN_KU
-// waves per work-group of the narrow passes (K split over them): 4 in FP64, 8
-// in the mixed form, whose FP32 pass 1 takes 17.8 instead of 19.7 us at argon
-// size with 8 (FP64: 22.6 against 22.1 us)
+// waves per work-group of the narrow passes (K split over them): with 8 the
+// pass 1 takes 17.8 instead of 19.7 us at argon size
 #ifndef KIN_NW
-#define KIN_NW 4
-#endif
-#ifndef KIN_NW32
-#define KIN_NW32 8
+#define KIN_NW 8
 #endif
 // waves 0..3 finish accumulator rows 0..3 of every tile after the K split
-static_assert(KIN_NW >= 4 && KIN_NW <= 16 && KIN_NW32 >= 4 && KIN_NW32 <= 16, "4 to 16 waves per narrow work-group");
-template <typename T>
-struct kin_nw {
-    static constexpr int value = mfma_t<T>::mixed ? KIN_NW32 : KIN_NW;
-};
-#define KIN_WG_MAX (64 * (KIN_NW > KIN_NW32 ? KIN_NW : KIN_NW32))
+static_assert(KIN_NW >= 4 && KIN_NW <= 16, "4 to 16 waves per narrow work-group");
+#define KIN_NARROW_WG (64 * KIN_NW)
 // Panel form: one work-group takes the 16 TA eigen rows a0 .. a0 + 16 TA - 1 as
 // TA tiles with interleaved rows (row ar of tile t is a = a0 + TA ar + t).  A
 // lane reads its TA table values of a K row as one vector, the 16 lanes of the
 // row read one run of 16 TA values, and each state load feeds TA products.
 // Every tile keeps the K split, the product order and the fixed-order LDS sum
 // of one tile per work-group, so the result does not depend on TA.  TA = 2
-// takes an argon FP64 pass from 25.4 to 22.9 us (FP32 22.8 to 20.7); TA = 4
-// is no faster in FP64 and slower in FP32.
+// takes an argon pass from 22.8 to 20.7 us; TA = 4 is slower.
 #ifndef KIN_TA
 #define KIN_TA 2
 #endif
 static_assert(KIN_TA == 1 || KIN_TA == 2 || KIN_TA == 4, "KIN_TA: 1, 2 or 4 (a divisor of 16)");
-template <typename T, int TA>
-__global__ __launch_bounds__(KIN_WG_MAX) void k_kin_fwd(const T *__restrict__ Q,
+template <int TA>
+__global__ __launch_bounds__(KIN_NARROW_WG) void k_kin_fwd(const float *__restrict__ Q,
                                                 const double2 *__restrict__ kph,
                                                 const int32_t *__restrict__ nkeep,
                                                 const double *__restrict__ psi, KinRef ref,
-                                                T *__restrict__ Y, int N, int nk_max, int C,
+                                                float *__restrict__ Y, int N, int nk_max, int C,
                                                 int n_orb) {
-    typedef typename mfma_t<T>::v4 v4;
-    typedef T vta __attribute__((ext_vector_type(TA)));
-    constexpr int NW = kin_nw<T>::value;
+    typedef typename mfma_t<float>::v4 v4;
+    typedef float vta __attribute__((ext_vector_type(TA)));
+    constexpr int NW = KIN_NW;
     __shared__ double red[NW][TA][64][4];
     const tile3 tb = xcd_tile();  // (eigen panel, column tile, l): panels of one l share psi
     const int l = tb.z;
     const int nk = nkeep[l];
     const int a0 = tb.x * 16 * TA;
     if (a0 >= nk) return;  // block-uniform
-    if (!kin_cols_active(ref, tb.y * 16, 16, C, n_orb)) return;  // idle instances only
+    if (!kin_cols_active(ref.active, tb.y * 16, 16, C, n_orb)) return;  // idle instances only
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int kr = lane >> 4, lc = lane & 15;
     const int col = tb.y * 16 + lc;
     const int c = col >> 1, p = col & 1;
     const bool colok = c < C;
-    const T *Ql = Q + (size_t)l * N * nk_max + a0 + TA * lc;
+    const float *Ql = Q + (size_t)l * N * nk_max + a0 + TA * lc;
     const bool lv = a0 + TA * lc < nk;  // interleaved rows: this lane's TA rows hold some a < nkeep
     const double *Xl = psi + ((size_t)l * C + (colok ? c : 0)) * N * 2 + p;
     const int kq = (((N + NW - 1) / NW + 3) / 4) * 4;  // K share of a wave, multiple of 4
     const int kb = wave * kq, ke = min(N, kb + kq);
     double rc = 0.0;
-    const double *rrow = (mfma_t<T>::mixed && colok) ? kin_ref_row(ref, l, c, p, N, n_orb, false, &rc) : nullptr;
+    const double *rrow = colok ? kin_ref_row(ref, l, c, p, N, n_orb, false, &rc) : nullptr;
     // wave w < 4 finishes accumulator row w of every tile: its phase factors
     // are loaded ahead of the products
-    const int ar = mfma_t<T>::row(kr, wave & 3);
+    const int ar = mfma_t<float>::row(kr, wave & 3);
     double2 kp[TA];
     if (wave < 4) {
 #pragma unroll
@@ -312,13 +305,13 @@ __global__ __launch_bounds__(KIN_WG_MAX) void k_kin_fwd(const T *__restrict__ Q,
 #pragma unroll
     for (int t = 0; t < TA; ++t) acc[t] = v4{0, 0, 0, 0};
     for (int k0 = kb; k0 < ke; k0 += 4 * KU) {
-        T av[KU][TA], bv[KU];
+        float av[KU][TA], bv[KU];
 #pragma unroll
         for (int u = 0; u < KU; ++u) {
             const int i = k0 + 4 * u + kr;
             const bool ok = i < ke;
 #pragma unroll
-            for (int t = 0; t < TA; ++t) av[u][t] = (T)0;
+            for (int t = 0; t < TA; ++t) av[u][t] = 0.f;
             if (ok && lv) {
                 const vta q = *reinterpret_cast<const vta *>(Ql + (size_t)i * nk_max);
 #pragma unroll
@@ -326,12 +319,12 @@ __global__ __launch_bounds__(KIN_WG_MAX) void k_kin_fwd(const T *__restrict__ Q,
             }
             double x = (ok && colok) ? Xl[(size_t)i * 2] : 0.0;
             if (rrow && ok) x -= rc * rrow[i];
-            bv[u] = (T)x;
+            bv[u] = (float)x;
         }
 #pragma unroll
         for (int u = 0; u < KU; ++u)
 #pragma unroll
-            for (int t = 0; t < TA; ++t) acc[t] = mfma_t<T>::op(av[u][t], bv[u], acc[t]);
+            for (int t = 0; t < TA; ++t) acc[t] = mfma_t<float>::op(av[u][t], bv[u], acc[t]);
     }
     // partial tiles through LDS (wave 0's in the last slot); wave w < 4 then finishes
     // accumulator row r = w of every tile, so the four epilogues run side by side
@@ -348,7 +341,7 @@ __global__ __launch_bounds__(KIN_WG_MAX) void k_kin_fwd(const T *__restrict__ Q,
         for (int w = 0; w < NW - 1; ++w) v += red[w][t][lane][r];
         const double vo = lane_xor1(v);
         const int a = a0 + TA * ar + t;
-        const T o = kin_factor<T>(v, vo, p, kp[t]);
+        const float o = kin_factor<float>(v, vo, p, kp[t]);
         if (colok && a < nk) Y[(((size_t)l * C + c) * 2 + p) * nk_max + a] = o;
     }
 }
@@ -371,20 +364,19 @@ static __host__ __device__ __forceinline__ size_t kin_qt_index(size_t l, size_t 
 #define KIN_KU2 2
 #endif
 #define KU2 KIN_KU2
-template <typename T>
-__global__ __launch_bounds__(KIN_WG_MAX) void k_kin_bwd(const T *__restrict__ QT,
+__global__ __launch_bounds__(KIN_NARROW_WG) void k_kin_bwd(const float *__restrict__ QT,
                                                 const int32_t *__restrict__ nkeep,
-                                                const T *__restrict__ Y, KinRef ref,
+                                                const float *__restrict__ Y, KinRef ref,
                                                 double *__restrict__ psi, int N, int nk_max,
                                                 int C, int n_orb) {
-    typedef typename mfma_t<T>::v4 v4;
-    constexpr int NW = kin_nw<T>::value;
+    typedef typename mfma_t<float>::v4 v4;
+    constexpr int NW = KIN_NW;
     __shared__ double red[NW][64][4];
     const tile3 tb = xcd_tile();  // (radial tile, column tile, l): tiles of one l share Y
     const int l = tb.z;
     const int nk = nkeep[l];
     const int kend = min(nk_max, (nk + 15) & ~15);
-    if (!kin_cols_active(ref, tb.y * 16, 16, C, n_orb)) return;  // idle instances only
+    if (!kin_cols_active(ref.active, tb.y * 16, 16, C, n_orb)) return;  // idle instances only
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int i0 = tb.x * 16;
     const int kr = lane >> 4, lc = lane & 15;
@@ -394,18 +386,18 @@ __global__ __launch_bounds__(KIN_WG_MAX) void k_kin_bwd(const T *__restrict__ QT
     const int im_ = i0 + lc;
     // the transposed table, quad-interleaved (kin_qt_index): a lane's four
     // consecutive a (one K group of its MFMAs) are one vector, and the 16 lanes
-    // of a row read 16 consecutive i (a 256- or 512-byte run).  Against the
-    // plain transpose (four scalar loads per K group) it takes 21.1 instead of
-    // 24.2 us per FP64 argon pass (13.7 instead of 15.3 in FP32).
-    const T *Qc = QT + kin_qt_index(l, im_ < N ? im_ : 0, 4 * kr, N, nk_max);
-    const T *Yr = Y + (((size_t)l * C + (colok ? c : 0)) * 2 + p) * nk_max + 4 * kr;
+    // of a row read 16 consecutive i (a 256-byte run).  Against the plain
+    // transpose (four scalar loads per K group) it takes 13.7 instead of
+    // 15.3 us per argon pass.
+    const float *Qc = QT + kin_qt_index(l, im_ < N ? im_ : 0, 4 * kr, N, nk_max);
+    const float *Yr = Y + (((size_t)l * C + (colok ? c : 0)) * 2 + p) * nk_max + 4 * kr;
     const int kq = (((kend + 15) / 16 + NW - 1) / NW) * 16;  // K share of a wave, multiple of 16
     const int kb = wave * kq, ke = min(kend, kb + kq);
     // wave w < 4 finishes accumulator row w: the mixed form's ground-state term
     // of that element is loaded ahead of the products
-    const int io = i0 + mfma_t<T>::row(kr, wave & 3);
+    const int io = i0 + mfma_t<float>::row(kr, wave & 3);
     double rc = 0.0, rv = 0.0;
-    const double *rrow = (mfma_t<T>::mixed && colok && wave < 4) ? kin_ref_row(ref, l, c, p, N, n_orb, true, &rc) : nullptr;
+    const double *rrow = (colok && wave < 4) ? kin_ref_row(ref, l, c, p, N, n_orb, true, &rc) : nullptr;
     if (rrow) rv = rrow[io < N ? io : 0];
     v4 acc = {0, 0, 0, 0};
     for (int k0 = kb; k0 < ke; k0 += 16 * KU2) {
@@ -423,7 +415,7 @@ __global__ __launch_bounds__(KIN_WG_MAX) void k_kin_bwd(const T *__restrict__ QT
 #pragma unroll
         for (int u = 0; u < KU2; ++u)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc = mfma_t<T>::op(av[u][j], bv[u][j], acc);
+            for (int j = 0; j < 4; ++j) acc = mfma_t<float>::op(av[u][j], bv[u][j], acc);
     }
     // partial tiles through LDS (wave 0's in the last slot); wave w < 4 then finishes
     // accumulator row r = w, so the four epilogues run side by side
@@ -442,10 +434,216 @@ __global__ __launch_bounds__(KIN_WG_MAX) void k_kin_bwd(const T *__restrict__ QT
 }
 
 // ---------------------------------------------------------------------------
-// Tiled kinetic passes for many columns (instances sharing the tables).
+// FP64 kinetic passes.  Both are one product per l, D[c][m] = sum_k A[k][m] B[c][k]
+// with a real table A and complex columns B:
+//   PASS 0: A = Q[l] (k = radial node, m = eigen index), B = psi, and D = Y gets
+//           the factor e^{-i lam dt};
+//   PASS 1: A = QT[l], the plain transpose with rows padded to np = a multiple
+//           of 16 (k = eigen index, m = radial node), B = Y, D = psi.
+// A work-group takes a panel of 16 TA rows m (as TA tiles with interleaved rows:
+// row 4 r + kr of tile t is m0 + TA (4 r + kr) + t) by TB tiles of 16 real columns
+// (8 complex ones); its K64_NW waves take equal shares of k and add their
+// partial tiles in fixed order through LDS.  No tile is staged: every wave loads
+// its operands straight into registers, one block of 8 k ahead of the products
+// on the block before.
+//  * A lane reads its TA table values of a row k as 16-byte vectors, and each value
+//    feeds TB products; each column value feeds TA.
+//  * Columns are read as whole complex values: in a block of 8 k, lane (kr, c, p)
+//    loads k = k0 + 2 kr + p, and the two lanes of a column swap halves, so that the
+//    first K step multiplies the even k and the second the odd ones.  A wave's load
+//    covers whole 128-byte lines; component-wise loads touched each line twice.
+// What bounds it: HBM up to about 16 columns (the table is read once), the FP64
+// matrix pipe beyond.  At argon size (N = 512, 65 l) passes 0 / 1 take, against the
+// LDS-tiled kernels that ran from 9 columns on: 14 columns 28 / 26 us (91 / 122),
+// 28 columns 45 / 43 us (94 / 124), 224 columns 237 / 234 us (369 / 349, 53 TFLOP/s);
+// krypton (N = 768, 97 l, 13 columns) 91 / 88 us (258 / 293).
+// ---------------------------------------------------------------------------
+#define K64_NW 4
+#define K64_WG (64 * K64_NW)
+typedef double d2_t __attribute__((ext_vector_type(2)));
+struct Kin64Args {
+    const double *A;       // PASS 0: Q [l][N][nk_max], PASS 1: QT [l][nk_max][np]
+    const double2 *B;      // PASS 0: psi [l][C][N], PASS 1: Y [l][C][nk_max]
+    double2 *D;            // PASS 0: Y, PASS 1: psi
+    const double2 *kph;    // [l][nk_max] (cos, sin)(lam dt)
+    const int32_t *nkeep;  // [l]
+    const int32_t *active;
+    int N, nk_max, np, C, n_orb;
+};
+
+template <int PASS, int TA, int TB>
+static __device__ __forceinline__ void kin64_tiles(const Kin64Args &g, int l, int nk, int m0, int n0,
+                                                   double (*red)[TA][64][4]) {
+    constexpr int NW = K64_NW;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int kr = lane >> 4, lc = lane & 15, p = lc & 1;
+    const int C = g.C;
+    const int nk8 = (nk + 7) & ~7;                // <= nk_max (a multiple of 16)
+    const int K = PASS ? nk8 : g.N;
+    const int lda = PASS ? g.np : g.nk_max;       // row length of A, a multiple of 16
+    const int rowsA = PASS ? g.nk_max : g.N, ldb = rowsA, ldd = PASS ? g.N : g.nk_max;
+    // panel rows past the row length read its first rows: their outputs are not stored
+    const double *Al = g.A + (size_t)l * rowsA * lda + (m0 + TA * lc < lda ? m0 + TA * lc : 0);
+    int c[TB];
+    const double2 *Bl[TB];
+#pragma unroll
+    for (int q = 0; q < TB; ++q) {
+        c[q] = (n0 + 16 * q + lc) >> 1;           // columns c >= C read column 0 and are not stored
+        Bl[q] = g.B + ((size_t)l * C + (c[q] < C ? c[q] : 0)) * ldb;
+    }
+    // wave w < 4 finishes accumulator row r = w of every tile: this lane then
+    // holds rows mr .. mr + TA - 1, and stores the complex rows mr + p TA / 2 ..;
+    // their phase factors are loaded ahead of the products
+    const int mr = m0 + TA * mfma_t<double>::row(kr, wave & 3);
+    double2 kp[TA / 2];
+    if (PASS == 0 && wave < 4) {
+#pragma unroll
+        for (int t = 0; t < TA / 2; ++t) {
+            const int m = mr + t + p * (TA / 2);
+            kp[t] = g.kph[(size_t)l * g.nk_max + (m < nk ? m : 0)];
+        }
+    }
+    d4_t acc[TB][TA];
+#pragma unroll
+    for (int q = 0; q < TB; ++q)
+#pragma unroll
+        for (int t = 0; t < TA; ++t) acc[q][t] = (d4_t){0.0, 0.0, 0.0, 0.0};
+    double av[2][2][TA];
+    double2 bv[2][TB];
+    const int kq = (((K + NW - 1) / NW + 7) / 8) * 8;  // K share of a wave, multiple of 8
+    const int kb = wave * kq, ke = min(K, kb + kq);
+    // block of 8 k into buffer b; guard: rows k >= ke read an in-range row and
+    // count as zero through the table operand
+    auto load = [&](int b, int k0, bool guard) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int k = k0 + 2 * kr + h;
+            const double *ap = Al + (size_t)(guard ? min(k, K - 1) : k) * lda;
+#pragma unroll
+            for (int t = 0; t < TA; t += 2) {
+                const d2_t v = *reinterpret_cast<const d2_t *>(ap + t);
+                av[b][h][t] = (guard && k >= ke) ? 0.0 : v[0];
+                av[b][h][t + 1] = (guard && k >= ke) ? 0.0 : v[1];
+            }
+        }
+        const int kk = k0 + 2 * kr + p;
+#pragma unroll
+        for (int q = 0; q < TB; ++q) bv[b][q] = Bl[q][guard ? min(kk, K - 1) : kk];
+    };
+    auto mma = [&](int b) {
+        double be[TB], bo[TB];
+#pragma unroll
+        for (int q = 0; q < TB; ++q) {
+            const double2 v = bv[b][q];
+            const double o = lane_xor1(p ? v.x : v.y);  // the partner's half of the other k
+            be[q] = p ? o : v.x;
+            bo[q] = p ? v.y : o;
+        }
+#pragma unroll
+        for (int q = 0; q < TB; ++q)
+#pragma unroll
+            for (int t = 0; t < TA; ++t) acc[q][t] = mfma64(av[b][0][t], be[q], acc[q][t]);
+#pragma unroll
+        for (int q = 0; q < TB; ++q)
+#pragma unroll
+            for (int t = 0; t < TA; ++t) acc[q][t] = mfma64(av[b][1][t], bo[q], acc[q][t]);
+    };
+    if (kb < ke) {
+        const int nb = (ke - kb) / 8;  // whole blocks
+        int k0 = kb, b = 0;
+        if (nb > 0) load(0, k0, false);
+        for (; b + 2 < nb; b += 2, k0 += 16) {
+            load(1, k0 + 8, false);
+            mma(0);
+            load(0, k0 + 16, false);
+            mma(1);
+        }
+        if (b + 1 < nb) {
+            load(1, k0 + 8, false);
+            mma(0);
+            mma(1);
+            k0 += 16;
+        } else if (b < nb) {
+            mma(0);
+            k0 += 8;
+        }
+        if (k0 < ke) {
+            load(0, k0, true);
+            mma(0);
+        }
+    }
+    // partial tiles through LDS, one column tile per round (wave 0's in the last
+    // slot), the four rows r finished side by side by waves 0..3
+#pragma unroll
+    for (int q = 0; q < TB; ++q) {
+        if (q > 0) __syncthreads();
+#pragma unroll
+        for (int t = 0; t < TA; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) red[wave > 0 ? wave - 1 : NW - 1][t][lane][r] = acc[q][t][r];
+        __syncthreads();
+        if (wave >= 4) continue;
+        double v[TA];
+#pragma unroll
+        for (int t = 0; t < TA; ++t) {
+            v[t] = red[NW - 1][t][lane][wave];
+            for (int w = 0; w < NW - 1; ++w) v[t] += red[w][t][lane][wave];
+        }
+        double2 *Dc = g.D + ((size_t)l * C + (c[q] < C ? c[q] : 0)) * ldd;
+#pragma unroll
+        for (int t = 0; t < TA / 2; ++t) {
+            // the lanes p = 0 (re) and p = 1 (im) of a column trade rows
+            const double own = p ? v[t + TA / 2] : v[t], o = lane_xor1(p ? v[t] : v[t + TA / 2]);
+            const double re = p ? o : own, im = p ? own : o;
+            const int m = mr + t + p * (TA / 2);
+            if (c[q] >= C) continue;
+            if (PASS) {
+                if (m < g.N) Dc[m] = make_double2(re, im);
+            } else if (m < nk8) {  // pass 1 reads Y up to nk8
+                const double2 f = kp[t];
+                Dc[m] = m < nk ? make_double2(f.x * re + f.y * im, f.x * im - f.y * re) : make_double2(0.0, 0.0);
+            }
+        }
+    }
+}
+
+template <int PASS, int TA, int TB>
+__global__ __launch_bounds__(K64_WG) void k_kin64(Kin64Args g) {
+    __shared__ double red[K64_NW][TA][64][4];
+    const tile3 tb = xcd_tile();  // (row panel, column group, l): panels of one l share B
+    const int l = tb.z;
+    const int nk = g.nkeep[l];
+    const int m0 = tb.x * 16 * TA;
+    if (m0 >= (PASS ? g.N : nk)) return;  // block-uniform
+    const int n0 = tb.y * 16 * TB;
+    if (!kin_cols_active(g.active, n0, 16 * TB, g.C, g.n_orb)) return;  // idle instances only
+    if (TB > 1 && n0 + 16 >= 2 * g.C)  // last group with one tile left
+        kin64_tiles<PASS, TA, 1>(g, l, nk, m0, n0, red);
+    else
+        kin64_tiles<PASS, TA, TB>(g, l, nk, m0, n0, red);
+}
+
+// QT[l][a][i] = Q[l][i][a], rows of np >= N values (zero from N on), through LDS
+// tiles of 32 x 32 so that reads and writes are both contiguous
+__global__ __launch_bounds__(WG) void k_kin_transpose(const double *__restrict__ Q, double *__restrict__ QT, int N,
+                                                      int nk_max, int np) {
+    __shared__ double tile[32][33];
+    const int l = blockIdx.z, a0 = blockIdx.x * 32, i0 = blockIdx.y * 32;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const double *Ql = Q + (size_t)l * N * nk_max;
+    double *Tl = QT + (size_t)l * nk_max * np;
+    for (int y = ty; y < 32; y += WG / 32)
+        tile[y][tx] = (i0 + y < N && a0 + tx < nk_max) ? Ql[(size_t)(i0 + y) * nk_max + a0 + tx] : 0.0;
+    __syncthreads();
+    for (int y = ty; y < 32; y += WG / 32)
+        if (a0 + y < nk_max && i0 + tx < np) Tl[(size_t)(a0 + y) * np + i0 + tx] = tile[tx][y];
+}
+
+// ---------------------------------------------------------------------------
+// Mixed form, tiled passes for many columns (instances sharing the tables).
 // Work-group tile 64 (M) x 128 (real columns); wave w owns the 32 x 64
 // sub-tile (w >> 1, w & 1) as 2 x 4 MFMA tiles.  K advances in chunks of
-// TKT values (16, or 32 in FP32) staged in LDS, double buffered, the
+// TKT values (16 or 32) staged in LDS, double buffered, the
 // next chunk prefetched into registers while the current one is multiplied;
 // one barrier per chunk.  Rows of the LDS tiles are padded by 16 values so
 // that the four K rows a wave reads per product fall on distinct banks.
@@ -459,47 +657,43 @@ __global__ __launch_bounds__(KIN_WG_MAX) void k_kin_bwd(const T *__restrict__ QT
 #define TNP (TN + 16)
 
 // 8 products of one K step of 4 for the wave's 2 x 4 tiles
-template <typename T>
-static __device__ __forceinline__ void kin_tile_step(const T (*As)[TMP], const T (*Bs)[TNP], int kk,
+static __device__ __forceinline__ void kin_tile_step(const float (*As)[TMP], const float (*Bs)[TNP], int kk,
                                                      int wm, int wn, int lc,
-                                                     typename mfma_t<T>::v4 (&acc)[2][4]) {
-    const T a0 = As[kk][wm + lc], a1 = As[kk][wm + 16 + lc];
-    T b[4];
+                                                     mfma_t<float>::v4 (&acc)[2][4]) {
+    const float a0 = As[kk][wm + lc], a1 = As[kk][wm + 16 + lc];
+    float b[4];
 #pragma unroll
     for (int y = 0; y < 4; ++y) b[y] = Bs[kk][wn + 16 * y + lc];
 #pragma unroll
     for (int y = 0; y < 4; ++y) {
-        acc[0][y] = mfma_t<T>::op(a0, b[y], acc[0][y]);
-        acc[1][y] = mfma_t<T>::op(a1, b[y], acc[1][y]);
+        acc[0][y] = mfma_t<float>::op(a0, b[y], acc[0][y]);
+        acc[1][y] = mfma_t<float>::op(a1, b[y], acc[1][y]);
     }
 }
 
-template <typename T, int TKT>
-__global__ __launch_bounds__(WG) void k_kin_fwd_tiled(const T *__restrict__ Q,
+template <int TKT>
+__global__ __launch_bounds__(WG) void k_kin_fwd_tiled(const float *__restrict__ Q,
                                                       const double2 *__restrict__ kph,
                                                       const int32_t *__restrict__ nkeep,
-                                                      const double *__restrict__ psi,
                                                       const float2 *__restrict__ psi32, KinRef ref,
-                                                      T *__restrict__ Y, int N, int nk_max,
+                                                      float *__restrict__ Y, int N, int nk_max,
                                                       int C, int n_orb) {
-    // FP32 (mixed): the state comes from psi32 (k_kin_prep), FP64: from psi
-    typedef typename mfma_t<T>::v4 v4;
+    typedef mfma_t<float>::v4 v4;
     constexpr int AV = TKT * TM / WG;  // A values per thread (consecutive a)
     constexpr int BV = TKT * 64 / WG;  // complex B values per thread (consecutive i)
-    __shared__ T As[2][TKT][TMP];      // [k = i][m = a]
-    __shared__ T Bs[2][TKT][TNP];      // [k = i][n = real column]
+    __shared__ float As[2][TKT][TMP];      // [k = i][m = a]
+    __shared__ float Bs[2][TKT][TNP];      // [k = i][n = real column]
     const tile3 tb = xcd_tile();       // (eigen tile, column tile, l)
     const int l = tb.z;
     const int nk = nkeep[l];
     const int a0 = tb.x * TM;
     if (a0 >= nk) return;  // block-uniform
     const int n0 = tb.y * TN;
-    if (!kin_cols_active(ref, n0, TN, C, n_orb)) return;  // idle instances only
+    if (!kin_cols_active(ref.active, n0, TN, C, n_orb)) return;  // idle instances only
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const int kr = lane >> 4, lc = lane & 15;
     const int wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
-    const T *Ql = Q + (size_t)l * N * nk_max;
-    const double2 *Xl = (const double2 *)psi + (size_t)l * C * N;
+    const float *Ql = Q + (size_t)l * N * nk_max;
     // global -> register mapping
     const int ar = t / (TM / AV), am = (t % (TM / AV)) * AV;  // A: row i, AV consecutive a
     const int bc = t / (TKT / BV), bk = (t % (TKT / BV)) * BV;  // B: complex column, BV consecutive i
@@ -507,25 +701,19 @@ __global__ __launch_bounds__(WG) void k_kin_fwd_tiled(const T *__restrict__ Q,
     const bool cok = cg < C;
     const bool aok = a0 + am < nk_max;  // nk_max is a multiple of 16 >= AV: all or none
     const float2 *Xs = psi32 + ((size_t)l * C + (cok ? cg : 0)) * N;
-    T ra[AV], rb[2 * BV];
+    float ra[AV], rb[2 * BV];
     auto load = [&](int k0) {
         const int i = k0 + ar;
         const bool ok = aok && i < N;
 #pragma unroll
-        for (int u = 0; u < AV; ++u) ra[u] = ok ? Ql[(size_t)i * nk_max + a0 + am + u] : (T)0;
+        for (int u = 0; u < AV; ++u) ra[u] = ok ? Ql[(size_t)i * nk_max + a0 + am + u] : 0.f;
 #pragma unroll
         for (int u = 0; u < BV; ++u) {
             const int ii = k0 + bk + u;
             const bool okb = cok && ii < N;
-            if (mfma_t<T>::mixed) {
-                const float2 v = okb ? Xs[ii] : make_float2(0.f, 0.f);
-                rb[2 * u] = (T)v.x;
-                rb[2 * u + 1] = (T)v.y;
-            } else {
-                const double2 v = okb ? Xl[(size_t)cg * N + ii] : make_double2(0.0, 0.0);
-                rb[2 * u] = (T)v.x;
-                rb[2 * u + 1] = (T)v.y;
-            }
+            const float2 v = okb ? Xs[ii] : make_float2(0.f, 0.f);
+            rb[2 * u] = v.x;
+            rb[2 * u + 1] = v.y;
         }
     };
     auto stash = [&](int buf) {
@@ -557,7 +745,7 @@ __global__ __launch_bounds__(WG) void k_kin_fwd_tiled(const T *__restrict__ Q,
         const bool more = k0 + TKT < N;
         if (more) load(k0 + TKT);
 #pragma unroll
-        for (int ks = 0; ks < TKT / 4; ++ks) kin_tile_step<T>(As[buf], Bs[buf], ks * 4 + kr, wm, wn, lc, acc);
+        for (int ks = 0; ks < TKT / 4; ++ks) kin_tile_step(As[buf], Bs[buf], ks * 4 + kr, wm, wn, lc, acc);
         if (more) stash(buf ^ 1);
 #pragma unroll
         for (int x = 0; x < 2; ++x)
@@ -574,19 +762,19 @@ __global__ __launch_bounds__(WG) void k_kin_fwd_tiled(const T *__restrict__ Q,
             const int col = n0 + wn + 16 * y + lc;
             const int c = col >> 1, p = col & 1;
             const int ab = a0 + wm + 16 * x;
-            T o[4];
+            float o[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int a = ab + mfma_t<T>::row(kr, r);
+                const int a = ab + mfma_t<float>::row(kr, r);
                 const double v = (double)hi[x][y][r];
                 const double vo = lane_xor1(v);
-                o[r] = kin_factor<T>(v, vo, p, kphl[a < nk ? a : 0]);
+                o[r] = kin_factor<float>(v, vo, p, kphl[a < nk ? a : 0]);
             }
             if (c < C) {
-                T *Yo = Y + (((size_t)l * C + c) * 2 + p) * nk_max;
+                float *Yo = Y + (((size_t)l * C + c) * 2 + p) * nk_max;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int a = ab + mfma_t<T>::row(kr, r);
+                    const int a = ab + mfma_t<float>::row(kr, r);
                     if (a < nk) Yo[a] = o[r];
                 }
             }
@@ -597,7 +785,7 @@ __global__ __launch_bounds__(WG) void k_kin_fwd_tiled(const T *__restrict__ Q,
 // FP32 tiled pass 1 with the tiles copied from global memory straight into
 // LDS (global_load_lds_dwordx4: no staging registers, no LDS stores), three
 // buffers and two K chunks in flight; one barrier per chunk.  It forms the
-// products of k_kin_fwd_tiled<float, 16> in the same order (same chunks, same
+// products of k_kin_fwd_tiled<16> in the same order (same chunks, same
 // MFMA sequence, same two-level sum), so the stored Y is the same bit for bit.
 // Layouts, swizzled so that the operand reads of each half-wave hit 32
 // distinct banks (the LDS serves 32 banks per half-wave):
@@ -623,7 +811,7 @@ __global__ __launch_bounds__(WG) void k_kin_fwd_dma(const float *__restrict__ Q,
     const int a0 = tb.x * TM;
     if (a0 >= nk) return;  // block-uniform
     const int n0 = tb.y * TN;
-    if (!kin_cols_active(ref, n0, TN, C, n_orb)) return;  // idle instances only
+    if (!kin_cols_active(ref.active, n0, TN, C, n_orb)) return;  // idle instances only
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const int kr = lane >> 4, lc = lane & 15;
     const int wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
@@ -732,28 +920,28 @@ __global__ __launch_bounds__(WG) void k_kin_fwd_dma(const float *__restrict__ Q,
     }
 }
 
-template <typename T, int TKT>
-__global__ __launch_bounds__(WG) void k_kin_bwd_tiled(const T *__restrict__ Q,
+template <int TKT>
+__global__ __launch_bounds__(WG) void k_kin_bwd_tiled(const float *__restrict__ Q,
                                                       const int32_t *__restrict__ nkeep,
-                                                      const T *__restrict__ Y, KinRef ref,
+                                                      const float *__restrict__ Y, KinRef ref,
                                                       double *__restrict__ psi, int N, int nk_max,
                                                       int C, int n_orb) {
-    typedef typename mfma_t<T>::v4 v4;
+    typedef mfma_t<float>::v4 v4;
     constexpr int AV = TKT * TM / WG;  // A values per thread (consecutive a of one row i)
     constexpr int BV = TKT * TN / WG;  // B values per thread (consecutive a of one column)
-    __shared__ T As[2][TKT][TMP];      // [k = a][m = i]
-    __shared__ T Bs[2][TKT][TNP];      // [k = a][n = real column]
+    __shared__ float As[2][TKT][TMP];      // [k = a][m = i]
+    __shared__ float Bs[2][TKT][TNP];      // [k = a][n = real column]
     const tile3 tb = xcd_tile();       // (radial tile, column tile, l)
     const int l = tb.z;
     const int nk = nkeep[l];
     const int i0 = tb.x * TM;
     const int n0 = tb.y * TN;
-    if (!kin_cols_active(ref, n0, TN, C, n_orb)) return;  // idle instances only
+    if (!kin_cols_active(ref.active, n0, TN, C, n_orb)) return;  // idle instances only
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const int kr = lane >> 4, lc = lane & 15;
     const int wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
-    const T *Ql = Q + (size_t)l * N * nk_max;
-    const T *Yl = Y + (size_t)l * C * 2 * nk_max;
+    const float *Ql = Q + (size_t)l * N * nk_max;
+    const float *Yl = Y + (size_t)l * C * 2 * nk_max;
     const int am = t / (TKT / AV), ak = (t % (TKT / AV)) * AV;  // A: row i, AV consecutive a
     const int bn = t / (TKT / BV), bk = (t % (TKT / BV)) * BV;  // B: real column, BV consecutive a
     const int ia = i0 + am;
@@ -761,14 +949,14 @@ __global__ __launch_bounds__(WG) void k_kin_bwd_tiled(const T *__restrict__ Q,
     const bool bok = (colb >> 1) < C;
     // the tables and Y are zero from nkeep up to nk_max: runs of AV, BV (<= 16,
     // dividing 16) are wholly inside or outside [0, nk_max)
-    T ra[AV], rb[BV];
+    float ra[AV], rb[BV];
     auto load = [&](int k0) {
         const bool oka = ia < N && k0 + ak < nk_max;
 #pragma unroll
-        for (int u = 0; u < AV; ++u) ra[u] = oka ? Ql[(size_t)ia * nk_max + k0 + ak + u] : (T)0;
+        for (int u = 0; u < AV; ++u) ra[u] = oka ? Ql[(size_t)ia * nk_max + k0 + ak + u] : 0.f;
         const bool okb = bok && k0 + bk < nk_max;
 #pragma unroll
-        for (int u = 0; u < BV; ++u) rb[u] = okb ? Yl[(size_t)colb * nk_max + k0 + bk + u] : (T)0;
+        for (int u = 0; u < BV; ++u) rb[u] = okb ? Yl[(size_t)colb * nk_max + k0 + bk + u] : 0.f;
     };
     auto stash = [&](int buf) {
 #pragma unroll
@@ -796,7 +984,7 @@ __global__ __launch_bounds__(WG) void k_kin_bwd_tiled(const T *__restrict__ Q,
         const bool more = k0 + TKT < nk;
         if (more) load(k0 + TKT);
 #pragma unroll
-        for (int ks = 0; ks < TKT / 4; ++ks) kin_tile_step<T>(As[buf], Bs[buf], ks * 4 + kr, wm, wn, lc, acc);
+        for (int ks = 0; ks < TKT / 4; ++ks) kin_tile_step(As[buf], Bs[buf], ks * 4 + kr, wm, wn, lc, acc);
         if (more) stash(buf ^ 1);
 #pragma unroll
         for (int x = 0; x < 2; ++x)
@@ -814,10 +1002,10 @@ __global__ __launch_bounds__(WG) void k_kin_bwd_tiled(const T *__restrict__ Q,
             const int c = col >> 1, p = col & 1;
             if (c >= C) continue;
             double rc = 0.0;
-            const double *rrow = mfma_t<T>::mixed ? kin_ref_row(ref, l, c, p, N, n_orb, true, &rc) : nullptr;
+            const double *rrow = kin_ref_row(ref, l, c, p, N, n_orb, true, &rc);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int i = i0 + wm + 16 * x + mfma_t<T>::row(kr, r);
+                const int i = i0 + wm + 16 * x + mfma_t<float>::row(kr, r);
                 if (i < N) {
                     double v = (double)hi[x][y][r];
                     if (rrow) v += rc * rrow[i];
@@ -829,7 +1017,7 @@ __global__ __launch_bounds__(WG) void k_kin_bwd_tiled(const T *__restrict__ Q,
 }
 
 // FP32 tiled pass 2 with direct global-to-LDS copies, as k_kin_fwd_dma: the
-// products, chunks and sums of k_kin_bwd_tiled<float, 16> in the same order
+// products, chunks and sums of k_kin_bwd_tiled<16> in the same order
 // (the same psi bit for bit).  Both operands are K-contiguous in memory (Q
 // rows i, Y rows of a column), so the chunk tiles are kept row-major by their
 // M or N index: element (row, k) at row 16 + 4 ((k / 4 + (row / 4)) & 3) + k % 4.
@@ -849,7 +1037,7 @@ __global__ __launch_bounds__(WG) void k_kin_bwd_dma(const float *__restrict__ Q,
     const int nk = nkeep[l];
     const int i0 = tb.x * TM;
     const int n0 = tb.y * TN;
-    if (!kin_cols_active(ref, n0, TN, C, n_orb)) return;  // idle instances only
+    if (!kin_cols_active(ref.active, n0, TN, C, n_orb)) return;  // idle instances only
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const int kr = lane >> 4, lc = lane & 15;
     const int wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
@@ -1006,7 +1194,7 @@ __global__ __launch_bounds__(WG) void k_kin_fwd_split(const float *__restrict__ 
     const int a0 = tb.x * TM;
     if (a0 >= nk) return;  // block-uniform
     const int n0 = tb.y * TN;
-    if (!kin_cols_active(ref, n0, TN, C, n_orb)) return;  // idle instances only
+    if (!kin_cols_active(ref.active, n0, TN, C, n_orb)) return;  // idle instances only
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const int kr = lane >> 4, lc = lane & 15;
     const int wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
@@ -1132,7 +1320,7 @@ __global__ __launch_bounds__(WG) void k_kin_bwd_split(const float *__restrict__ 
     const int nk = nkeep[l];
     const int i0 = tb.x * TM;
     const int n0 = tb.y * TN;
-    if (!kin_cols_active(ref, n0, TN, C, n_orb)) return;  // idle instances only
+    if (!kin_cols_active(ref.active, n0, TN, C, n_orb)) return;  // idle instances only
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const int kr = lane >> 4, lc = lane & 15;
     const int wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
@@ -2562,6 +2750,13 @@ extern "C" void ggb_destroy(ggb_ctx *ctx) {
     delete ctx;
 }
 
+static int round16(int n) { return (n + 15) & ~15; }
+
+// values of the transposed kinetic table: rows of N padded to a multiple of 16 in FP64
+static size_t qt_values(const ggb_problem *p) {
+    return (size_t)p->n_l * p->nk_max * (p->precision ? p->n_r : round16(p->n_r));
+}
+
 static size_t footprint_bytes(const ggb_problem *p, int ntiles) {
     const size_t N = p->n_r, Nl = p->n_l, C = (size_t)p->n_orb * p->n_inst, Nth = p->n_theta;
     const size_t nI = p->n_inst, nk = p->nk_max, nh = p->n_har;
@@ -2570,7 +2765,7 @@ static size_t footprint_bytes(const ggb_problem *p, int ntiles) {
     const size_t es = p->precision ? 4 : 8;
     const size_t nblk = ang_geometry(p).nblk;
     // Y, Q, QT (not in precision 2), B; precision 2 adds the low parts of Q and Y
-    size_t tbytes = (Nl * C * nk * 2 + (p->precision == 2 ? 1 : 2) * Nl * N * nk + (size_t)p->n_m * nblk) * es;
+    size_t tbytes = (Nl * C * nk * 2 + Nl * N * nk + (p->precision == 2 ? 0 : qt_values(p)) + (size_t)p->n_m * nblk) * es;
     if (p->precision == 2) tbytes += (Nl * N * nk + Nl * C * nk * 2) * sizeof(float);
     d += 2 * Nl * nk;                    // e^{-i lam dt}
     d += 2 * Nth * nh + 2 * Nth;         // PL, PLT, chi, omega
@@ -2669,8 +2864,8 @@ extern "C" int ggb_create(const ggb_problem *p, ggb_ctx **out) {
     const size_t nB = (size_t)p->n_m * ctx->ang.nblk;
     ok &= dalloc(&ctx->Y, (nY * es + 7) / 8) == hipSuccess;
     ok &= dalloc(&ctx->Q, (nQ * es + 7) / 8) == hipSuccess;
-    if (p->precision != 2)  // [l][a][i] for the narrow pass 2 (precision 2 runs the split passes only)
-        ok &= dalloc(&ctx->QT, (nQ * es + 7) / 8) == hipSuccess;
+    if (p->precision != 2)  // the transposed table of pass 2 (precision 2 runs the split passes only)
+        ok &= dalloc(&ctx->QT, (qt_values(p) * es + 7) / 8) == hipSuccess;
     ok &= dalloc(&ctx->kph, Nl * (size_t)p->nk_max) == hipSuccess;
     ok &= dalloc(&ctx->nkeep, Nl) == hipSuccess;
     ok &= dalloc(&ctx->B, (nB * es + 7) / 8) == hipSuccess;
@@ -2708,7 +2903,7 @@ extern "C" int ggb_create(const ggb_problem *p, ggb_ctx **out) {
     if (!ok) return bail("ggb_create: device allocation failed", GGB_E_NOMEM);
     // zero everything that kernels may read before it is written
     if (hipMemset(ctx->B, 0, nB * es) != hipSuccess || hipMemset(ctx->Q, 0, nQ * es) != hipSuccess ||
-        (ctx->QT && hipMemset(ctx->QT, 0, nQ * es) != hipSuccess) ||
+        (ctx->QT && hipMemset(ctx->QT, 0, qt_values(p) * es) != hipSuccess) ||
         (ctx->Qlo && hipMemset(ctx->Qlo, 0, nQ * sizeof(float)) != hipSuccess) ||
         (ctx->Ylo && hipMemset(ctx->Ylo, 0, nY * sizeof(float)) != hipSuccess) ||
         hipMemset(ctx->kph, 0, Nl * (size_t)p->nk_max * sizeof(double2)) != hipSuccess ||
@@ -2763,15 +2958,14 @@ extern "C" int ggb_upload_static(ggb_ctx *ctx, const ggb_static *s) {
     HIPCHK(ctx, hipMemcpyAsync(ctx->v_gs, s->v_gs, N * 8, hipMemcpyHostToDevice, st));
     HIPCHK(ctx, hipMemcpyAsync(ctx->mask, s->mask, N * 8, hipMemcpyHostToDevice, st));
     {
-        // Q[l][i][a] and its quad-interleaved transpose QT (read by the narrow pass 2), compute type
+        // Q[l][i][a] in the compute type, and for pass 2 its transpose QT: [l][a][i] with rows
+        // padded to a multiple of 16 (FP64), or quad-interleaved (mixed form, narrow pass 2)
         const size_t nk = p.nk_max, nQ = Nl * N * nk;
         if (p.precision == 0) {
             HIPCHK(ctx, hipMemcpy(ctx->Q, s->Q, nQ * 8, hipMemcpyHostToDevice));
-            std::vector<double> qt(nQ);
-            for (size_t l = 0; l < Nl; ++l)
-                for (size_t i = 0; i < N; ++i)
-                    for (size_t a = 0; a < nk; ++a) qt[kin_qt_index(l, i, a, N, nk)] = s->Q[(l * N + i) * nk + a];
-            HIPCHK(ctx, hipMemcpy(ctx->QT, qt.data(), nQ * 8, hipMemcpyHostToDevice));
+            const int np = round16(p.n_r);
+            k_kin_transpose<<<dim3((p.nk_max + 31) / 32, (np + 31) / 32, p.n_l), WG, 0, st>>>(ctx->Q, ctx->QT, p.n_r, p.nk_max, np);
+            HIPCHK(ctx, hipGetLastError());
         } else {
             std::vector<float> q32(nQ);
             for (size_t k = 0; k < nQ; ++k) q32[k] = (float)s->Q[k];
@@ -3068,16 +3262,53 @@ static void kin_launch(void (*k)(KArgs...), dim3 g, int threads, hipStream_t st,
         k<<<g, threads, 0, st>>>(args...);
 }
 
+template <int TA, int TB>
+static void launch_kin64_t(ggb_ctx *ctx, int pass, hipEvent_t e0, hipEvent_t e1) {
+    const ggb_problem &p = ctx->p;
+    Kin64Args g;
+    g.A = pass ? ctx->QT : ctx->Q;
+    g.B = reinterpret_cast<const double2 *>(pass ? ctx->Y : ctx->psi);
+    g.D = reinterpret_cast<double2 *>(pass ? ctx->psi : ctx->Y);
+    g.kph = ctx->kph;
+    g.nkeep = ctx->nkeep;
+    g.active = ctx->active;
+    g.N = p.n_r;
+    g.nk_max = p.nk_max;
+    g.np = round16(p.n_r);
+    g.C = ctx->C;
+    g.n_orb = p.n_orb;
+    const int rows = pass ? p.n_r : p.nk_max;
+    const dim3 grid((rows + 16 * TA - 1) / (16 * TA), (2 * g.C + 16 * TB - 1) / (16 * TB), p.n_l);
+    if (pass)
+        kin_launch(k_kin64<1, TA, TB>, grid, K64_WG, ctx->stream, e0, e1, g);
+    else
+        kin_launch(k_kin64<0, TA, TB>, grid, K64_WG, ctx->stream, e0, e1, g);
+}
+
+// Shape of the FP64 passes.  NARROW: one tile of 16 real columns per work-group
+// (idle instances are skipped 8 columns at a time), and the only one up to 8
+// columns.  Otherwise two tiles, which read the table half as often; panels of
+// 32 rows up to 32 columns, where the work-groups are few, of 64 beyond
+// (argon size, passes 0 / 1: 28 columns 45 / 43 us with 32 rows, 47 / 45 with 64;
+// 63 columns 80 / 77 against 81 / 77, 224 columns 249 / 245 against 237 / 234).
+// Every element is formed by the same products in the same order in all of them.
+static void launch_kin64(ggb_ctx *ctx, int pass, hipEvent_t e0, hipEvent_t e1) {
+    if (ctx->kin_variant == GGB_KIN_NARROW || ctx->C <= 8)
+        launch_kin64_t<2, 1>(ctx, pass, e0, e1);
+    else if (ctx->C <= 32)
+        launch_kin64_t<2, 2>(ctx, pass, e0, e1);
+    else
+        launch_kin64_t<4, 2>(ctx, pass, e0, e1);
+}
+
 // e0/e1 (optional): events stamped with the start and end of the pass's
 // product kernel itself, for the kernel-duration timing
-template <typename T>
-static void launch_kinetic_t(ggb_ctx *ctx, int pass, bool fresh, hipEvent_t e0 = nullptr,
-                             hipEvent_t e1 = nullptr) {
+static void launch_kinetic_mixed(ggb_ctx *ctx, int pass, bool fresh, hipEvent_t e0, hipEvent_t e1) {
     const ggb_problem &p = ctx->p;
-    const T *Q = reinterpret_cast<const T *>(ctx->Q);
-    T *Y = reinterpret_cast<T *>(ctx->Y);
+    const float *Q = reinterpret_cast<const float *>(ctx->Q);
+    float *Y = reinterpret_cast<float *>(ctx->Y);
     KinRef ref;
-    ref.phi = (mfma_t<T>::mixed && ctx->have_ref) ? ctx->phi_ref : nullptr;
+    ref.phi = ctx->have_ref ? ctx->phi_ref : nullptr;
     ref.l0 = ctx->l0;
     ref.ab = ctx->ab;
     ref.active = ctx->active;
@@ -3108,35 +3339,33 @@ static void launch_kinetic_t(ggb_ctx *ctx, int pass, bool fresh, hipEvent_t e0 =
     if (var >= GGB_KIN_TILED16) {
         const int nct = (2 * ctx->C + TN - 1) / TN;
         const dim3 gf((p.nk_max + TM - 1) / TM, nct, p.n_l), gb((p.n_r + TM - 1) / TM, nct, p.n_l);
-        if (pass == 0 && mfma_t<T>::mixed && !(fresh && !ref.phi))
+        if (pass == 0 && !(fresh && !ref.phi))
             k_kin_prep<<<dim3((p.n_r + WG - 1) / WG, ctx->C, fresh ? 1 : p.n_l), WG, 0, ctx->stream>>>(
                 (const double2 *)ctx->psi, ref, ctx->psi32, p.n_r, ctx->C, p.n_orb, fresh ? 1 : 0);
-        // FP64 chunks stay at 16 (32 would need 114 KB of LDS)
-        const bool k32 = var == GGB_KIN_TILED32 && mfma_t<T>::mixed;
+        const bool k32 = var == GGB_KIN_TILED32;
         const double2 *kph = ctx->kph;
         const int32_t *nkeep = ctx->nkeep;
-        const double *psi_in = ctx->psi;
         double *psi_out = ctx->psi;
         const float2 *psi32 = ctx->psi32;
         const int N = p.n_r, nkm = p.nk_max, C = ctx->C, no = p.n_orb;
         if (pass == 0 && k32)
-            kin_launch(k_kin_fwd_tiled<T, 32>, gf, WG, ctx->stream, e0, e1, Q,
-                                  kph, nkeep, psi_in, psi32, ref, Y, N, nkm, C, no);
-        else if (pass == 0 && mfma_t<T>::mixed && KIN_DMA && N % 16 == 0)
-            kin_launch(k_kin_fwd_dma, gf, WG, ctx->stream, e0, e1, reinterpret_cast<const float *>(Q),
-                       kph, nkeep, psi32, ref, reinterpret_cast<float *>(Y), N, nkm, C, no);
+            kin_launch(k_kin_fwd_tiled<32>, gf, WG, ctx->stream, e0, e1, Q,
+                                  kph, nkeep, psi32, ref, Y, N, nkm, C, no);
+        else if (pass == 0 && KIN_DMA && N % 16 == 0)
+            kin_launch(k_kin_fwd_dma, gf, WG, ctx->stream, e0, e1, Q,
+                       kph, nkeep, psi32, ref, Y, N, nkm, C, no);
         else if (pass == 0)
-            kin_launch(k_kin_fwd_tiled<T, 16>, gf, WG, ctx->stream, e0, e1, Q,
-                                  kph, nkeep, psi_in, psi32, ref, Y, N, nkm, C, no);
+            kin_launch(k_kin_fwd_tiled<16>, gf, WG, ctx->stream, e0, e1, Q,
+                                  kph, nkeep, psi32, ref, Y, N, nkm, C, no);
         else if (k32)
-            kin_launch(k_kin_bwd_tiled<T, 32>, gb, WG, ctx->stream, e0, e1,
-                                  (const T *)Q, nkeep, (const T *)Y, ref, psi_out, N, nkm, C, no);
-        else if (mfma_t<T>::mixed && KIN_DMA)
-            kin_launch(k_kin_bwd_dma, gb, WG, ctx->stream, e0, e1, reinterpret_cast<const float *>(Q), nkeep,
-                       reinterpret_cast<const float *>(Y), ref, psi_out, N, nkm, C, no);
+            kin_launch(k_kin_bwd_tiled<32>, gb, WG, ctx->stream, e0, e1,
+                                  Q, nkeep, (const float *)Y, ref, psi_out, N, nkm, C, no);
+        else if (KIN_DMA)
+            kin_launch(k_kin_bwd_dma, gb, WG, ctx->stream, e0, e1, Q, nkeep,
+                       (const float *)Y, ref, psi_out, N, nkm, C, no);
         else
-            kin_launch(k_kin_bwd_tiled<T, 16>, gb, WG, ctx->stream, e0, e1,
-                                  (const T *)Q, nkeep, (const T *)Y, ref, psi_out, N, nkm, C, no);
+            kin_launch(k_kin_bwd_tiled<16>, gb, WG, ctx->stream, e0, e1,
+                                  Q, nkeep, (const float *)Y, ref, psi_out, N, nkm, C, no);
         return;
     }
     const int ncol = (2 * ctx->C + 15) / 16;
@@ -3145,13 +3374,13 @@ static void launch_kinetic_t(ggb_ctx *ctx, int pass, bool fresh, hipEvent_t e0 =
     const int N = p.n_r, nkm = p.nk_max, C = ctx->C, no = p.n_orb;
     if (pass == 0) {
         const double *psi_in = ctx->psi;
-        kin_launch(k_kin_fwd<T, KIN_TA>, dim3((p.nk_max / 16 + KIN_TA - 1) / KIN_TA, ncol, p.n_l), 64 * kin_nw<T>::value,
+        kin_launch(k_kin_fwd<KIN_TA>, dim3((p.nk_max / 16 + KIN_TA - 1) / KIN_TA, ncol, p.n_l), KIN_NARROW_WG,
                    ctx->stream,
                    e0, e1, Q, kph, nkeep,
                    psi_in, ref, Y, N, nkm, C, no);
     } else {
-        kin_launch(k_kin_bwd<T>, dim3((p.n_r + 15) / 16, ncol, p.n_l), 64 * kin_nw<T>::value, ctx->stream, e0, e1,
-                   reinterpret_cast<const T *>(ctx->QT), nkeep, (const T *)Y, ref, ctx->psi, N, nkm,
+        kin_launch(k_kin_bwd, dim3((p.n_r + 15) / 16, ncol, p.n_l), KIN_NARROW_WG, ctx->stream, e0, e1,
+                   reinterpret_cast<const float *>(ctx->QT), nkeep, (const float *)Y, ref, ctx->psi, N, nkm,
                    C, no);
     }
 }
@@ -3159,9 +3388,9 @@ static void launch_kinetic_t(ggb_ctx *ctx, int pass, bool fresh, hipEvent_t e0 =
 static int launch_kinetic_pass(ggb_ctx *ctx, int pass, bool fresh = false, hipEvent_t e0 = nullptr,
                                hipEvent_t e1 = nullptr) {
     if (ctx->p.precision)
-        launch_kinetic_t<float>(ctx, pass, fresh, e0, e1);
+        launch_kinetic_mixed(ctx, pass, fresh, e0, e1);
     else
-        launch_kinetic_t<double>(ctx, pass, fresh, e0, e1);
+        launch_kin64(ctx, pass, e0, e1);
     HIPCHK(ctx, hipGetLastError());
     return GGB_OK;
 }
