@@ -4483,7 +4483,7 @@ extern "C" int ggb_selftest_copy(int32_t device, uint64_t bytes, double *ms) {
 // One SCF iteration:
 //   k_gs_potential  rho_u = sum_s occ_s u_s^2,  v_out = V_0[rho_u] + v_xc[rho],
 //                   v <- v + mix (v_out - v)   (v = v_out at the first)
-//   k_gs_sweep      one work-group per l group, `sweeps` passes over its
+//   k_gs_sweep      a team of work-groups per l group, `sweeps` passes over its
 //                   shells in shell order; for shell s:
 //                     x <- u_s made orthogonal to the group's lower shells
 //                          (modified Gram-Schmidt) and normalised
@@ -4502,6 +4502,11 @@ extern "C" int ggb_selftest_copy(int32_t device, uint64_t bytes, double *ms) {
 // ---------------------------------------------------------------------------
 #define GS_WG 1024
 #define GS_MAX_N 1536   // k_gs_sweep keeps 5 N-vectors in LDS (60 KiB) plus 8 KiB of scratch
+#define GS_ROWS 16      // rows of a product per work-group of a team (128 bytes), or a multiple
+#define GS_TEAM_MIN_N 144  // below, a group's products stay in one work-group
+#define GS_MAX_WG 224   // work-groups of all teams (7/8 of the CUs: they wait for each other, so all are resident)
+#define GS_LDS_MAX 98304  // the shells are kept in LDS too up to this size
+#define GS_WAIT 1000000000LL  // ticks of the 100 MHz clock after which a wait gives up (10 s)
 #define GS_MAX_K 8      // shells per l group
 
 struct GsArgs {
@@ -4513,13 +4518,46 @@ struct GsArgs {
     double *eps;         // [n_shell] (first iteration: +inf)
     double *v, *rho_u;   // [N]
     double *res;         // [0] max |v_out - v|, [1 + g] max |eps - eps_prev| of group g
+    double *ex;          // [n_group][3][N] product vectors in exchange between a team's work-groups
+    double *priv;        // [n_group][team][GS_MAX_K][N] each work-group's shells, or null (kept in LDS)
+    int team, rows;      // work-groups per group, rows of a product of each
     int N, n_shell, n_group, sweeps, interacting, first, final_;
     double Z, mix, gamma;
 };
 
+// v of lane + OFF (OFF = 32, 16, 8, 4, 2 or 1; meaningful in the lanes below OFF), as __shfl_down
+// gives it but through permlane swaps and DPP row shifts, not an LDS round trip
+template <int OFF>
+static __device__ __forceinline__ unsigned gs_lane_down(unsigned v) {
+    if constexpr (OFF == 32)
+        return __builtin_amdgcn_permlane32_swap(v, v, false, false)[1];
+    else if constexpr (OFF == 16)
+        return __builtin_amdgcn_permlane16_swap(v, v, false, false)[1];
+    else
+        return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x100 + OFF, 0xF, 0xF, false);  // row_shl
+}
+template <int CTRL>
+static __device__ __forceinline__ double gs_dpp(double x) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xF, 0xF, false);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xF, 0xF, false);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <int OFF>
+static __device__ __forceinline__ double gs_down(double x) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+    const unsigned lo = gs_lane_down<OFF>((unsigned)b), hi = gs_lane_down<OFF>((unsigned)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 // sum over the work-group, fixed order (every thread gets the result)
 static __device__ double gs_sum(double v, double *red) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
+    v += gs_down<32>(v);
+    v += gs_down<16>(v);
+    v += gs_down<8>(v);
+    v += gs_down<4>(v);
+    v += gs_down<2>(v);
+    v += gs_down<1>(v);
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     __syncthreads();  // earlier readers of red are done
     if (lane == 0) red[w] = v;
@@ -4556,11 +4594,17 @@ static __device__ double gs_scan(double v, int dir, double *buf) {
     return buf[me];
 }
 
+// an exchange slot that holds no value yet: a NaN with a payload of its own, which no
+// arithmetic forms
+static __device__ __forceinline__ double gs_empty() { return __longlong_as_double(0x7ff8a5a55a5a0001LL); }
+
 // rho_u, V_0 + v_xc and the damped update (final_: v <- v_out, no mixing)
 __global__ __launch_bounds__(GS_WG) void k_gs_potential(GsArgs a) {
     __shared__ double buf[GS_WG];
     __shared__ double red[GS_WG / 64];
     const int t = threadIdx.x, nt = blockDim.x, N = a.N;
+    // the sweep that follows starts with empty exchange slots
+    for (int k = t; k < a.n_group * 3 * N; k += nt) a.ex[k] = gs_empty();
     // thread t owns the radial chunk [i0, i1)
     const int ch = (N + nt - 1) / nt;
     const int i0 = min(N, t * ch), i1 = min(N, i0 + ch);
@@ -4598,7 +4642,7 @@ __global__ __launch_bounds__(GS_WG) void k_gs_potential(GsArgs a) {
 }
 
 // out[c] = sum_j M[j][c] x[j] (M row-major N x N; threads read along c,
-// coalesced).  With N < blockDim the j range is split into P = blockDim / N
+// coalesced; one work-group alone).  With N < blockDim the j range is split into P = blockDim / N
 // parts (more loads in flight), the parts added in fixed order through scr
 // ((P - 1) N <= blockDim doubles); eight partial sums per thread.
 template <typename TE>
@@ -4634,11 +4678,103 @@ static __device__ void gs_colsum(const TE *M, const double *x, int N, double *ou
     }
 }
 
-// y = H x for the group's l (T symmetric, read by columns)
-static __device__ void gs_apply_h(const GsArgs &a, int l, const double *x, double *y, double *scr) {
+// ---------------------------------------------------------------------------
+// Teams.  A pass over one shell is four matrix-vector products in sequence (H x,
+// Q0^T r, Q0 t, H w) with short vector work between them.  One work-group per group
+// read all of T, Q0 and Q0^T through one CU: 99 us a pass at N = 512, 2.4 ms an
+// iteration.  Now a team of work-groups shares the rows of each product, 16 rows a
+// work-group where the device holds all teams, and only product rows are exchanged.
+// An argon iteration at N = 512 takes 0.59 ms (2.38), a krypton one at N = 768 0.94 ms
+// (7.37); every sum keeps its terms and their order, so the results are the same bit
+// for bit.  What bounds it is the latency of a phase (a product of 16 rows, a
+// store and a load across the device), not its bytes.  Below N = 128 one work-group alone
+// is as fast (He, N = 96: 11.2 against 15.8 ms in a team) and keeps gs_colsum.
+//   A phase: each work-group writes its rows to one of three exchange slots, and
+// every thread polls the values it needs until none is empty: there are no flags and
+// no barrier over the team.  The slot of phase n - 1 is emptied again, each
+// work-group its own rows, when phase n is complete (then every work-group has
+// read it) and before its rows of phase n + 1 are written, so whoever reaches phase
+// n + 2 finds it empty or filled anew.  Values go through agent-scope atomic
+// stores and loads, as the team spreads over XCDs with an L2 each.  The launch is
+// cooperative (all work-groups resident), and a wait ends after GS_WAIT whatever
+// happens, with res[1 + g] = -1.
+// ---------------------------------------------------------------------------
+struct GsTeam {
+    double *ex;  // [3][N]
+    int me, phase;
+    bool ok;
+};
+
+// out = M x for a team (MT: the transpose, for a team of one; x, out in LDS, scr [GS_WG] scratch),
+// with the sums of gs_colsum: the eight partial sums of a part are in eight lanes.
+template <bool TEAM, typename TE>
+static __device__ __forceinline__ void gs_matvec(const GsArgs &a, GsTeam &tm, const TE *M, const TE *MT, const double *x, double *out,
+                                 double *scr) {
+    if (!TEAM) return gs_colsum(MT, x, a.N, out, scr);
+    const int N = a.N, t = threadIdx.x;
+    const int P = N < GS_WG ? GS_WG / N : 1;
+    const int jl = (N + P - 1) / P;
+    const int i0 = tm.me * a.rows, nrow = min(N, i0 + a.rows) - i0;
+    double *slot = tm.ex + (size_t)(tm.phase % 3) * N;
+    const int per = GS_WG / (8 * P);  // rows per round, at least one
+    for (int c0 = 0; c0 < nrow; c0 += per) {
+        const int u = t & 7, part = (t >> 3) % P, c = c0 + (t >> 3) / P;
+        const int j0 = part * jl, j1 = min(N, j0 + jl);
+        double s = 0.0;
+        const bool in = (t >> 3) / P < per && c < nrow;
+        if (in) {
+            const TE *Mc = M + (size_t)(i0 + c) * N;
+            int j = j0;
+#pragma unroll 8
+            for (; j + 8 <= j1; j += 8) s += (double)Mc[j + u] * x[j + u];
+            if (u == 0)
+                for (; j < j1; ++j) s += (double)Mc[j] * x[j];
+        }
+        // ((s0 + s1) + (s2 + s3)) + ((s4 + s5) + (s6 + s7)) in every lane of the eight
+        s += gs_dpp<0xB1>(s);   // quad_perm [1,0,3,2]
+        s += gs_dpp<0x4E>(s);   // quad_perm [2,3,0,1]
+        s += gs_dpp<0x141>(s);  // row_half_mirror
+        if (in && u == 0) scr[(t >> 3) / P * P + part] = s;
+        __syncthreads();
+        // the rows leave in one store of whole lines, not 8 bytes at a time from the lanes that
+        // hold them (neon, N = 384: 28 against 33 ms; krypton, N = 768: 145 against 160)
+        if (t < per && c0 + t < nrow) {
+            double v = scr[t * P];
+            for (int q = 1; q < P; ++q) v += scr[t * P + q];
+            __hip_atomic_store(slot + i0 + c0 + t, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (c0 + per < nrow) __syncthreads();
+    }
+    // the whole vector, as its rows arrive
+    const long long empty = __double_as_longlong(gs_empty());
+    const long long t0 = wall_clock64();
+    for (int i = t; i < N; i += GS_WG) {
+        double v = __hip_atomic_load(slot + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        while (__double_as_longlong(v) == empty && tm.ok) {
+            v = __hip_atomic_load(slot + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (wall_clock64() - t0 > GS_WAIT) tm.ok = false;
+        }
+        out[i] = v;
+    }
+    tm.ok = __syncthreads_and(tm.ok) != 0;  // all of it is in `out`
+    double *prev = tm.ex + (size_t)((tm.phase + 2) % 3) * N;
+    if (tm.phase > 0 && t < nrow) __hip_atomic_store(prev + i0 + t, gs_empty(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // emptied before this work-group's next rows are written: every access to the
+    // slots is an agent-scope atomic, which goes past the L2s, so it is enough that
+    // this wave's store has arrived (an agent fence here writes back and drops
+    // whole caches, and costs half as much again as the phase)
+    asm volatile("" ::: "memory");
+    KD_WAIT(0);
+    asm volatile("" ::: "memory");
+    ++tm.phase;
+}
+
+// y = H x for the group's l (T symmetric)
+template <bool TEAM>
+static __device__ void gs_apply_h(const GsArgs &a, GsTeam &tm, int l, const double *x, double *y, double *scr) {
     const int N = a.N;
     const double cl = 0.5 * (double)l * (double)(l + 1);
-    gs_colsum(a.T, x, N, y, scr);
+    gs_matvec<TEAM>(a, tm, a.T, a.T, x, y, scr);
     for (int i = threadIdx.x; i < N; i += blockDim.x) {
         const double ri = a.r[i];
         const double d = cl / (ri * ri) - a.Z / ri + a.v[i];
@@ -4648,16 +4784,17 @@ static __device__ void gs_apply_h(const GsArgs &a, int l, const double *x, doubl
 
 // w = Q0 diag(1/(|lam0 - theta| + gamma)) Q0^T r, through tmp (all in LDS); the
 // eigenvector tables in FP32 (the preconditioner only sets the rate)
-static __device__ void gs_precondition(const GsArgs &a, int g, double theta, const double *rv,
+template <bool TEAM>
+static __device__ void gs_precondition(const GsArgs &a, GsTeam &tm, int g, double theta, const double *rv,
                                        double *tmp, double *w, double *scr) {
     const int N = a.N;
     const float *Q = a.Q0 + (size_t)g * N * N;    // [i][k]
     const float *QT = a.Q0T + (size_t)g * N * N;  // [k][i]
     const double *lam = a.lam0 + (size_t)g * N;
-    gs_colsum(Q, rv, N, tmp, scr);
+    gs_matvec<TEAM>(a, tm, QT, Q, rv, tmp, scr);
     for (int k = threadIdx.x; k < N; k += blockDim.x) tmp[k] /= fabs(lam[k] - theta) + a.gamma;
     __syncthreads();
-    gs_colsum(QT, tmp, N, w, scr);
+    gs_matvec<TEAM>(a, tm, Q, QT, tmp, w, scr);
 }
 
 static __device__ double gs_dot(const double *x, const double *y, int N, double *red) {
@@ -4667,45 +4804,52 @@ static __device__ double gs_dot(const double *x, const double *y, int N, double 
 }
 
 // x -= (q.x) q for each lower shell q of the group, in shell order
-static __device__ void gs_deflate(const GsArgs &a, const int32_t *sh, int j, double *x, double *red) {
+static __device__ void gs_deflate(const GsArgs &a, const double *u, int j, double *x, double *red) {
     const int N = a.N;
     for (int q = 0; q < j; ++q) {
-        const double *uq = a.u + (size_t)sh[q] * N;
+        const double *uq = u + (size_t)q * N;
         const double c = gs_dot(uq, x, N, red);
         for (int i = threadIdx.x; i < N; i += blockDim.x) x[i] -= c * uq[i];
         __syncthreads();
     }
 }
 
-// one work-group per l group: `sweeps` preconditioned Rayleigh-Ritz passes
+// one team of work-groups per l group: `sweeps` preconditioned Rayleigh-Ritz passes
 // over the group's shells with the potential a.v; eps and the group's
-// largest eps change into a.res[1 + g]
+// largest eps change into a.res[1 + g].  Every work-group keeps all vectors and
+// does the same vector work in the same order, so all hold the same bits; the orbitals
+// are kept in LDS until the last sweep, when the team's first work-group stores them.
+template <bool TEAM, bool LDSU>
 __global__ __launch_bounds__(GS_WG) void k_gs_sweep(GsArgs a) {
     extern __shared__ double gsm[];
     __shared__ double red[GS_WG / 64];
     __shared__ double scr[GS_WG];
-    const int g = blockIdx.x, N = a.N, l = a.gl[g];
+    const int g = blockIdx.x % a.n_group, N = a.N, l = a.gl[g];
+    GsTeam tm{a.ex + (size_t)g * 3 * N, (int)blockIdx.x / a.n_group, 0, true};
     const int32_t *sh = a.gsh + (size_t)g * GS_MAX_K;
     int k = 0;
     while (k < GS_MAX_K && sh[k] >= 0) ++k;
     double *x = gsm, *hx = gsm + N, *w = gsm + 2 * N, *hw = gsm + 3 * N, *tmp = gsm + 4 * N;
+    double *u = LDSU ? gsm + 5 * N : a.priv + ((size_t)g * a.team + tm.me) * GS_MAX_K * N;  // [k][N]
+    for (int j = 0; j < k; ++j)
+        for (int i = threadIdx.x; i < N; i += blockDim.x) u[(size_t)j * N + i] = a.u[(size_t)sh[j] * N + i];
     double dmax = 0.0;
     for (int sw = 0; sw < a.sweeps; ++sw) {
         for (int j = 0; j < k; ++j) {
-            double *us = a.u + (size_t)sh[j] * N;
+            double *us = u + (size_t)j * N;
             for (int i = threadIdx.x; i < N; i += blockDim.x) x[i] = us[i];
             __syncthreads();
-            gs_deflate(a, sh, j, x, red);
+            gs_deflate(a, u, j, x, red);
             const double nx = sqrt(gs_dot(x, x, N, red));
             for (int i = threadIdx.x; i < N; i += blockDim.x) x[i] /= nx;
             __syncthreads();
-            gs_apply_h(a, l, x, hx, scr);
+            gs_apply_h<TEAM>(a, tm, l, x, hx, scr);
             __syncthreads();
             const double theta = gs_dot(x, hx, N, red);
             for (int i = threadIdx.x; i < N; i += blockDim.x) hw[i] = hx[i] - theta * x[i];  // residual
             __syncthreads();
-            gs_precondition(a, g, theta, hw, tmp, w, scr);
-            gs_deflate(a, sh, j, w, red);
+            gs_precondition<TEAM>(a, tm, g, theta, hw, tmp, w, scr);
+            gs_deflate(a, u, j, w, red);
             const double cx = gs_dot(x, w, N, red);
             for (int i = threadIdx.x; i < N; i += blockDim.x) w[i] -= cx * x[i];
             __syncthreads();
@@ -4715,7 +4859,7 @@ __global__ __launch_bounds__(GS_WG) void k_gs_sweep(GsArgs a) {
             if (nw > 1e-300) {
                 for (int i = threadIdx.x; i < N; i += blockDim.x) w[i] /= nw;
                 __syncthreads();
-                gs_apply_h(a, l, w, hw, scr);
+                gs_apply_h<TEAM>(a, tm, l, w, hw, scr);
                 __syncthreads();
                 const double b = gs_dot(x, hw, N, red);
                 const double c = gs_dot(w, hw, N, red);
@@ -4746,11 +4890,14 @@ __global__ __launch_bounds__(GS_WG) void k_gs_sweep(GsArgs a) {
                 const double e = gs_dot(x, hx, N, red);
                 dmax = fmax(dmax, fabs(e - a.eps[sh[j]]));
                 __syncthreads();
-                if (threadIdx.x == 0) a.eps[sh[j]] = e;
+                if (tm.me == 0) {
+                    if (threadIdx.x == 0) a.eps[sh[j]] = e;
+                    for (int i = threadIdx.x; i < N; i += blockDim.x) a.u[(size_t)sh[j] * N + i] = us[i];
+                }
             }
         }
     }
-    if (threadIdx.x == 0) a.res[1 + g] = dmax;
+    if (tm.me == 0 && threadIdx.x == 0) a.res[1 + g] = tm.ok ? dmax : -1.0;
 }
 
 extern "C" int ggb_ground_state(const ggb_gs_problem *p, const int32_t *shell_l, const double *occ,
@@ -4815,9 +4962,24 @@ extern "C" int ggb_ground_state(const ggb_gs_problem *p, const int32_t *shell_l,
     hipStream_t st = nullptr;
     double *dr = nullptr, *dwr = nullptr, *dT = nullptr, *dlam = nullptr, *docc = nullptr, *du = nullptr,
            *deps = nullptr, *dv = nullptr, *drho = nullptr, *dres = nullptr;
+    double *dex = nullptr, *dpriv = nullptr;
     float *dQ = nullptr, *dQT = nullptr;
     int32_t *dgsh = nullptr, *dgl = nullptr;
     int rc = GGB_OK;
+    // teams of the sweep kernel, and where each work-group keeps its shells
+    int kmax = 0;
+    for (int g = 0; g < G; ++g) {
+        int k = 0;
+        while (k < GS_MAX_K && gsh[(size_t)g * GS_MAX_K + k] >= 0) ++k;
+        kmax = std::max(kmax, k);
+    }
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) != hipSuccess) cus = 1;
+    const int tmax = N < GS_TEAM_MIN_N ? 1 : std::max(1, std::min(64, std::min(GS_MAX_WG, cus - cus / 8) / G));
+    const int rows = tmax == 1 ? N : ((N + tmax - 1) / tmax + GS_ROWS - 1) / GS_ROWS * GS_ROWS;  // whole lines of the exchange
+    const int team = (N + rows - 1) / rows;
+    const size_t lds5 = (size_t)5 * N * sizeof(double), ldsu = (size_t)(5 + kmax) * N * sizeof(double);
+    const bool in_lds = ldsu <= GS_LDS_MAX;
     auto hip = [&](hipError_t e, const char *what) {
         if (e != hipSuccess && rc == GGB_OK) {
             g_create_err = std::string("ggb_ground_state: ") + what + ": " + hipGetErrorString(e);
@@ -4837,6 +4999,8 @@ extern "C" int ggb_ground_state(const ggb_gs_problem *p, const int32_t *shell_l,
         hip(dalloc(&du, (size_t)ns * N), "alloc") && hip(dalloc(&deps, ns), "alloc") &&
         hip(dalloc(&dv, N), "alloc") && hip(dalloc(&drho, N), "alloc") && hip(dalloc(&dres, 1 + G), "alloc") &&
         hip(dalloc(&dgsh, (size_t)G * GS_MAX_K), "alloc") && hip(dalloc(&dgl, G), "alloc") &&
+        hip(dalloc(&dex, (size_t)G * 3 * N), "alloc") &&
+        (in_lds || hip(dalloc(&dpriv, (size_t)G * team * GS_MAX_K * N), "alloc")) &&
         up(dr, r, N * 8) && up(dwr, wr, N * 8) && up(dT, T, NN * 8) && up(dQ, q0f.data(), (size_t)G * NN * 4) &&
         up(dQT, q0t.data(), (size_t)G * NN * 4) && up(dlam, lam0, (size_t)G * N * 8) &&
         up(docc, occ, ns * 8) && up(du, u0.data(), (size_t)ns * N * 8) && up(deps, einit.data(), ns * 8) &&
@@ -4847,18 +5011,33 @@ extern "C" int ggb_ground_state(const ggb_gs_problem *p, const int32_t *shell_l,
         a.N = N, a.n_shell = ns, a.n_group = G, a.sweeps = p->sweeps, a.interacting = p->interacting ? 1 : 0;
         a.Z = p->Z, a.mix = p->mix, a.gamma = p->gamma;
         a.final_ = 0;
-        const size_t lds = (size_t)5 * N * sizeof(double);
+        a.ex = dex, a.priv = dpriv, a.team = team, a.rows = rows;
         std::vector<double> res(1 + G);
         for (it = 1; it <= p->max_iter; ++it) {
             a.first = it == 1;
             k_gs_potential<<<1, GS_WG, 0, st>>>(a);
-            k_gs_sweep<<<G, GS_WG, lds, st>>>(a);
+            void *args[] = {&a};
+            // one set of teams on the device at a time: two could each hold a part of it and wait
+            static std::mutex teams;
+            std::unique_lock<std::mutex> alone(teams, std::defer_lock);
+            if (team > 1) alone.lock();
             if (!hip(hipGetLastError(), "launch") ||
+                !hip(hipLaunchCooperativeKernel(reinterpret_cast<const void *>(team == 1 ? k_gs_sweep<false, true>
+                                                                               : in_lds  ? k_gs_sweep<true, true>
+                                                                                         : k_gs_sweep<true, false>),
+                                                dim3(G * team), dim3(GS_WG), args, (unsigned)(in_lds ? ldsu : lds5), st),
+                     "launch") ||
                 !hip(hipMemcpyAsync(res.data(), dres, (1 + G) * 8, hipMemcpyDeviceToHost, st), "download") ||
                 !hip(hipStreamSynchronize(st), "sync"))
                 break;
             double de = 0.0;
-            for (int g = 0; g < G; ++g) de = std::max(de, res[1 + g]);
+            bool waited = false;  // a work-group gave up waiting for its team
+            for (int g = 0; g < G; ++g) waited |= res[1 + g] < 0.0, de = std::max(de, res[1 + g]);
+            if (waited) {
+                g_create_err = "ggb_ground_state: the device did not run all work-groups of a sweep together";
+                rc = GGB_E_HIP;
+                break;
+            }
             if (de < p->tol && res[0] < 1e3 * p->tol) {
                 conv = true;
                 break;
@@ -4877,7 +5056,8 @@ extern "C" int ggb_ground_state(const ggb_gs_problem *p, const int32_t *shell_l,
         }
     }
     for (void *d : {(void *)dr, (void *)dwr, (void *)dT, (void *)dQ, (void *)dQT, (void *)dlam, (void *)docc,
-                    (void *)du, (void *)deps, (void *)dv, (void *)drho, (void *)dres, (void *)dgsh, (void *)dgl})
+                    (void *)du, (void *)deps, (void *)dv, (void *)drho, (void *)dres, (void *)dgsh, (void *)dgl,
+                    (void *)dex, (void *)dpriv})
         if (d) (void)hipFree(d);
     if (st) (void)hipStreamDestroy(st);
     *iterations = it;
