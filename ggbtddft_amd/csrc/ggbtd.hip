@@ -1140,6 +1140,248 @@ __global__ __launch_bounds__(WG) void k_kin_bwd_dma(const float *__restrict__ Q,
 }
 
 // ---------------------------------------------------------------------------
+// Mixed form, few instances: the products, chunks and sums of k_kin_fwd_dma / k_kin_bwd_dma in the
+// same order (the same Y and psi bit for bit), operands straight from memory into registers
+// as in the FP64 passes:
+//   PASS 0: A = Q[l] (k = radial node, m = eigen index, TA tiles with interleaved rows
+//           m0 + TA (4 kr + r) + t), B = psi32, D = Y with the factor e^{-i lam dt};
+//   PASS 1: A = QT[l], quad-interleaved (kin_qt_index; k = eigen index, m = radial node, 16
+//           rows per tile), B = Y, D = psi with the ground-state component beta phi added in FP64.
+// A wave owns 16 TA rows by 16 TB real columns and goes through all of k, in chunks of 16: one
+// chunk in the MFMA accumulator, then added to a second one, K32_PD - 1 chunks of operands ahead.
+// The four waves of a work-group take neighbouring panels, which share the columns in L1;
+// there is no LDS and no barrier.
+//  * A lane loads four consecutive k as one vector where k is contiguous (columns as whole complex
+//    values, QT as a quad); an MFMA step wants k = k0 + 4 s + kr in lane row kr instead, so the
+//    two lanes of a column trade halves and four rows of 16 lanes are transposed in
+//    registers (rows_transpose).
+//  * The loads are not conditional: past the end they read the last whole chunk again, so that the
+//    compiler can count those in flight (with conditional ones it waits for all of them:
+//    neon, 12 columns 20 / 22 us instead of 13 / 12).
+// What bounds it: L2 traffic and latency.  Passes 0 / 1 against the 64 x 128 tiles: neon (N = 384,
+// 49 l) 12 columns 13 / 12 us (27 / 31), 32 columns 19 / 18 us (29 / 35); argon (512, 65 l) 14 columns
+// 24 / 23 us (50 / 58), 35 columns 42 / 40 us (52 / 60); krypton (768, 97 l) 13 columns 53 / 56 us
+// (125 / 123).  Trading the chunks of a tile between four waves through LDS, which keeps the order
+// of the sums too, was no faster (12 / 12, 18 / 20, 23 / 26, 50 / 50, 62 / 62 us).
+// ---------------------------------------------------------------------------
+#ifndef K32_PD
+#define K32_PD 3
+#endif
+// two complex values of a column; a column starts at any multiple of 8 bytes (odd N)
+typedef f4_t k32_b4_t __attribute__((aligned(8)));
+struct Kin32Args {
+    const float *A;        // PASS 0: Q [l][N][nk_max], PASS 1: QT (kin_qt_index)
+    const float2 *B;       // PASS 0: psi32 [l][C][N], PASS 1: Y [l][C][nk_max]
+    float2 *Y;             // PASS 0
+    double2 *psi;          // PASS 1
+    const double2 *kph;    // [l][nk_max] (cos, sin)(lam dt)
+    const int32_t *nkeep;  // [l]
+    KinRef ref;
+    int N, nk_max, C, n_orb;
+};
+
+// x[s] of lane row g becomes x[g] of lane row s (rows of 16 lanes): a 4 x 4 transpose
+static __device__ __forceinline__ void rows_transpose(float (&x)[4]) {
+    unsigned v[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) v[s] = __float_as_uint(x[s]);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {  // rows 2, 3 of x[s] with rows 0, 1 of x[s + 2]
+        const auto r = __builtin_amdgcn_permlane32_swap(v[s], v[s + 2], false, false);
+        v[s] = r[0];
+        v[s + 2] = r[1];
+    }
+#pragma unroll
+    for (int s = 0; s < 4; s += 2) {  // odd rows of x[s] with even rows of x[s + 1]
+        const auto r = __builtin_amdgcn_permlane16_swap(v[s], v[s + 1], false, false);
+        v[s] = r[0];
+        v[s + 1] = r[1];
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) x[s] = __uint_as_float(v[s]);
+}
+
+template <int PASS, int TA, int TB>
+__global__ __launch_bounds__(WG) void k_kin32(Kin32Args g) {
+    typedef float vta __attribute__((ext_vector_type(TA)));
+    const tile3 tb = xcd_tile();  // (group of 4 row panels, column group, l): they share the columns
+    const int l = tb.z;
+    const int nk = g.nkeep[l];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int m0 = (tb.x * 4 + wave) * 16 * TA;
+    if (m0 >= (PASS ? g.N : nk)) return;  // per wave: there is no barrier below
+    const int n0 = tb.y * 16 * TB;
+    if (!kin_cols_active(g.ref.active, n0, 16 * TB, g.C, g.n_orb)) return;  // idle instances only
+    const int kr = lane >> 4, lc = lane & 15, p = lc & 1;
+    const int N = g.N, C = g.C, nkm = g.nk_max;
+    const int K = PASS ? min(nkm, (nk + 15) & ~15) : N;
+    const int ldb = PASS ? nkm : N;
+    // operand addresses: a base of the work-group and the chunk, and a byte offset of the lane (below
+    // 2^32: N and nk_max <= 4096, C <= 65535)
+    const char *Ab = reinterpret_cast<const char *>(g.A + (size_t)l * N * nkm);
+    const char *Bb = reinterpret_cast<const char *>(g.B + (size_t)l * C * ldb);
+    unsigned ao[PASS ? TA : 1], col[TB];
+    if constexpr (PASS == 0) {
+        // panel rows past the row length read its first rows: their outputs are not stored
+        ao[0] = 4u * (unsigned)(m0 + TA * lc < nkm ? m0 + TA * lc : 0);
+    } else {
+#pragma unroll
+        for (int t = 0; t < TA; ++t) {
+            const int i = m0 + 16 * t + lc;  // rows i >= N read row 0 and are not stored
+            ao[t] = 16u * (unsigned)(kr * N + (i < N ? i : 0));
+        }
+    }
+    int c[TB];
+#pragma unroll
+    for (int q = 0; q < TB; ++q) {
+        c[q] = (n0 + 16 * q + lc) >> 1;      // columns c >= C read column 0 and are not stored
+        col[q] = 8u * (unsigned)(c[q] < C ? c[q] : 0) * (unsigned)ldb;
+    }
+    float av[K32_PD][4][TA];
+    f4_t bv[K32_PD][TB];
+    // whole chunk n into buffer b
+    auto load = [&](int b, int n) {
+        const int k0 = 16 * n;
+        if constexpr (PASS == 0) {
+            const unsigned row = 4u * (unsigned)(kr * nkm);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const vta v = *reinterpret_cast<const vta *>(Ab + (size_t)4 * (k0 + 4 * s) * nkm + (row + ao[0]));
+#pragma unroll
+                for (int t = 0; t < TA; ++t) av[b][s][t] = v[t];
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < TA; ++t) {
+                const f4_t v = *reinterpret_cast<const f4_t *>(Ab + (size_t)4 * k0 * N + ao[t]);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) av[b][s][t] = v[s];
+            }
+        }
+        const unsigned off = 8u * (unsigned)(4 * kr + 2 * p);
+#pragma unroll
+        for (int q = 0; q < TB; ++q) bv[b][q] = *reinterpret_cast<const k32_b4_t *>(Bb + (size_t)8 * k0 + (col[q] + off));
+    };
+    f4_t acc[TB][TA], hi[TB][TA];
+#pragma unroll
+    for (int q = 0; q < TB; ++q)
+#pragma unroll
+        for (int t = 0; t < TA; ++t) hi[q][t] = (f4_t){0, 0, 0, 0};
+    auto chunk = [&](int b) {
+        float bs[TB][4];
+#pragma unroll
+        for (int q = 0; q < TB; ++q) {
+            // component p of the column's four values k0 + 4 kr + 0..3
+            const f4_t v = bv[b][q];
+            const float o0 = lane_xor1(p ? v[0] : v[1]), o1 = lane_xor1(p ? v[2] : v[3]);
+            bs[q][0] = p ? o0 : v[0];
+            bs[q][1] = p ? o1 : v[2];
+            bs[q][2] = p ? v[1] : o0;
+            bs[q][3] = p ? v[3] : o1;
+            rows_transpose(bs[q]);  // now of k0 + 4 s + kr, s = 0..3
+        }
+        if constexpr (PASS == 1) {
+#pragma unroll
+            for (int t = 0; t < TA; ++t) {
+                float x[4] = {av[b][0][t], av[b][1][t], av[b][2][t], av[b][3][t]};
+                rows_transpose(x);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) av[b][s][t] = x[s];
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int q = 0; q < TB; ++q)
+#pragma unroll
+                for (int t = 0; t < TA; ++t)
+                    acc[q][t] = mfma_t<float>::op(av[b][s][t], bs[q][s], s ? acc[q][t] : (f4_t){0, 0, 0, 0});
+#pragma unroll
+        for (int q = 0; q < TB; ++q)
+#pragma unroll
+            for (int t = 0; t < TA; ++t) hi[q][t] += acc[q][t];
+    };
+    const int nfull = K / 16;
+    if (nfull > 0) {
+#pragma unroll
+        for (int b = 0; b < K32_PD - 1; ++b) load(b, min(b, nfull - 1));
+        for (int n = 0; n < nfull; n += K32_PD) {
+#pragma unroll
+            for (int b = 0; b < K32_PD; ++b) {
+                load((b + K32_PD - 1) % K32_PD, min(n + b + K32_PD - 1, nfull - 1));
+                if (n + b < nfull) chunk(b);
+            }
+        }
+    }
+    if constexpr (PASS == 0) {
+        const int k0 = 16 * nfull;
+        if (k0 < K) {  // a ragged N: rows k >= N count as zero through the table operand
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int k = k0 + 4 * s + kr;
+                const vta v = *reinterpret_cast<const vta *>(Ab + (size_t)4 * min(k, N - 1) * nkm + ao[0]);
+#pragma unroll
+                for (int t = 0; t < TA; ++t) av[0][s][t] = k < N ? v[t] : 0.f;
+            }
+#pragma unroll
+            for (int q = 0; q < TB; ++q) {
+                const float2 *cp = reinterpret_cast<const float2 *>(Bb + col[q]);
+                const int ka = k0 + 4 * kr + 2 * p;
+                const float2 u = cp[min(ka, N - 1)], v = cp[min(ka + 1, N - 1)];
+                bv[0][q] = (f4_t){u.x, u.y, v.x, v.y};
+            }
+            chunk(0);
+        }
+    }
+    // a lane holds component p of 4 TA consecutive rows (PASS 0: m0 + 4 TA kr + TA r + t) or of 4
+    // per tile (PASS 1: m0 + 16 t + 4 kr + r); the lanes of a column trade halves and store complex values
+#pragma unroll
+    for (int q = 0; q < TB; ++q) {
+        const bool cok = c[q] < C;
+        if constexpr (PASS == 0) {
+            float2 *Yc = g.Y + ((size_t)l * C + (cok ? c[q] : 0)) * nkm;
+#pragma unroll
+            for (int j = 0; j < 2 * TA; ++j) {
+                // rows j (p = 0) and j + 2 TA (p = 1) of the lane's 4 TA
+                const float a0 = hi[q][j % TA][j / TA], a1 = hi[q][(j + 2 * TA) % TA][(j + 2 * TA) / TA];
+                const float own = p ? a1 : a0, o = lane_xor1(p ? a0 : a1);
+                const double re = p ? o : own, im = p ? own : o;
+                const int m = m0 + 4 * TA * kr + j + 2 * TA * p;
+                if (!cok) continue;
+                if (m < nk) {
+                    const double2 f = g.kph[(size_t)l * nkm + m];
+                    Yc[m] = make_float2((float)(f.x * re + f.y * im), (float)(f.x * im - f.y * re));
+                } else if (m < nkm && m < ((nk + 15) & ~15)) {
+                    Yc[m] = make_float2(0.f, 0.f);  // pass 1 reads Y up to there
+                }
+            }
+        } else {
+            double cre = 0.0, cim = 0.0;
+            const double *rrow = cok ? kin_ref_row(g.ref, l, c[q], 0, N, g.n_orb, true, &cre) : nullptr;
+            if (rrow) (void)kin_ref_row(g.ref, l, c[q], 1, N, g.n_orb, true, &cim);
+            double2 *Xc = g.psi + ((size_t)l * C + (cok ? c[q] : 0)) * N;
+#pragma unroll
+            for (int t = 0; t < TA; ++t)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const float a0 = hi[q][t][j], a1 = hi[q][t][j + 2];
+                    const float own = p ? a1 : a0, o = lane_xor1(p ? a0 : a1);
+                    double re = p ? o : own, im = p ? own : o;
+                    const int i = m0 + 16 * t + 4 * kr + j + 2 * p;
+                    if (cok && i < N) {
+                        if (rrow) {
+                            const double f = rrow[i];
+                            re += cre * f;
+                            im += cim * f;
+                        }
+                        Xc[i] = make_double2(re, im);
+                    }
+                }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Compensated split-FP32 kinetic passes (precision 2).  Every FP64 operand is
 // split into FP32 parts, v = v_hi + v_lo with v_hi = fl32(v), v_lo =
 // fl32(v - v_hi), and a product a b is formed as a_hi b_hi + a_hi b_lo +
@@ -3303,6 +3545,48 @@ static void launch_kin64(ggb_ctx *ctx, int pass, hipEvent_t e0, hipEvent_t e1) {
 
 // e0/e1 (optional): events stamped with the start and end of the pass's
 // product kernel itself, for the kernel-duration timing
+template <int TA, int TB>
+static void launch_kin32_t(ggb_ctx *ctx, int pass, const KinRef &ref, hipEvent_t e0, hipEvent_t e1) {
+    const ggb_problem &p = ctx->p;
+    Kin32Args g;
+    g.A = reinterpret_cast<const float *>(pass ? ctx->QT : ctx->Q);
+    g.Y = reinterpret_cast<float2 *>(ctx->Y);
+    g.B = pass ? g.Y : ctx->psi32;
+    g.psi = reinterpret_cast<double2 *>(ctx->psi);
+    g.kph = ctx->kph;
+    g.nkeep = ctx->nkeep;
+    g.ref = ref;
+    g.N = p.n_r;
+    g.nk_max = p.nk_max;
+    g.C = ctx->C;
+    g.n_orb = p.n_orb;
+    const int rows = pass ? p.n_r : p.nk_max;
+    const dim3 grid((rows + 64 * TA - 1) / (64 * TA), (2 * g.C + 16 * TB - 1) / (16 * TB), p.n_l);
+    if (pass)
+        kin_launch(k_kin32<1, TA, TB>, grid, WG, ctx->stream, e0, e1, g);
+    else
+        kin_launch(k_kin32<0, TA, TB>, grid, WG, ctx->stream, e0, e1, g);
+}
+
+// TILED16 up to K32_MAX_C columns; beyond, the 64 x 128 tiles waste less than the half-width column
+// groups cost (argon, passes 0 / 1: 35 columns 42 / 40 against 52 / 60 us, 63 columns 64 / 60
+// against 53 / 61; krypton, 52 columns 151 / 137 against 130 / 144)
+#define K32_MAX_C 40
+// Shape by the number of 16 x 16 output tiles of a pass.  Up to about four waves per SIMD one tile per
+// wave (neon, 32 columns, 4116 tiles: 19 / 18 us; two rows of tiles 21 / 18, four 24 / 21); with more, operand
+// traffic counts: 2 x 2 tiles for one pair of column tiles (krypton, 13 columns, 7372 tiles: 53 / 56
+// against 73 / 59), 4 x 1 for more columns (argon, 35 columns, 8775 tiles: 42 / 40 against 45 / 45).
+static void launch_kin32(ggb_ctx *ctx, int pass, const KinRef &ref, hipEvent_t e0, hipEvent_t e1) {
+    const int nct = (2 * ctx->C + 15) / 16;
+    const long tiles = (long)(ctx->p.nk_max / 16) * nct * ctx->p.n_l;
+    if (tiles <= 5000)
+        launch_kin32_t<1, 1>(ctx, pass, ref, e0, e1);
+    else if (nct <= 2)
+        launch_kin32_t<2, 2>(ctx, pass, ref, e0, e1);
+    else
+        launch_kin32_t<4, 1>(ctx, pass, ref, e0, e1);
+}
+
 static void launch_kinetic_mixed(ggb_ctx *ctx, int pass, bool fresh, hipEvent_t e0, hipEvent_t e1) {
     const ggb_problem &p = ctx->p;
     const float *Q = reinterpret_cast<const float *>(ctx->Q);
@@ -3342,6 +3626,7 @@ static void launch_kinetic_mixed(ggb_ctx *ctx, int pass, bool fresh, hipEvent_t 
         if (pass == 0 && !(fresh && !ref.phi))
             k_kin_prep<<<dim3((p.n_r + WG - 1) / WG, ctx->C, fresh ? 1 : p.n_l), WG, 0, ctx->stream>>>(
                 (const double2 *)ctx->psi, ref, ctx->psi32, p.n_r, ctx->C, p.n_orb, fresh ? 1 : 0);
+        if (var == GGB_KIN_TILED16 && ctx->C <= K32_MAX_C) return launch_kin32(ctx, pass, ref, e0, e1);
         const bool k32 = var == GGB_KIN_TILED32;
         const double2 *kph = ctx->kph;
         const int32_t *nkeep = ctx->nkeep;

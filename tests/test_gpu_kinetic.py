@@ -51,3 +51,49 @@ def test_fp64_passes_at_tile_edges(N, columns):
             prop.substep(1)
             got = prop.download_orbitals()
         assert np.abs(got - ref).max() < 4 * N * 2.0 ** -53, (variant, np.abs(got - ref).max())
+
+
+def _mixed(S, psi, columns, variant):
+    from ggbtddft_amd.engine import Propagator
+    with Propagator(S, n_inst=columns, precision=1) as prop:
+        prop.set_field(np.zeros(1))
+        prop.set_kinetic_variant(variant)
+        prop.upload_orbitals(psi)
+        prop.substep(1)
+        return prop.download_orbitals()
+
+
+# The mixed form at the edges of its few-column kernel (9 to 40 columns) and just outside it.  Its
+# columns are independent and every shape forms the same sums in the same order, so a column's
+# result is the same bit for bit whatever the number of columns.  Against numpy: the ground-state
+# component is advanced in FP64, the remainder (norm <= 1) in FP32 with chunk sums of 16, tables
+# and columns rounded once: 2 (rounding of both operands) + 16 + N / 16 roundings per pass at most,
+# two passes, so 4 (18 + N / 16) eps32.
+@pytest.mark.parametrize("N", [96, 75, 52, 21])
+def test_mixed_passes_at_tile_edges(N):
+    print("case: mixed kinetic passes, N", N, flush=True)
+    S = _system(N)
+    psi = _random_columns(S, 48)
+    ref = _kinetic(S, psi)
+    wide = _mixed(S, psi, 48, "tiled16")
+    assert np.abs(wide - ref).max() < 4 * (18 + N / 16) * 2.0 ** -24
+    for columns in (40, 33, 17, 9):
+        got = _mixed(S, psi[:, :columns].copy(), columns, "tiled16")
+        assert np.array_equal(got, wide[:, :columns]), (columns, np.abs(got - wide[:, :columns]).max())
+
+
+def test_mixed_passes_large_shapes():
+    """The 2 x 2 and 4 x 1 tile shapes, which a pass with many output tiles takes (N = 330, 128 l, 12 to 40 columns)."""
+    print("case: mixed kinetic passes, 2 x 2 and 4 x 1 tiles", flush=True)
+    S = AtomSystem("Ne", 330, 60.0, 127, 0.05, ground_state="device", tables="device")
+    rng = np.random.default_rng(5)
+    psi = rng.standard_normal((S.n_l, 44, S.N)) + 1j * rng.standard_normal((S.n_l, 44, S.N))
+    psi /= np.linalg.norm(psi, axis=2, keepdims=True)
+
+    def run(inst):
+        return _mixed(S, np.ascontiguousarray(psi[:, :4 * inst]), inst, "tiled16")
+    wide = run(11)
+    assert np.abs(wide - _kinetic(S, psi)).max() < 4 * (18 + S.N / 16) * 2.0 ** -24
+    for inst in (10, 4, 3):
+        got = run(inst)
+        assert np.array_equal(got, wide[:, :4 * inst]), inst
