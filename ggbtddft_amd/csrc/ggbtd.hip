@@ -2677,11 +2677,22 @@ struct DvEpi {
 // ---------------------------------------------------------------------------
 // HHG spectrum on the device (analysis.py:447-460, internal.py:361-379):
 // Kaiser window (sym = False), optional 8th-order central second difference,
-// zero padding by n_pad * n on each side (M = (2 n_pad + 1) n points),
+// zero padding by n_pad * n on each side (M = P n points, P = 2 n_pad + 1),
 // |fftshift(fft(fftshift(x)))|^2, and the super-Gaussian harmonic masks of
-// argonInSitu/arg.py:42-67.  M is any length: the DFT is Bluestein's
-// algorithm, X_k = w_k sum_j (y_j w_j) conj(w_{k-j}), w_j = e^{-i pi j^2 / M},
-// with the convolution done by radix-2 Stockham FFTs of length L >= 2M - 1.
+// argonInSitu/arg.py:42-67.
+//   |X|^2 does not see the shift of the padded signal, so X_q = sum_{k<n} x_k e^{-2 pi i k q/M} over the
+// n samples alone, and with q = P s + t that is one DFT of length n over s for each t:
+//     X_{P s + t} = sum_k (x_k e^{-2 pi i k t/M}) e^{-2 pi i k s/n}.
+// The signal is real, so |X_{M-q}| = |X_q| and t = 0..n_pad are enough (t and P - t mirror each
+// other).  n is any length: each DFT is Bluestein's algorithm, X_s = w_s sum_k (.. w_k) conj(w_{s-k}),
+// w_j = e^{-i pi j^2/n}, as a convolution by FFTs of length L >= 2 n - 1; |w_s| = 1 drops out.
+//   One FFT of length 2^m runs in ceil(m / 9) passes (k_spec_fft).  The forward passes leave the
+// values in digit-reversed order and the inverse ones take them in it, and the product with
+// the chirp's transform is made in between on the tile in LDS: nothing is transposed.  The first
+// pass makes its inputs from x, the last one stores |.|^2.
+//   For 44,128 samples (P = 17, L = 2^17) the kernels take 117 us where 3 FFTs of length 2^21 in 63
+// radix-2 passes and their chirps took 815 us.  What is left of the call is the copy of the
+// spectrum to the host, its frequency axis and the allocation.
 // ---------------------------------------------------------------------------
 static __device__ double bessel_i0(double x) {
     // power series sum_k ((x/2)^2)^k / (k!)^2, all terms positive
@@ -2718,74 +2729,190 @@ __global__ __launch_bounds__(WG) void k_spec_fd8(const double *__restrict__ x,
     y[j] = v * inv_dt2;
 }
 
-// e^{sign i pi j^2 / M}, with j^2 reduced mod 2M exactly
-static __device__ double2 chirp(long j, long M, double sign) {
-    const long r = (j * j) % (2 * M);
+#define SF_W 8       // columns of a tile (128-byte runs of a strided pass)
+#define SF_RMAX 9    // bits of a pass at most: 512 x 9 complex values are 74 KB of LDS
+#define SF_EPT 16    // values per thread at most: 512 x 8 / 256
+struct SpecFft {
+    double2 *buf;         // transforms of length 2^m
+    const double2 *F;     // chirp transform (mid)
+    const double *x;      // windowed signal [n] (gen)
+    double *power;        // [M] (out)
+    long n, M, ncols;     // ncols: columns of this pass, over all transforms
+    int m, lo, r;         // index bits lo .. lo + r - 1 are this pass's
+    int P, filter;        // gen: transform `filter` holds the chirp, the others are t = 0, 1, ..
+    int gen, fwd, mid, inv, out;
+};
+
+// e^{-2 pi i k / 2^bits}
+static __device__ __forceinline__ double2 sf_root(long k, int bits) {
     double s, c;
-    sincospi(sign * (double)r / (double)M, &s, &c);
+    sincospi(-2.0 * (double)k / (double)(1L << bits), &s, &c);
     return make_double2(c, s);
 }
+static __device__ __forceinline__ double2 sf_mul(double2 a, double2 b) {
+    return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+}
 
-// a_j = y_j w_j for j < M (y = fftshift of the padded signal), zero up to L
-__global__ __launch_bounds__(WG) void k_blue_a(const double *__restrict__ x, double2 *__restrict__ a,
-                                               int n, int n_pad, long M, long L) {
-    const long j = (long)blockIdx.x * WG + threadIdx.x;
-    if (j >= L) return;
-    double2 v = make_double2(0.0, 0.0);
-    if (j < M) {
-        const long i = (j - M / 2 + M) % M;       // index into the padded signal
-        const long k = i - (long)n_pad * n;       // index into x
-        if (k >= 0 && k < n) {
-            const double2 w = chirp(j, M, -1.0);
-            v = make_double2(x[k] * w.x, x[k] * w.y);
+// DFT over the 2^r rows of every column of the tile, natural order in and out (Stockham: one radix-2
+// stage if r is odd, then radix 4), sign -1 (fwd) or +1; tw[i] = e^{-2 pi i i / 2^r}
+static __device__ void sf_tile_fft(double2 *X, const double2 *tw, int r, bool fwd) {
+    const int R = 1 << r, t = threadIdx.x;
+    constexpr int PI = SF_W + 1;
+    int Ns = 1;
+    if (r & 1) {
+        double2 v[SF_EPT / 2][2];
+        const int nb = R / 2 * SF_W;
+#pragma unroll
+        for (int e = 0; e < SF_EPT / 2; ++e) {
+            const int b = t + WG * e, w = b % SF_W, j = b / SF_W;
+            if (b < nb) {
+                const double2 p = X[j * PI + w], q = X[(j + R / 2) * PI + w];
+                v[e][0] = make_double2(p.x + q.x, p.y + q.y);
+                v[e][1] = make_double2(p.x - q.x, p.y - q.y);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < SF_EPT / 2; ++e) {
+            const int b = t + WG * e, w = b % SF_W, j = b / SF_W;
+            if (b < nb) X[2 * j * PI + w] = v[e][0], X[(2 * j + 1) * PI + w] = v[e][1];
+        }
+        __syncthreads();
+        Ns = 2;
+    }
+    const int nb = R / 4 * SF_W;
+    for (; Ns < R; Ns *= 4) {
+        double2 v[SF_EPT / 4][4];
+        const int step = R / (4 * Ns);
+#pragma unroll
+        for (int e = 0; e < SF_EPT / 4; ++e) {
+            const int b = t + WG * e, w = b % SF_W, j = b / SF_W, k = j & (Ns - 1);
+            if (b < nb) {
+                double2 u[4];
+                u[0] = X[j * PI + w];
+#pragma unroll
+                for (int q = 1; q < 4; ++q) {
+                    double2 z = tw[q * k * step];
+                    if (!fwd) z.y = -z.y;
+                    u[q] = sf_mul(X[(j + q * (R / 4)) * PI + w], z);
+                }
+                const double2 s0 = make_double2(u[0].x + u[2].x, u[0].y + u[2].y);
+                const double2 d0 = make_double2(u[0].x - u[2].x, u[0].y - u[2].y);
+                const double2 s1 = make_double2(u[1].x + u[3].x, u[1].y + u[3].y);
+                const double2 d1 = make_double2(u[1].x - u[3].x, u[1].y - u[3].y);
+                // -i d1 (fwd) or +i d1
+                const double2 e1 = fwd ? make_double2(d1.y, -d1.x) : make_double2(-d1.y, d1.x);
+                v[e][0] = make_double2(s0.x + s1.x, s0.y + s1.y);
+                v[e][1] = make_double2(d0.x + e1.x, d0.y + e1.y);
+                v[e][2] = make_double2(s0.x - s1.x, s0.y - s1.y);
+                v[e][3] = make_double2(d0.x - e1.x, d0.y - e1.y);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < SF_EPT / 4; ++e) {
+            const int b = t + WG * e, w = b % SF_W, j = b / SF_W, k = j & (Ns - 1);
+            if (b < nb) {
+                const int d = (j - k) * 4 + k;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) X[(d + q * Ns) * PI + w] = v[e][q];
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// One pass over index bits lo .. lo + r - 1: a tile is SF_W columns (the other index bits) of 2^r values
+// each, 2^lo apart.  fwd: the DFT over the column, then value k of a column at offset `low` times
+// e^{-2 pi i k low / 2^(lo + r)}; inv: the conjugate factors, then the inverse DFT; mid (lo = 0): fwd, times
+// F, inv.  What bounds it: the LDS exchanges of the stages and the root factors (25 us a pass over 9
+// transforms of 2^17, of which HBM needs 8).
+__global__ __launch_bounds__(WG) void k_spec_fft(SpecFft g) {
+    extern __shared__ __align__(16) double2 sf_lds[];
+    constexpr int PI = SF_W + 1;
+    const int R = 1 << g.r, t = threadIdx.x;
+    double2 *X = sf_lds, *tw = sf_lds + R * PI;
+    for (int i = t; i < R; i += WG) tw[i] = sf_root(i, g.r);
+    const long c0 = (long)blockIdx.x * SF_W;
+    const long lmask = (1L << g.lo) - 1, imask = (1L << g.m) - 1;
+    // element e of the tile: row j, column w, and its index over all transforms (-1: no such column)
+    auto place = [&](int e, int &j, int &w) -> long {
+        if (g.lo) {
+            w = e % SF_W;
+            j = e / SF_W;
+        } else {
+            j = e & (R - 1);
+            w = e >> g.r;
+        }
+        const long c = c0 + w;
+        if (c >= g.ncols) return -1;
+        return ((c >> g.lo) << (g.lo + g.r)) + ((long)j << g.lo) + (c & lmask);
+    };
+    for (int e = t; e < R * SF_W; e += WG) {
+        int j, w;
+        const long a = place(e, j, w);
+        double2 v = make_double2(0.0, 0.0);
+        if (a >= 0) {
+            if (g.gen) {
+                const long i = a & imask, L = imask + 1;
+                const int tr = (int)(a >> g.m);
+                double s, c;
+                if (tr == g.filter) {  // conj(w_i), wrapped
+                    const long k = i < g.n ? i : (i > L - g.n ? L - i : -1);
+                    if (k >= 0) {
+                        sincospi((double)((k * k) % (2 * g.n)) / (double)g.n, &s, &c);
+                        v = make_double2(c, s);
+                    }
+                } else if (i < g.n) {  // x_i e^{-i pi (P i^2 + 2 i t) / M}, the phase reduced mod 2M exactly
+                    const long ph = (g.P * i * i + 2 * i * tr) % (2 * g.M);
+                    sincospi(-(double)ph / (double)g.M, &s, &c);
+                    v = make_double2(g.x[i] * c, g.x[i] * s);
+                }
+            } else {
+                v = g.buf[a];
+                if (g.inv && !g.mid && g.lo) {
+                    double2 z = sf_root((long)j * ((c0 + w) & lmask), g.lo + g.r);
+                    z.y = -z.y;
+                    v = sf_mul(v, z);
+                }
+            }
+        }
+        X[j * PI + w] = v;
+    }
+    __syncthreads();
+    if (g.fwd) sf_tile_fft(X, tw, g.r, true);
+    if (g.mid) {
+        for (int e = t; e < R * SF_W; e += WG) {
+            int j, w;
+            const long a = place(e, j, w);
+            if (a >= 0) X[j * PI + w] = sf_mul(X[j * PI + w], g.F[a & imask]);
+        }
+        __syncthreads();
+    }
+    if (g.inv) sf_tile_fft(X, tw, g.r, false);
+    for (int e = t; e < R * SF_W; e += WG) {
+        int j, w;
+        const long a = place(e, j, w);
+        if (a < 0) continue;
+        double2 v = X[j * PI + w];
+        if (g.out) {  // power[(q + M/2) mod M] = |X_q|^2, q = P s + t, and its mirror M - q
+            const long s = a & imask, tr = a >> g.m;
+            if (s < g.n) {
+                const double sc = 1.0 / (double)(imask + 1), re = v.x * sc, im = v.y * sc;
+                const double p = re * re + im * im;
+                const long q = g.P * s + tr, h = g.M / 2;
+                const long q0 = q + h < g.M ? q + h : q + h - g.M;
+                g.power[q0] = p;
+                if (tr > 0) {
+                    const long q1 = g.M - q + h;
+                    g.power[q1 < g.M ? q1 : q1 - g.M] = p;
+                }
+            }
+        } else {
+            if (g.fwd && !g.mid && g.lo) v = sf_mul(v, sf_root((long)j * ((c0 + w) & lmask), g.lo + g.r));
+            g.buf[a] = v;
         }
     }
-    a[j] = v;
-}
-
-// b_j = conj(w_j) for |j| < M, wrapped to length L
-__global__ __launch_bounds__(WG) void k_blue_b(double2 *__restrict__ b, long M, long L) {
-    const long j = (long)blockIdx.x * WG + threadIdx.x;
-    if (j >= L) return;
-    double2 v = make_double2(0.0, 0.0);
-    if (j < M) v = chirp(j, M, 1.0);
-    else if (j > L - M) v = chirp(L - j, M, 1.0);
-    b[j] = v;
-}
-
-// one radix-2 Stockham pass (sub-transform size Ns -> 2 Ns), natural order at the end
-__global__ __launch_bounds__(WG) void k_fft_pass(const double2 *__restrict__ in,
-                                                 double2 *__restrict__ out, long L, long Ns,
-                                                 double sign) {
-    const long j = (long)blockIdx.x * WG + threadIdx.x;
-    if (j >= L / 2) return;
-    const long k = j % Ns;
-    double s, c;
-    sincospi(sign * (double)k / (double)Ns, &s, &c);
-    const double2 v0 = in[j], u = in[j + L / 2];
-    const double2 v1 = make_double2(u.x * c - u.y * s, u.x * s + u.y * c);
-    const long d = (j / Ns) * 2 * Ns + k;
-    out[d] = make_double2(v0.x + v1.x, v0.y + v1.y);
-    out[d + Ns] = make_double2(v0.x - v1.x, v0.y - v1.y);
-}
-
-__global__ __launch_bounds__(WG) void k_cmul(double2 *__restrict__ a, const double2 *__restrict__ b,
-                                             long L) {
-    const long j = (long)blockIdx.x * WG + threadIdx.x;
-    if (j >= L) return;
-    const double2 u = a[j], v = b[j];
-    a[j] = make_double2(u.x * v.x - u.y * v.y, u.x * v.y + u.y * v.x);
-}
-
-// power[q] = |X_{(q - M/2) mod M}|^2, X_k = w_k C_k / L
-__global__ __launch_bounds__(WG) void k_blue_power(const double2 *__restrict__ C,
-                                                   double *__restrict__ power, long M, long L) {
-    const long q = (long)blockIdx.x * WG + threadIdx.x;
-    if (q >= M) return;
-    const long k = (q - M / 2 + M) % M;
-    const double2 w = chirp(k, M, -1.0), cv = C[k];
-    const double xr = (w.x * cv.x - w.y * cv.y) / (double)L, xi = (w.x * cv.y + w.y * cv.x) / (double)L;
-    power[q] = xr * xr + xi * xi;
 }
 
 // intensity of harmonic `order`: sum_q exp(-((q - i0) / (0.25 (ip - im)))^32) S_q, with
@@ -4341,27 +4468,12 @@ extern "C" int ggb_get_timing(const ggb_ctx *ctx, double *ms_total, int64_t *cou
     return GGB_OK;
 }
 
-// radix-2 Stockham FFT of length L = 2^m in place of buf (tmp: scratch of L)
-static hipError_t fft_pow2(double2 *buf, double2 *tmp, long L, double sign, hipStream_t st) {
-    double2 *in = buf, *out = tmp;
-    const unsigned nb = (unsigned)((L / 2 + WG - 1) / WG);
-    for (long Ns = 1; Ns < L; Ns *= 2) {
-        k_fft_pass<<<nb, WG, 0, st>>>(in, out, L, Ns, sign);
-        double2 *t = in;
-        in = out;
-        out = t;
-    }
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess && in != buf) e = hipMemcpyAsync(buf, in, L * sizeof(double2), hipMemcpyDeviceToDevice, st);
-    return e;
-}
-
-// device buffers of one spectrum: the signal and its windowed copy (n), the
-// power spectrum (M), the three Bluestein/FFT buffers (L) and the harmonic
-// orders and intensities (n_orders)
+// device buffers of one spectrum: the signal and its windowed copy (n), the power spectrum (M), the
+// transforms ((n_pad + 2) of length L: the n_pad + 1 of the signal, then the chirp's) and the
+// harmonic orders and intensities (n_orders)
 struct SpecBufs {
     double *sig, *x, *pow, *ord, *inten;
-    double2 *A, *B, *T;
+    double2 *A;
 };
 
 static bool spec_args_ok(const double *signal, int32_t n, double dt, double beta, int32_t n_pad,
@@ -4379,10 +4491,11 @@ static bool spec_args_ok(const double *signal, int32_t n, double dt, double beta
     return true;
 }
 
-static long spec_fft_length(long M) {
-    long L = 1;
-    while (L < 2 * M - 1) L *= 2;
-    return L;
+// length of the FFTs: the power of two >= 2 n - 1
+static int spec_fft_bits(long n) {
+    int m = 0;
+    while ((1L << m) < 2 * n - 1) ++m;
+    return m;
 }
 
 // the spectrum on stream st into the buffers b; copies in and out, then
@@ -4391,7 +4504,8 @@ static int spectrum_on(const SpecBufs &b, hipStream_t st, const double *signal, 
                        int32_t differentiate, double beta, int32_t n_pad, double omega0,
                        const double *orders, int32_t n_orders, double *power, double *intensity,
                        const char *who) {
-    const long M = (2L * n_pad + 1) * n, L = spec_fft_length(M);
+    const long M = (2L * n_pad + 1) * n;
+    const int m = spec_fft_bits(n), T = n_pad + 1;
     int rc = GGB_OK;
     auto hip = [&](hipError_t e, const char *what) {
         if (e != hipSuccess && rc == GGB_OK) {
@@ -4403,31 +4517,54 @@ static int spectrum_on(const SpecBufs &b, hipStream_t st, const double *signal, 
     if (!hip(hipMemcpyAsync(b.sig, signal, (size_t)n * 8, hipMemcpyHostToDevice, st), "upload"))
         return rc;
     const unsigned gn = (unsigned)((n + WG - 1) / WG);
-    const unsigned gL = (unsigned)((L + WG - 1) / WG);
-    const unsigned gM = (unsigned)((M + WG - 1) / WG);
     k_spec_window<<<gn, WG, 0, st>>>(b.sig, b.x, n, beta);
     double *x = b.x;
     if (differentiate) {
         k_spec_fd8<<<gn, WG, 0, st>>>(b.x, b.sig, n, 1.0 / (dt * dt));
         x = b.sig;
     }
-    k_blue_a<<<gL, WG, 0, st>>>(x, b.A, n, n_pad, M, L);
-    k_blue_b<<<gL, WG, 0, st>>>(b.B, M, L);
-    if (hip(hipGetLastError(), "launch") && hip(fft_pow2(b.A, b.T, L, -1.0, st), "fft") &&
-        hip(fft_pow2(b.B, b.T, L, -1.0, st), "fft")) {
-        k_cmul<<<gL, WG, 0, st>>>(b.A, b.B, L);
-        if (hip(fft_pow2(b.A, b.T, L, 1.0, st), "inverse fft")) {
-            k_blue_power<<<gM, WG, 0, st>>>(b.A, b.pow, M, L);
-            if (n_orders > 0 &&
-                hip(hipMemcpyAsync(b.ord, orders, (size_t)n_orders * 8, hipMemcpyHostToDevice, st), "upload"))
-                k_harmonics<<<n_orders, WG, 0, st>>>(b.pow, b.ord, b.inten, M, dt, omega0);
-            if (hip(hipGetLastError(), "launch") && power)
-                hip(hipMemcpyAsync(power, b.pow, (size_t)M * 8, hipMemcpyDeviceToHost, st), "download");
-            if (rc == GGB_OK && n_orders > 0)
-                hip(hipMemcpyAsync(intensity, b.inten, (size_t)n_orders * 8, hipMemcpyDeviceToHost, st),
-                    "download");
+    // passes of at most SF_RMAX bits, the top bits first
+    const int np = (m + SF_RMAX - 1) / SF_RMAX;
+    auto pass = [&](SpecFft g, int k, int nb) {  // pass k over nb transforms
+        int hi = m;
+        for (int j = 0; j <= k; ++j) {
+            g.r = m / np + (j < m % np ? 1 : 0);
+            hi -= g.r;
         }
+        g.lo = hi;
+        g.ncols = (long)nb << (m - g.r);
+        const size_t lds = ((size_t)(SF_W + 1) + 1) * (1 << g.r) * sizeof(double2);
+        k_spec_fft<<<(unsigned)((g.ncols + SF_W - 1) / SF_W), WG, lds, st>>>(g);
+    };
+    SpecFft g;
+    g.buf = b.A;
+    double2 *F = b.A + ((size_t)T << m);
+    g.F = F;
+    g.x = x;
+    g.power = b.pow;
+    g.n = n, g.M = M, g.m = m, g.P = 2 * n_pad + 1, g.filter = T;
+    g.gen = 1, g.fwd = 1, g.mid = g.inv = g.out = 0;
+    for (int k = 0; k + 1 < np; ++k) {  // all transforms, the chirp's among them
+        pass(g, k, T + 1);
+        g.gen = 0;
     }
+    SpecFft gf = g;  // the chirp's last forward pass
+    gf.buf = F, gf.filter = 0;
+    pass(gf, np - 1, 1);
+    g.mid = g.inv = 1, g.out = np == 1;
+    pass(g, np - 1, T);
+    g.gen = g.fwd = g.mid = 0;
+    for (int k = np - 2; k >= 0; --k) {
+        g.out = k == 0;
+        pass(g, k, T);
+    }
+    if (n_orders > 0 &&
+        hip(hipMemcpyAsync(b.ord, orders, (size_t)n_orders * 8, hipMemcpyHostToDevice, st), "upload"))
+        k_harmonics<<<n_orders, WG, 0, st>>>(b.pow, b.ord, b.inten, M, dt, omega0);
+    if (hip(hipGetLastError(), "launch") && power)
+        hip(hipMemcpyAsync(power, b.pow, (size_t)M * 8, hipMemcpyDeviceToHost, st), "download");
+    if (rc == GGB_OK && n_orders > 0)
+        hip(hipMemcpyAsync(intensity, b.inten, (size_t)n_orders * 8, hipMemcpyDeviceToHost, st), "download");
     hip(hipStreamSynchronize(st), "synchronize");
     return rc;
 }
@@ -4437,30 +4574,33 @@ extern "C" int ggb_spectrum(int32_t device, const double *signal, int32_t n, dou
                             const double *orders, int32_t n_orders, double *power, double *intensity) {
     if (!spec_args_ok(signal, n, dt, beta, n_pad, omega0, orders, n_orders, intensity, "ggb_spectrum"))
         return GGB_E_ARG;
-    const long M = (2L * n_pad + 1) * n, L = spec_fft_length(M);
+    const long M = (2L * n_pad + 1) * n;
     if (hipSetDevice(device) != hipSuccess) {
         g_create_err = "ggb_spectrum: hipSetDevice failed";
         return GGB_E_HIP;
     }
     hipStream_t st = nullptr;
-    SpecBufs b = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+    double *block = nullptr;
     int rc = GGB_E_HIP;
+    // one block: the transforms (16-byte values) first
+    const size_t nA = (size_t)(n_pad + 2) << spec_fft_bits(n), no = n_orders > 0 ? n_orders : 1;
     if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) {
         g_create_err = "ggb_spectrum: stream creation failed";
-    } else if (dalloc(&b.sig, (size_t)n) != hipSuccess || dalloc(&b.x, (size_t)n) != hipSuccess ||
-               dalloc(&b.pow, (size_t)M) != hipSuccess || dalloc(&b.A, (size_t)L) != hipSuccess ||
-               dalloc(&b.B, (size_t)L) != hipSuccess || dalloc(&b.T, (size_t)L) != hipSuccess ||
-               dalloc(&b.ord, (size_t)(n_orders > 0 ? n_orders : 1)) != hipSuccess ||
-               dalloc(&b.inten, (size_t)(n_orders > 0 ? n_orders : 1)) != hipSuccess) {
+    } else if (dalloc(&block, 2 * nA + (size_t)M + 2 * (size_t)n + 2 * no) != hipSuccess) {
         g_create_err = "ggb_spectrum: device allocation failed";
         rc = GGB_E_NOMEM;
     } else {
+        SpecBufs b;
+        b.A = reinterpret_cast<double2 *>(block);
+        b.pow = block + 2 * nA;
+        b.sig = b.pow + M;
+        b.x = b.sig + n;
+        b.ord = b.x + n;
+        b.inten = b.ord + no;
         rc = spectrum_on(b, st, signal, n, dt, differentiate, beta, n_pad, omega0, orders, n_orders,
                          power, intensity, "ggb_spectrum");
     }
-    void *bufs[] = {b.sig, b.x, b.pow, b.ord, b.inten, b.A, b.B, b.T};
-    for (void *q : bufs)
-        if (q) (void)hipFree(q);
+    if (block) (void)hipFree(block);
     if (st) (void)hipStreamDestroy(st);
     return rc;
 }
@@ -4470,14 +4610,14 @@ extern "C" int ggb_spectrum(int32_t device, const double *signal, int32_t n, dou
 // device array of fixed size (each device holds its own copy until the process
 // ends).  Host code never passes the array's name to a kernel: its device
 // address is looked up once per device (hipGetSymbolAddress) and that address
-// is carved into the buffers.  Capacity: FFT length L <= 2^20, so
-// M = (2 n_pad + 1) n <= 2^19 (L >= 2M - 1), and at most 256 harmonic orders.
+// is carved into the buffers.  Capacity: M = (2 n_pad + 1) n <= 2^19, whose transforms,
+// n_pad + 2 of length L < 4 n, fit in 3 * 2^20 values, and at most 256 harmonic orders.
 // ---------------------------------------------------------------------------
 #define SPEC_NA_L (1L << 20)
 #define SPEC_NA_ORDERS 256
 #define SPEC_NA_DEVICES 64
 static constexpr size_t SPEC_NA_BYTES =
-    3 * (size_t)SPEC_NA_L * sizeof(double2)          // A, B, T
+    3 * (size_t)SPEC_NA_L * sizeof(double2)          // transforms
     + 3 * (size_t)(SPEC_NA_L / 2) * sizeof(double)   // sig, x (n <= M), pow (M <= L / 2)
     + 2 * (size_t)SPEC_NA_ORDERS * sizeof(double);   // orders, intensities
 static __device__ __align__(256) unsigned char scratch[SPEC_NA_BYTES];
@@ -4492,8 +4632,8 @@ extern "C" int ggb_spectrum_noalloc(int32_t device, const double *signal, int32_
                       "ggb_spectrum_noalloc"))
         return GGB_E_ARG;
     const long M = (2L * n_pad + 1) * n;
-    if (spec_fft_length(M) > SPEC_NA_L || n_orders > SPEC_NA_ORDERS) {
-        g_create_err = "ggb_spectrum_noalloc: (2 n_pad + 1) n must be <= 2^19 (FFT length <= 2^20) "
+    if (M > SPEC_NA_L / 2 || n_orders > SPEC_NA_ORDERS) {
+        g_create_err = "ggb_spectrum_noalloc: (2 n_pad + 1) n must be <= 2^19 "
                        "and n_orders <= 256; use ggb_spectrum for larger spectra";
         return GGB_E_ARG;
     }
@@ -4521,9 +4661,7 @@ extern "C" int ggb_spectrum_noalloc(int32_t device, const double *signal, int32_
     }
     SpecBufs b;
     b.A = reinterpret_cast<double2 *>(base);
-    b.B = b.A + SPEC_NA_L;
-    b.T = b.B + SPEC_NA_L;
-    b.sig = reinterpret_cast<double *>(b.T + SPEC_NA_L);
+    b.sig = reinterpret_cast<double *>(b.A + 3 * SPEC_NA_L);
     b.x = b.sig + SPEC_NA_L / 2;
     b.pow = b.x + SPEC_NA_L / 2;
     b.ord = b.pow + SPEC_NA_L / 2;

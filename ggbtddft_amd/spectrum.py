@@ -13,8 +13,8 @@ argonInSitu/argonInSitu/arg.py:42-67; ``cutoff_energy`` is 3.17 U_p + I_p
 (internal.py:203).
 
 ``device_spectrum`` computes the same power spectrum and harmonic intensities
-on the GPU (``ggb_spectrum``: window, difference, Bluestein DFT of any length
-on radix-2 Stockham FFTs, masks), for the serving path's time-to-spectrum.
+on the GPU (``ggb_spectrum``: window, difference, Bluestein DFTs of any length
+of the samples by FFTs, masks), for the serving path's time-to-spectrum.
 """
 import threading
 

@@ -297,8 +297,8 @@ int ggb_spectrum(int32_t device, const double *signal, int32_t n, double dt,
  * that forbid hipMalloc).  No counterpart in the reference.  Same arguments,
  * results and errors as ggb_spectrum (bit for bit), computed on the legacy
  * stream in a fixed device scratch of 60 MiB that each device holds from its
- * first call until the process ends.  Limits: (2 n_pad + 1) n <= 2^19 (FFT
- * length <= 2^20; e.g. n <= 30840 samples at n_pad = 8) and n_orders <= 256,
+ * first call until the process ends.  Limits: (2 n_pad + 1) n <= 2^19
+ * (e.g. n <= 30840 samples at n_pad = 8) and n_orders <= 256,
  * else GGB_E_ARG with a message.  All calls on one device share the scratch:
  * calls that overlap on one device race (serialise them); the scratch keeps
  * the last call's contents, and every buffer is written before it is read. */
