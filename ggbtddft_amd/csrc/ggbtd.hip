@@ -4929,7 +4929,9 @@ extern "C" int ggb_selftest_copy(int32_t device, uint64_t bytes, double *ms) {
 #define GS_TEAM_MIN_N 144  // below, a group's products stay in one work-group
 #define GS_MAX_WG 224   // work-groups of all teams (7/8 of the CUs: they wait for each other, so all are resident)
 #define GS_LDS_MAX 98304  // the shells are kept in LDS too up to this size
-#define GS_WAIT 1000000000LL  // ticks of the 100 MHz clock after which a wait gives up (10 s)
+#ifndef GS_WAIT
+#define GS_WAIT 200000000LL  // ticks of the 100 MHz clock after which a wait gives up (2 s)
+#endif
 #define GS_MAX_K 8      // shells per l group
 
 struct GsArgs {
@@ -4943,7 +4945,9 @@ struct GsArgs {
     double *res;         // [0] max |v_out - v|, [1 + g] max |eps - eps_prev| of group g
     double *ex;          // [n_group][3][N] product vectors in exchange between a team's work-groups
     double *priv;        // [n_group][team][GS_MAX_K][N] each work-group's shells, or null (kept in LDS)
+    int32_t *ticket;     // work-groups of the sweep started so far
     int team, rows;      // work-groups per group, rows of a product of each
+    int redo;            // only the groups with res[1 + g] < 0, whose team gave up waiting
     int N, n_shell, n_group, sweeps, interacting, first, final_;
     double Z, mix, gamma;
 };
@@ -5028,6 +5032,7 @@ __global__ __launch_bounds__(GS_WG) void k_gs_potential(GsArgs a) {
     const int t = threadIdx.x, nt = blockDim.x, N = a.N;
     // the sweep that follows starts with empty exchange slots
     for (int k = t; k < a.n_group * 3 * N; k += nt) a.ex[k] = gs_empty();
+    if (t == 0) *a.ticket = 0;
     // thread t owns the radial chunk [i0, i1)
     const int ch = (N + nt - 1) / nt;
     const int i0 = min(N, t * ch), i1 = min(N, i0 + ch);
@@ -5118,9 +5123,15 @@ static __device__ void gs_colsum(const TE *M, const double *x, int N, double *ou
 // work-group its own rows, when phase n is complete (then every work-group has
 // read it) and before its rows of phase n + 1 are written, so whoever reaches phase
 // n + 2 finds it empty or filled anew.  Values go through agent-scope atomic
-// stores and loads, as the team spreads over XCDs with an L2 each.  The launch is
-// cooperative (all work-groups resident), and a wait ends after GS_WAIT whatever
-// happens, with res[1 + g] = -1.
+// stores and loads, as the team spreads over XCDs with an L2 each.
+//   Work-groups take their place in a team by a ticket as they start, so at most one team of a
+// launch is incomplete at any time, all others run to their end, and the missing members
+// start when any work-group of the device ends.  (A cooperative launch would promise more, but
+// the queue it opens stays with the process, and the lanes of a ggb_group, which share four
+// hardware queues, then overlap less: 26.1 -> 37.3 ms for a scan of three.)  Should the teams of
+// several processes hold all CUs while each waits, a wait ends after GS_WAIT: that work-group
+// writes no more rows, its whole team ends the same way, and the group's sweeps are done
+// again from the same start by one work-group alone, with the same sums.
 // ---------------------------------------------------------------------------
 struct GsTeam {
     double *ex;  // [3][N]
@@ -5134,6 +5145,7 @@ template <bool TEAM, typename TE>
 static __device__ __forceinline__ void gs_matvec(const GsArgs &a, GsTeam &tm, const TE *M, const TE *MT, const double *x, double *out,
                                  double *scr) {
     if (!TEAM) return gs_colsum(MT, x, a.N, out, scr);
+    if (!tm.ok) return;  // gave up
     const int N = a.N, t = threadIdx.x;
     const int P = N < GS_WG ? GS_WG / N : 1;
     const int jl = (N + P - 1) / P;
@@ -5247,8 +5259,14 @@ __global__ __launch_bounds__(GS_WG) void k_gs_sweep(GsArgs a) {
     extern __shared__ double gsm[];
     __shared__ double red[GS_WG / 64];
     __shared__ double scr[GS_WG];
-    const int g = blockIdx.x % a.n_group, N = a.N, l = a.gl[g];
-    GsTeam tm{a.ex + (size_t)g * 3 * N, (int)blockIdx.x / a.n_group, 0, true};
+    __shared__ int ticket;
+    if (TEAM) {
+        if (threadIdx.x == 0) ticket = atomicAdd(a.ticket, 1);
+        __syncthreads();
+    }
+    const int g = TEAM ? ticket / a.team : blockIdx.x, N = a.N, l = a.gl[g];
+    if (!TEAM && a.redo && !(a.res[1 + g] < 0.0)) return;  // this group's team did not give up
+    GsTeam tm{a.ex + (size_t)g * 3 * N, TEAM ? ticket % a.team : 0, 0, true};
     const int32_t *sh = a.gsh + (size_t)g * GS_MAX_K;
     int k = 0;
     while (k < GS_MAX_K && sh[k] >= 0) ++k;
@@ -5313,7 +5331,7 @@ __global__ __launch_bounds__(GS_WG) void k_gs_sweep(GsArgs a) {
                 const double e = gs_dot(x, hx, N, red);
                 dmax = fmax(dmax, fabs(e - a.eps[sh[j]]));
                 __syncthreads();
-                if (tm.me == 0) {
+                if (tm.me == 0 && tm.ok) {
                     if (threadIdx.x == 0) a.eps[sh[j]] = e;
                     for (int i = threadIdx.x; i < N; i += blockDim.x) a.u[(size_t)sh[j] * N + i] = us[i];
                 }
@@ -5387,7 +5405,7 @@ extern "C" int ggb_ground_state(const ggb_gs_problem *p, const int32_t *shell_l,
            *deps = nullptr, *dv = nullptr, *drho = nullptr, *dres = nullptr;
     double *dex = nullptr, *dpriv = nullptr;
     float *dQ = nullptr, *dQT = nullptr;
-    int32_t *dgsh = nullptr, *dgl = nullptr;
+    int32_t *dgsh = nullptr, *dgl = nullptr, *dticket = nullptr;
     int rc = GGB_OK;
     // teams of the sweep kernel, and where each work-group keeps its shells
     int kmax = 0;
@@ -5422,7 +5440,7 @@ extern "C" int ggb_ground_state(const ggb_gs_problem *p, const int32_t *shell_l,
         hip(dalloc(&du, (size_t)ns * N), "alloc") && hip(dalloc(&deps, ns), "alloc") &&
         hip(dalloc(&dv, N), "alloc") && hip(dalloc(&drho, N), "alloc") && hip(dalloc(&dres, 1 + G), "alloc") &&
         hip(dalloc(&dgsh, (size_t)G * GS_MAX_K), "alloc") && hip(dalloc(&dgl, G), "alloc") &&
-        hip(dalloc(&dex, (size_t)G * 3 * N), "alloc") &&
+        hip(dalloc(&dex, (size_t)G * 3 * N), "alloc") && hip(dalloc(&dticket, 1), "alloc") &&
         (in_lds || hip(dalloc(&dpriv, (size_t)G * team * GS_MAX_K * N), "alloc")) &&
         up(dr, r, N * 8) && up(dwr, wr, N * 8) && up(dT, T, NN * 8) && up(dQ, q0f.data(), (size_t)G * NN * 4) &&
         up(dQT, q0t.data(), (size_t)G * NN * 4) && up(dlam, lam0, (size_t)G * N * 8) &&
@@ -5434,33 +5452,39 @@ extern "C" int ggb_ground_state(const ggb_gs_problem *p, const int32_t *shell_l,
         a.N = N, a.n_shell = ns, a.n_group = G, a.sweeps = p->sweeps, a.interacting = p->interacting ? 1 : 0;
         a.Z = p->Z, a.mix = p->mix, a.gamma = p->gamma;
         a.final_ = 0;
-        a.ex = dex, a.priv = dpriv, a.team = team, a.rows = rows;
+        a.ex = dex, a.priv = dpriv, a.ticket = dticket, a.team = team, a.rows = rows;
         std::vector<double> res(1 + G);
         for (it = 1; it <= p->max_iter; ++it) {
             a.first = it == 1;
             k_gs_potential<<<1, GS_WG, 0, st>>>(a);
-            void *args[] = {&a};
-            // one set of teams on the device at a time: two could each hold a part of it and wait
+            // one set of teams of this process on the device at a time
             static std::mutex teams;
             std::unique_lock<std::mutex> alone(teams, std::defer_lock);
             if (team > 1) alone.lock();
-            if (!hip(hipGetLastError(), "launch") ||
-                !hip(hipLaunchCooperativeKernel(reinterpret_cast<const void *>(team == 1 ? k_gs_sweep<false, true>
-                                                                               : in_lds  ? k_gs_sweep<true, true>
-                                                                                         : k_gs_sweep<true, false>),
-                                                dim3(G * team), dim3(GS_WG), args, (unsigned)(in_lds ? ldsu : lds5), st),
-                     "launch") ||
-                !hip(hipMemcpyAsync(res.data(), dres, (1 + G) * 8, hipMemcpyDeviceToHost, st), "download") ||
-                !hip(hipStreamSynchronize(st), "sync"))
-                break;
-            double de = 0.0;
-            bool waited = false;  // a work-group gave up waiting for its team
-            for (int g = 0; g < G; ++g) waited |= res[1 + g] < 0.0, de = std::max(de, res[1 + g]);
-            if (waited) {
-                g_create_err = "ggb_ground_state: the device did not run all work-groups of a sweep together";
-                rc = GGB_E_HIP;
-                break;
+            auto sweeps = [&](bool in_team) {
+                const size_t lds = in_lds ? ldsu : lds5;
+                if (in_team) {
+                    if (in_lds)
+                        k_gs_sweep<true, true><<<G * team, GS_WG, lds, st>>>(a);
+                    else
+                        k_gs_sweep<true, false><<<G * team, GS_WG, lds, st>>>(a);
+                } else if (in_lds) {
+                    k_gs_sweep<false, true><<<G, GS_WG, lds, st>>>(a);
+                } else {
+                    k_gs_sweep<false, false><<<G, GS_WG, lds, st>>>(a);
+                }
+                return hip(hipGetLastError(), "launch") &&
+                       hip(hipMemcpyAsync(res.data(), dres, (1 + G) * 8, hipMemcpyDeviceToHost, st), "download") &&
+                       hip(hipStreamSynchronize(st), "sync");
+            };
+            a.redo = 0;
+            if (!hip(hipGetLastError(), "launch") || !sweeps(team > 1)) break;
+            if (team > 1 && std::any_of(res.begin() + 1, res.end(), [](double d) { return d < 0.0; })) {
+                a.redo = 1;  // the groups whose team gave up waiting
+                if (!sweeps(false)) break;
             }
+            double de = 0.0;
+            for (int g = 0; g < G; ++g) de = std::max(de, res[1 + g]);
             if (de < p->tol && res[0] < 1e3 * p->tol) {
                 conv = true;
                 break;
@@ -5480,7 +5504,7 @@ extern "C" int ggb_ground_state(const ggb_gs_problem *p, const int32_t *shell_l,
     }
     for (void *d : {(void *)dr, (void *)dwr, (void *)dT, (void *)dQ, (void *)dQT, (void *)dlam, (void *)docc,
                     (void *)du, (void *)deps, (void *)dv, (void *)drho, (void *)dres, (void *)dgsh, (void *)dgl,
-                    (void *)dex, (void *)dpriv})
+                    (void *)dex, (void *)dpriv, (void *)dticket})
         if (d) (void)hipFree(d);
     if (st) (void)hipStreamDestroy(st);
     *iterations = it;
