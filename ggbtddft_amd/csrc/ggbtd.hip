@@ -2168,6 +2168,446 @@ __global__ __launch_bounds__(64 * ANG_MAXW) void k_angular(AngArgs g) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// FP64 angular kernel, one wave per tile (k_angular_wave): the steps of k_angular without LDS exchange
+// and barriers, for contexts with many tiles (one orbital column x RT radial nodes; ang_geometry has the rule).
+//
+// A wave keeps its tile X in registers: xs[s] holds row k = 4 s + kr of the l = m + 2 k (lane row
+// kr, real column lc = 2 i_local + re/im), xa[s] that of the l = m + 1 + 2 k.  That is the MFMA B operand
+// of K step s and also the FP64 accumulator layout: item r of output tile t is row 16 t + 4 r + kr, K
+// step 4 t + r.  So for each theta tile the forward products (E = Bs X_s, O = Ba X_a), the phase and
+// the folded sums leave S and D in the registers in which the back products X_s += Bs^T S,
+// X_a += Ba^T D read them.
+//  * The even laser pairs (l - m even) are xs[s], xa[s] of one lane; the odd ones need xs of the next k, one lane
+//    row up.  The two lanes of a column compute half of the sines each.
+//  * Sizes N_l = 32 n + 1 leave one row l = m + 32 n at m = 0, sizes h = 16 n + 1 one theta row (often the
+//    middle node).  Both are taken outside the products (RS: xr, and rem_h): dot products and
+//    rank-1 updates of a few FMAs, where a tile of 16 rows for one of them costs a quarter of the work.
+//  * The tables of one m (k_angular's) are in LDS, staged once for the waves of a work-group.
+// Measured, 32 instances of N_l = 65, N_r = 512, 7 orbitals (14336 tiles), modes 0 / 1: 149 / 203 us;
+// k_angular 255 / 352, whose waves wait at its barriers and which computes the padding rows.  Bound by
+// the issue of vector instructions and FP64 products, which share a SIMD: 8192 / 12288 cycles of products
+// a wave (55 / 73 us; 1024 SIMDs, 14 waves each, 2.1 GHz) next to about 2200 / 3000 vector instructions
+// (3 waves per SIMD by registers).
+// ---------------------------------------------------------------------------
+#define ANGW_WAVES 4
+#define ANGW_MIN_TILES 1600         // tiles of a context from which it is used (see ang_geometry)
+#define ANGW_LDS_MAX (50 * 1024)    // tables of one m: three work-groups (12 waves) per CU
+// the sum over the four lane rows, in every lane
+static __device__ __forceinline__ double rows_sum(double x) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+    const auto l0 = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
+    const auto h0 = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+    const double y = __longlong_as_double((long long)(((unsigned long long)h0[0] << 32) | l0[0])) +
+                     __longlong_as_double((long long)(((unsigned long long)h0[1] << 32) | l0[1]));
+    const unsigned long long c = (unsigned long long)__double_as_longlong(y);
+    const auto l1 = __builtin_amdgcn_permlane32_swap((unsigned)c, (unsigned)c, false, false);
+    const auto h1 = __builtin_amdgcn_permlane32_swap((unsigned)(c >> 32), (unsigned)(c >> 32), false, false);
+    return __longlong_as_double((long long)(((unsigned long long)h1[0] << 32) | l1[0])) +
+           __longlong_as_double((long long)(((unsigned long long)h1[1] << 32) | l1[1]));
+}
+// 4 x 4 transpose of lane rows (rows_transpose) of doubles, by halves
+static __device__ __forceinline__ void rows_transpose(double (&x)[4]) {
+    float lo[4], hi[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        const unsigned long long b = (unsigned long long)__double_as_longlong(x[s]);
+        lo[s] = __uint_as_float((unsigned)b);
+        hi[s] = __uint_as_float((unsigned)(b >> 32));
+    }
+    rows_transpose(lo);
+    rows_transpose(hi);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+        x[s] = __longlong_as_double((long long)(((unsigned long long)__float_as_uint(hi[s]) << 32) | __float_as_uint(lo[s])));
+}
+
+// sin and cos for |x| < 1e5 (larger ones: the library): argument reduction to r + t, |r| <= pi / 4, by three parts of pi / 2 (the
+// first two products are exact), and the Taylor series of r, whose first terms left out are below
+// 2e-17 there.  Largest error 0.74 units in the last place over 1e6 arguments up to 1e5, also next to
+// the multiples of pi / 2 (the library's: 0.78), in about 50 instructions instead of 130.
+static __device__ __forceinline__ void ang_sincos(double x, double *sn, double *cs) {
+    if (__any(!(fabs(x) < 1e5))) {
+        sincos(x, sn, cs);
+        return;
+    }
+    const double n = rint(x * 0.63661977236758134308);  // 2 / pi
+    // pi / 2 = 0x1.921fb544 (33 bits) + 0x1.0b4611a6 2^-34 (33 bits) + the rest
+    const double u = fma(-n, 0x1.921fb544p+0, x);
+    const double p2 = 0x1.0b4611a6p-34, p3 = 0x1.3198a2e037073p-69;
+    const double v = fma(-n, p2, u), vt = fma(-n, p2, u - v);
+    const double r = fma(-n, p3, v), t = fma(-n, p3, v - r) + vt;
+    const double z = r * r, zt = fma(r, r, -z);
+    double a = 1.0 / 355687428096000.0;  // 1 / 17!
+    a = fma(a, z, -1.0 / 1307674368000.0);
+    a = fma(a, z, 1.0 / 6227020800.0);
+    a = fma(a, z, -1.0 / 39916800.0);
+    a = fma(a, z, 1.0 / 362880.0);
+    a = fma(a, z, -1.0 / 5040.0);
+    a = fma(a, z, 1.0 / 120.0);
+    a = fma(a, z, -1.0 / 6.0);
+    double b = -1.0 / 6402373705728000.0;  // -1 / 18!
+    b = fma(b, z, 1.0 / 20922789888000.0);
+    b = fma(b, z, -1.0 / 87178291200.0);
+    b = fma(b, z, 1.0 / 479001600.0);
+    b = fma(b, z, -1.0 / 3628800.0);
+    b = fma(b, z, 1.0 / 40320.0);
+    b = fma(b, z, -1.0 / 720.0);
+    b = fma(b, z, 1.0 / 24.0);
+    const double h = 0.5 * z, w = 1.0 - h;
+    const double s0 = r + fma(r * z, a, t * w);
+    const double c0 = w + fma(z * z, b, ((1.0 - w) - h) - fma(r, t, 0.5 * zt));
+    const int q = (int)n;
+    const double s1 = q & 1 ? c0 : s0, c1 = q & 1 ? s0 : c0;
+    *sn = q & 2 ? -s1 : s1;
+    *cs = (q + 1) & 2 ? -c1 : c1;
+}
+
+// one tile: K tiles of 16 k for each parity, RS: one more s row (k = 16 K)
+template <int K, bool RS>
+struct AngTile {
+    typedef mfma_t<double> M;
+    typedef M::v4 v4;
+    const AngArgs &g;
+    const double *Bs, *Ba;
+    const ang_par &pr;
+    int m, kr, lc, p;
+    double xs[4 * K], xa[4 * K], xr;
+
+    // E and O of theta tile w (rows j >= hq read row hq - 1: their results are not used)
+    __device__ __forceinline__ void forward(int w, v4 &e, v4 &o) const {
+        const int j = min(16 * w + lc, g.hq - 1);
+        const double *As = Bs + (size_t)j * g.sS + kr, *Aa = Ba + (size_t)j * g.sA + kr;
+        e = (v4){0, 0, 0, 0};
+        o = (v4){0, 0, 0, 0};
+#pragma unroll
+        for (int t = 0; t < K; ++t) {
+            if (16 * t + 16 <= pr.ks) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) e = M::op(As[16 * t + 4 * r], xs[4 * t + r], e);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (16 * t + 4 * r < pr.ks) e = M::op(As[16 * t + 4 * r], xs[4 * t + r], e);
+            }
+            if (16 * t + 16 <= pr.ka) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o = M::op(Aa[16 * t + 4 * r], xa[4 * t + r], o);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (16 * t + 4 * r < pr.ka) o = M::op(Aa[16 * t + 4 * r], xa[4 * t + r], o);
+            }
+        }
+        if (RS && pr.ns > 16 * K) {
+            const double *Ar = Bs + 16 * K;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) e[r] += Ar[(size_t)min(16 * w + M::row(kr, r), g.hq - 1) * g.sS] * xr;
+        }
+    }
+    // the same for the single row j, in every lane row
+    __device__ __forceinline__ void forward_row(int j, double &e, double &o) const {
+        const double *As = Bs + (size_t)j * g.sS + kr, *Aa = Ba + (size_t)j * g.sA + kr;
+        e = o = 0.0;
+#pragma unroll
+        for (int s = 0; s < 4 * K; ++s) {
+            if (4 * s < pr.ks && (!RS || 4 * s < 16 * K)) e += As[4 * s] * xs[s];
+            if (4 * s < pr.ka) o += Aa[4 * s] * xa[s];
+        }
+        e = rows_sum(e);
+        o = rows_sum(o);
+        if (RS && pr.ns > 16 * K) e += Bs[(size_t)j * g.sS + 16 * K] * xr;
+    }
+
+    // laser pairs (l, l + 1), l = m + parity + 2 q, for dt/2: a = dt E r / 2 of this lane's node
+    __device__ __forceinline__ void laser(int parity, double a, const double *cl) {
+        const double sg = p ? -1.0 : 1.0;
+        double y[4 * K];  // the pair's other member: xs of the same k, or of the next one
+        if (parity == 0) {
+#pragma unroll
+            for (int s = 0; s < 4 * K; ++s) y[s] = xs[s];
+        } else {
+            double z[4 * K + 1];
+#pragma unroll
+            for (int s = 0; s < 4 * K; ++s) z[s] = __shfl(xs[s], (threadIdx.x + 16) & 63);
+            z[4 * K] = RS ? xr : 0.0;
+#pragma unroll
+            for (int s = 0; s < 4 * K; ++s) y[s] = kr < 3 ? z[s] : z[s + 1];
+        }
+#pragma unroll
+        for (int u = 0; u < 2 * K; ++u) {
+            // this lane's sine and cosine: of K step 2 u + p; the partner has the other's
+            const int l = m + parity + 2 * (4 * (2 * u + p) + kr);
+            double sn, cs;
+            ang_sincos(a * cl[min(l, ANG_MAX_NL - 1)], &sn, &cs);
+            const double sno = lane_xor1(sn), cso = lane_xor1(cs);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int s = 2 * u + h;
+                const double s_ = p == h ? sn : sno, c_ = p == h ? cs : cso;
+                // [x0', x1'] = [[cs, -i sn], [-i sn, cs]] [x0, x1]; lower member of an even pair: xs, of an odd one: xa
+                const double xo = xa[s], yo = y[s];
+                const double xp = lane_xor1(xo), yp = lane_xor1(yo);
+                const double xn = c_ * xo + sg * s_ * yp, yn = c_ * yo + sg * s_ * xp;
+                if (m + parity + 2 * (4 * s + 3) + 1 < g.Nl) {  // in every lane row
+                    xa[s] = xn;
+                    y[s] = yn;
+                } else {
+                    const bool ok = m + parity + 2 * (4 * s + kr) + 1 < g.Nl;
+                    xa[s] = ok ? xn : xo;
+                    y[s] = ok ? yn : yo;
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);  // one pair of steps at a time: registers
+        }
+        if (parity == 0) {
+#pragma unroll
+            for (int s = 0; s < 4 * K; ++s) xs[s] = y[s];
+        } else {
+            double z[4 * K];
+#pragma unroll
+            for (int s = 0; s < 4 * K; ++s) z[s] = __shfl(y[s], (threadIdx.x - 16) & 63);
+            if (RS) xr = __shfl(y[4 * K - 1], 48 + lc);
+#pragma unroll
+            for (int s = 4 * K - 1; s > 0; --s) xs[s] = kr > 0 ? z[s] : z[s - 1];
+            xs[0] = kr > 0 ? z[0] : xs[0];
+        }
+    }
+};
+
+template <int MODE, int K, bool RS>
+__global__ __launch_bounds__(64 * ANGW_WAVES, K == 1 ? 4 : 3) void k_angular_wave(AngArgs g, int ntiles) {
+    typedef mfma_t<double> M;
+    typedef M::v4 v4;
+    extern __shared__ __align__(16) double lds[];
+    __shared__ double cl[ANG_MAX_NL];
+    // logical order (orbital, radial group, instance), orbital fastest: the orbitals
+    // of one instance and radial group share the phase factors in L2
+    const int lg = xcd_linear();
+    const int korb = lg % g.n_orb, rest = lg / g.n_orb;
+    const int grp = rest % gridDim.x, inst = rest / gridDim.x;
+    if (g.active && !g.active[inst]) return;  // idle serving slot (block-uniform)
+    const int c = inst * g.n_orb + korb;
+    const int m = g.mcol[korb];
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    const int kr = lane >> 4, lc = lane & 15, p = lc & 1;
+    const ang_par pr(g.Nl, m);
+    double *Tl = reinterpret_cast<double *>(lds);
+    {
+        const double *Bsrc = reinterpret_cast<const double *>(g.Bh) + (size_t)m * g.nblk;
+        const int n16 = g.nblk * (int)sizeof(double) / 16;  // the block of one m is a multiple of 16 bytes
+        for (int b = 64 * wave; b < n16; b += 64 * ANGW_WAVES)
+            if (b + lane < n16)
+                __builtin_amdgcn_global_load_lds((const void *)(reinterpret_cast<const int4 *>(Bsrc) + b + lane),
+                                                 (lds_void_t *)(reinterpret_cast<int4 *>(Tl) + b), 16, 0, 0);
+        if (MODE != 2)
+            for (int l = t; l < ANG_MAX_NL; l += 64 * ANGW_WAVES) cl[l] = l < g.Nl ? c_lm(l, m) : 0.0;
+    }
+    const int tile_i = grp * ANGW_WAVES + wave;
+    const bool live = tile_i < ntiles;
+    const int i = min(tile_i * RT + (lc >> 1), g.N - 1);  // nodes past N: node N - 1, not stored
+    const bool iok = live && tile_i * RT + (lc >> 1) < g.N;
+    AngTile<K, RS> X{g, Tl, Tl + (size_t)g.hq * g.sS, pr, m, kr, lc, p};
+    const size_t plane = (size_t)g.C * g.N * 2;  // one l of the state, doubles
+    // row l = m + 2 (4 s + kr) of this lane's column: a lane base and a step of 8 planes per s
+    const size_t off0 = ((size_t)c * g.N + i) * 2 + p, offk = off0 + (size_t)(m + 2 * kr) * plane;
+    double *px = g.psi + offk;
+#pragma unroll
+    for (int s = 0; s < 4 * K; ++s) {
+        const size_t o = 8 * s * plane;
+        X.xs[s] = X.xa[s] = 0.0;
+        if (4 * s + 3 < pr.ns || 4 * s + kr < pr.ns) X.xs[s] = px[o];
+        if (4 * s + 3 < pr.na || 4 * s + kr < pr.na) X.xa[s] = px[o + plane];
+    }
+    X.xr = RS && pr.ns > 16 * K ? g.psi[off0 + (size_t)(m + 32 * K) * plane] : 0.0;
+    double a = 0.0;
+    if (MODE != 2) {
+        const int fs = g.cur ? (int)(((long)g.cur[0] + g.step) % g.n_field) : g.step;
+        a = 0.5 * g.dt * g.E[(size_t)inst * g.n_field + fs] * g.r[i];
+    }
+    __syncthreads();
+    if (!live) return;
+
+    if (MODE == 1) {
+        X.laser(1, a, cl);
+        X.laser(0, a, cl);
+    }
+    const bool rem_h = g.h % 16 == 1 && g.h > 1;  // the last theta row by itself
+    const int mt = rem_h ? g.h / 16 : (g.h + 15) / 16;
+    if (MODE != 2) {
+        const double *Bs = X.Bs, *Ba = X.Ba;
+        const double2 *pf = reinterpret_cast<const double2 *>(g.phase) + ((size_t)inst * g.N + i) * g.Nth;
+        v4 vs[K], va[K];
+        double vr = 0.0;
+#pragma unroll
+        for (int q = 0; q < K; ++q) vs[q] = va[q] = (v4){0, 0, 0, 0};
+        for (int w = 0; w < mt; ++w) {
+            // phase factors of rows j and j' = Nth - 1 - j (FP64: f; mixed form: f - 1); a whole tile
+            // holds neither the middle node nor rows past h
+            const bool whole = 16 * w + 15 + (g.Nth & 1) < g.h;
+            double2 fa[4], fb[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int j = 16 * w + M::row(kr, r);
+                const int jq = whole || j < g.h ? j : 0;
+                fa[r] = pf[jq];
+                fb[r] = pf[g.Nth - 1 - jq];
+            }
+            v4 e, o;
+            X.forward(w, e, o);
+            double sv[4], dv[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const double pa = e[r] + o[r], pb = e[r] - o[r];
+                const double pao = lane_xor1(pa), pbo = lane_xor1(pb);
+                // component p of f (x + i y): x fx - y fy (p = 0), y fx + x fy (p = 1);
+                // this lane holds component p, its partner the other
+                const double sg = p ? 1 : -1;
+                const double qa = pa * fa[r].x + sg * pao * fa[r].y;
+                const double qb = pb * fb[r].x + sg * pbo * fb[r].y;
+                sv[r] = qa + qb;
+                dv[r] = qa - qb;
+                if (!whole) {
+                    const int j = 16 * w + M::row(kr, r);
+                    if (g.Nth - 1 - j == j) sv[r] = dv[r] = qa;
+                    if (j >= g.h) sv[r] = dv[r] = 0;
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (16 * w + 4 * r >= g.hq) continue;
+                const double *Rs = Bs + (size_t)(16 * w + 4 * r + kr) * g.sS, *Ra = Ba + (size_t)(16 * w + 4 * r + kr) * g.sA;
+                // output rows past the parity's last k read what follows in LDS and are cleared below
+#pragma unroll
+                for (int q = 0; q < K; ++q) {
+                    if (16 * q < pr.ks) vs[q] = M::op(Rs[16 * q + lc], sv[r], vs[q]);
+                    if (16 * q < pr.ka) va[q] = M::op(Ra[16 * q + lc], dv[r], va[q]);
+                }
+                if (RS && pr.ns > 16 * K) vr += Rs[16 * K] * sv[r];
+            }
+        }
+        if (RS && pr.ns > 16 * K) vr = rows_sum(vr);
+        // the remaining theta row, and the new X
+        double sR = 0.0, dR = 0.0;
+        const int jR = g.h - 1;
+        if (rem_h) {
+            const int jm = g.Nth - 1 - jR;
+            const double2 fa = pf[jR], fb = pf[jm];
+            double e, o;
+            X.forward_row(jR, e, o);
+            const double pa = e + o, pb = e - o, pao = lane_xor1(pa), pbo = lane_xor1(pb);
+            const double sg = p ? 1.0 : -1.0;
+            const double qa = pa * fa.x + sg * pao * fa.y, qb = pb * fb.x + sg * pbo * fb.y;
+            sR = jm == jR ? qa : qa + qb;
+            dR = jm == jR ? qa : qa - qb;
+        }
+#pragma unroll
+        for (int q = 0; q < K; ++q) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int s = 4 * q + r, k = 4 * s + kr;
+                double bs = vs[q][r], ba = va[q][r];
+                if (rem_h) {
+                    bs += Bs[(size_t)jR * g.sS + min(k, pr.ks - 1)] * sR;
+                    ba += Ba[(size_t)jR * g.sA + min(k, pr.ka - 1)] * dR;
+                }
+                X.xs[s] = k < pr.ns ? bs : 0.0;
+                X.xa[s] = k < pr.na ? ba : 0.0;
+            }
+        }
+        if (RS && pr.ns > 16 * K) X.xr = rem_h ? vr + Bs[(size_t)jR * g.sS + 16 * K] * sR : vr;
+    }
+    if (MODE == 0) {
+        X.laser(0, a, cl);
+        X.laser(1, a, cl);
+    }
+    // r_i ahead of the state stores (one vector-memory counter covers loads and stores)
+    double ri = 1.0;
+    if (MODE != 0) ri = g.r[i];
+    if (MODE != 2) {
+        if (iok) {
+#pragma unroll
+            for (int s = 0; s < 4 * K; ++s) {
+                const size_t o = 8 * s * plane;
+                const int k = 4 * s + kr;
+                if (4 * s + 3 < pr.ns || k < pr.ns) px[o] = X.xs[s];
+                if (4 * s + 3 < pr.na || k < pr.na) px[o + plane] = X.xa[s];
+            }
+            if (RS && pr.ns > 16 * K && kr == 0) g.psi[off0 + (size_t)(m + 32 * K) * plane] = X.xr;
+        }
+    }
+    if (MODE == 0) return;
+
+    // |B psi|^2 and observable partials (accumulated in FP64)
+    double sx = 0.0, sn = 0.0;
+    // folded |Psi|^2 rows: lanes p = 0 store the nodes j, lanes p = 1 their mirrors
+    double *dens = reinterpret_cast<double *>(g.dens) + (((size_t)c * g.N + i) * 2 + p) * g.hq;
+    // value stored by this lane; sums: sx = sum_j chi_j (|Psi_j|^2 - |Psi_j'|^2), sn the norm, in the lanes p = 0
+    auto point = [&](int j, double ed, double od, double ca, bool whole) -> double {
+        const double v0 = ed + od, v1 = ed - od;
+        // no contraction: both lanes of a column form the same sums
+        const double qa = __dmul_rn(v0, v0), qb = __dmul_rn(v1, v1), qe = __dmul_rn(ed, od);
+        const double s2a = qa + lane_xor1(qa), s2b = qb + lane_xor1(qb);
+        const double eo = 4.0 * (qe + lane_xor1(qe));  // |Psi_j|^2 - |Psi_j'|^2
+        if (whole || (j < g.h && g.Nth - 1 - j != j)) {
+            sx += ca * eo;
+            sn += s2a + s2b;
+        } else if (j < g.h) {
+            sn += s2a;  // middle node, chi = 0
+        }
+        return p ? s2b : s2a;
+    };
+    for (int w = 0; w < mt; ++w) {
+        const bool whole = 16 * w + 15 + (g.Nth & 1) < g.h;
+        double cd[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int j = 16 * w + M::row(kr, r);
+            cd[r] = g.chi[whole || j < g.h ? j : 0];
+        }
+        v4 e, o;
+        X.forward(w, e, o);
+        double dq[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            dq[r] = point(16 * w + M::row(kr, r), e[r], o[r], cd[r], whole);
+        rows_transpose(dq);  // now rows 4 kr + r
+        // rows h .. hq - 1 hold values that k_rho never reads, and so does the mirror half at the middle
+        // node of an odd N_theta
+        const int j0 = 16 * w + 4 * kr;
+        if (iok && j0 < g.hq) {
+            *reinterpret_cast<double2 *>(dens + j0) = make_double2(dq[0], dq[1]);
+            *reinterpret_cast<double2 *>(dens + j0 + 2) = make_double2(dq[2], dq[3]);
+        }
+    }
+    if (rem_h) {
+        double e, o;
+        X.forward_row(g.h - 1, e, o);
+        // every lane row holds it: the sums take it from row 0
+        const double k0 = sx, k1 = sn;
+        const double d = point(g.h - 1, e, o, g.chi[g.h - 1], false);
+        if (kr != 0) sx = k0, sn = k1;
+        if (iok && kr == 0) dens[g.h - 1] = d;
+    }
+    // the sums of the lanes p = 0 of this tile's nodes; dipole-type ones with r and 1 / r^2
+    if (p || !iok) sx = sn = 0.0;
+    double sd = ri * sx, sa = sx / (ri * ri);
+    sd = rows_sum(sd);
+    sa = rows_sum(sa);
+    sn = rows_sum(sn);
+    for (int off = 8; off > 1; off >>= 1) {
+        sd += __shfl_down(sd, off);
+        sa += __shfl_down(sa, off);
+        sn += __shfl_down(sn, off);
+    }
+    if (lane == 0) {
+        double *ob = g.obs_part + ((size_t)c * ntiles + tile_i) * 3;
+        ob[0] = sd;
+        ob[1] = sa;
+        ob[2] = sn;
+    }
+}
+
 // per-column sums of the observable partials -> obs[step_rel][c][3]
 struct ObsArgs {
     const double *part;  // [C][ntiles][3]
@@ -2983,7 +3423,8 @@ struct ang_geom {
     bool glb;    // tables read from global memory
     bool alias;  // mixed form: S/D share the l-space tile's LDS
     int nt;      // column tiles (of RT radial nodes) per work-group
-    int ntiles;  // work-groups along r
+    int ntiles;  // tiles along r (observable partials per column)
+    bool wave;   // k_angular_wave
 };
 static ang_geom ang_geometry(const ggb_problem *p) {
     ang_geom a;
@@ -3017,6 +3458,17 @@ static ang_geom ang_geometry(const ggb_problem *p) {
 #endif
     a.glb = ANG_FORCE_GLB || tiles + (size_t)a.nblk * es + stat > ANG_LDS_MAX;
     a.lds = a.glb ? tiles : tiles + (size_t)a.nblk * es;
+    // FP64: k_angular_wave where every SIMD gets more than one and a half tiles (below, a tile's
+    // four or five waves in k_angular finish sooner) and at least three quarters of its 16 K
+    // rows of each parity are l values.  Phases of a step, k_angular / k_angular_wave, us: N_l = 65,
+    // N_r = 512, 7 orbitals: 448 tiles 34 / 55, 896 59 / 58, 1792 97 / 74, 14336 606 / 354;
+    // N_l = 49: 1536 tiles 55 / 56, 1920 70 / 59, 3840 115 / 97; N_l = 33: 1280 tiles 35 / 37,
+    // 1920 48 / 39, 5120 93 / 68.  Emptier rows: N_l = 41: 3192 tiles 83 / 86; N_l = 13: 2400 tiles 29 / 30.
+    const int ak = na0 > 16 ? 2 : 1;  // K; RS: one s row more
+    const long wtiles = (long)((p->n_r + RT - 1) / RT) * p->n_orb * p->n_inst;
+    a.wave = !p->precision && na0 <= 32 && ns0 <= 16 * ak + 1 && 4 * ns0 >= 3 * 16 * ak && wtiles > ANGW_MIN_TILES &&
+             (size_t)(a.nblk + 64) * 8 <= ANGW_LDS_MAX;
+    if (a.wave) a.ntiles = (p->n_r + RT - 1) / RT;
     return a;
 }
 
@@ -3504,6 +3956,24 @@ static void launch_angular_t(ggb_ctx *ctx, const AngArgs &g) {
     }
 }
 
+template <int MODE, int K, bool RS>
+static void launch_angular_wave_t(ggb_ctx *ctx, const AngArgs &g) {
+    const size_t lds = ((size_t)ctx->ang.nblk + 64) * sizeof(double);  // partial tiles read a little past the tables
+    const int nt = ctx->ang.ntiles;
+    const dim3 ga((nt + ANGW_WAVES - 1) / ANGW_WAVES, ctx->C);
+    k_angular_wave<MODE, K, RS><<<ga, 64 * ANGW_WAVES, lds, ctx->stream>>>(g, nt);
+}
+template <int MODE>
+static void launch_angular_wave(ggb_ctx *ctx, const AngArgs &g) {
+    const int ns = (ctx->p.n_l + 1) / 2, na = ctx->p.n_l / 2;  // rows of each parity at m = 0
+    if (na > 16) {
+        if (ns > 32) return launch_angular_wave_t<MODE, 2, true>(ctx, g);
+        return launch_angular_wave_t<MODE, 2, false>(ctx, g);
+    }
+    if (ns > 16) return launch_angular_wave_t<MODE, 1, true>(ctx, g);
+    launch_angular_wave_t<MODE, 1, false>(ctx, g);
+}
+
 static int kin_variant(const ggb_ctx *ctx);
 
 template <int MODE>
@@ -3515,7 +3985,9 @@ static void launch_angular(ggb_ctx *ctx, int step, const int *cur = nullptr) {
         g.psi32 = ctx->psi32;  // the kinetic pass 1 that follows reads it
         g.l0 = ctx->have_ref ? ctx->l0 : nullptr;
     }
-    if (ctx->p.precision)
+    if (ctx->ang.wave)
+        launch_angular_wave<MODE>(ctx, g);
+    else if (ctx->p.precision)
         launch_angular_t<MODE, float>(ctx, g);
     else
         launch_angular_t<MODE, double>(ctx, g);
