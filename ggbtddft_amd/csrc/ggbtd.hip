@@ -19,7 +19,7 @@
 //   (mixed form: k_kin_fwd / k_kin_bwd, 16-wide tiles, or k_kin_*_dma / _tiled, 64 x 128 tiles)
 //   k_angular<mode 1>   Lo, Le, Vh, |B psi|^2, observable partials
 //   k_rho               rho_u = sum occ |Psi|^2, v_xc; observable sums
-//   k_tile_gemm<Qmom>   multipole moments q_L = P_L^T rho_u
+//   k_tile_gemm<Qmom>   multipole moments q_L = P_L^T rho_u (small contexts: both in k_rho_mom)
 //   k_hartree           V_L by prefix/suffix affine scans  grid (n_har, n_inst)
 //   k_tile_gemm<Dv>     dV = sum_L V_L P_L, v_xc - v_gs, phase factors of the next step
 //
@@ -2710,52 +2710,161 @@ static __device__ T lda_vxc(T rho) {
 }
 
 // Density and LDA v_xc (in T) pointwise on the (r_i, theta_j) grid:
-// rho_u(i, j) = sum_k occ_k |Psi_k(i, j)|^2 (+ the frozen core), kept for the
-// multipole moments, and v_xc of the density rho = rho_u / (2 pi omega_j wr_i r_i^2).
+// rho_u(i, j) = sum_k occ_k |Psi_k(i, j)|^2 (+ the frozen core), for the multipole moments,
+// and v_xc of the density rho = rho_u / (2 pi omega_j wr_i r_i^2).
+struct RhoArgs {
+    const void *dens;        // [C][N][2][hq], compute type
+    const double *occ, *rho_frozen, *r, *wr, *omega;
+    double *rho_u, *vxc;
+    int N, Nth, h, hq, n_orb;
+    const int32_t *active;
+};
+// grid blocks `block` of nrho, then the observable sums of the step, one (column, observable)
+// pair per wave (instance 0's blocks); rho_u is stored where it is not null
 template <typename T>
-__global__ __launch_bounds__(WG) void k_rho(const T *__restrict__ dens,
-                                            const double *__restrict__ occ,
-                                            const double *__restrict__ rho_frozen,
-                                            const double *__restrict__ r,
-                                            const double *__restrict__ wr,
-                                            const double *__restrict__ omega,
-                                            double *__restrict__ rho_u, double *__restrict__ vxc,
-                                            int N, int Nth, int h, int hq, int n_orb, ObsArgs ob,
-                                            const int32_t *__restrict__ active) {
-    // the blocks past the (r, theta) grid (instance row 0) reduce the observable
-    // partials of the step, one (column, observable) pair per wave
-    const int nrho = (int)(((size_t)N * Nth + WG - 1) / WG);
-    if ((int)blockIdx.x >= nrho) {
-        const int pair = ((int)blockIdx.x - nrho) * (WG / 64) + (threadIdx.x >> 6);
-        if (blockIdx.y == 0 && ob.obs && pair < ob.C * 3) obs_reduce_pair(ob, pair);
+static __device__ __forceinline__ void rho_block(const RhoArgs &a, const ObsArgs &ob, int block, int inst) {
+    const int nrho = (int)(((size_t)a.N * a.Nth + WG - 1) / WG);
+    if (block >= nrho) {
+        const int pair = (block - nrho) * (WG / 64) + (threadIdx.x >> 6);
+        if (inst == 0 && ob.obs && pair < ob.C * 3) obs_reduce_pair(ob, pair);
         return;
     }
-    const int inst = blockIdx.y;
-    if (active && !active[inst]) return;  // idle serving slot (block-uniform)
+    if (a.active && !a.active[inst]) return;  // idle serving slot (block-uniform)
+    const int N = a.N, Nth = a.Nth, h = a.h, n_orb = a.n_orb;
     const int npt = N * Nth;  // < 2^31 (ggb_create bounds N and N_theta)
-    const int idx = (int)blockIdx.x * WG + (int)threadIdx.x;
+    const int idx = block * WG + (int)threadIdx.x;
     if (idx >= npt) return;
     const int i = idx / Nth, j = idx - i * Nth;
     // the folded |Psi|^2 rows: node j < h in the first half, its mirror in the second
-    const size_t nd = (size_t)N * 2 * hq;  // one orbital column
-    const T *dk = dens + (size_t)inst * n_orb * nd + ((size_t)i * 2 + (j < h ? 0 : 1)) * hq + (j < h ? j : Nth - 1 - j);
+    const size_t nd = (size_t)N * 2 * a.hq;  // one orbital column
+    const T *dk = reinterpret_cast<const T *>(a.dens) + (size_t)inst * n_orb * nd + ((size_t)i * 2 + (j < h ? 0 : 1)) * a.hq +
+                  (j < h ? j : Nth - 1 - j);
     // four orbitals' loads in flight at a time, summed in orbital order
     double ru = 0.0;
     int k = 0;
     for (; k + 4 <= n_orb; k += 4) {
         const T d0 = dk[k * nd], d1 = dk[(k + 1) * nd];
         const T d2 = dk[(k + 2) * nd], d3 = dk[(k + 3) * nd];
-        ru += occ[k] * d0;
-        ru += occ[k + 1] * d1;
-        ru += occ[k + 2] * d2;
-        ru += occ[k + 3] * d3;
+        ru += a.occ[k] * d0;
+        ru += a.occ[k + 1] * d1;
+        ru += a.occ[k + 2] * d2;
+        ru += a.occ[k + 3] * d3;
     }
-    for (; k < n_orb; ++k) ru += occ[k] * dk[k * nd];
-    if (rho_frozen) ru += 0.5 * rho_frozen[i] * omega[j];
-    const double rho = ru / (2.0 * M_PI * omega[j] * wr[i] * r[i] * r[i]);
+    for (; k < n_orb; ++k) ru += a.occ[k] * dk[k * nd];
+    if (a.rho_frozen) ru += 0.5 * a.rho_frozen[i] * a.omega[j];
+    const double rho = ru / (2.0 * M_PI * a.omega[j] * a.wr[i] * a.r[i] * a.r[i]);
     const size_t o = (size_t)inst * N * Nth + idx;
-    rho_u[o] = ru;
-    vxc[o] = (double)lda_vxc<T>((T)rho);
+    if (a.rho_u) a.rho_u[o] = ru;
+    a.vxc[o] = (double)lda_vxc<T>((T)rho);
+}
+template <typename T>
+__global__ __launch_bounds__(WG) void k_rho(RhoArgs a, ObsArgs ob) {
+    rho_block<T>(a, ob, blockIdx.x, blockIdx.y);
+}
+
+// k_rho and the multipole moments q_L(i) = sum_j P_L(chi_j) rho_u(i, j) in one launch, for small
+// contexts, whose steps are bound by the latency of their launches: the first nmom blocks
+// form the moments, one tile of 16 radial nodes and 16 multipoles each, from their own sums over
+// the orbitals (rho_u of the 16 nodes, in LDS).  A wave takes a quarter of the theta range as in
+// k_tile_gemm; the terms and the order of every sum are those of k_rho and k_tile_gemm.
+// Each |Psi|^2 value is read once for every 16 multipoles, so the launch that is saved pays for
+// it up to MOM_MAX_READS values in MOM_MAX_BLOCKS tiles; the two phases together, two launches / one, us (FP64):
+// 4e3 values (N_r = 96, N_theta = 25, 2 tiles) 10.0 / 6.7; 5e5 (six instances of 256 x 65) 11.6 / 10.3;
+// 1.0e6 (384 x 97, 4 orbitals) 10.3 / 9.1; 4.2e6 (512 x 129, 7 orbitals) 12.7 / 12.8; the same
+// three times 17.2 / 22.8; 4.8e5 values in 1200 tiles (100 instances of 96 x 25) 17.1 / 18.9.  Sharing the sums between two or three multipole tiles is slower at the small
+// sizes (7.3, 7.6) and no better than two launches at the large ones.
+#define MOM_MAX_READS 2000000
+#define MOM_MAX_BLOCKS 512
+#define MOM_K 4  // orbitals' loads in flight
+#define MOM_P 4  // grid points of a thread at a time
+#define MOM_U 9  // theta values of a lane per round: a quarter of N_theta = 129
+static size_t mom_lds(int Nth) { return std::max<size_t>((size_t)16 * (Nth | 1), 4 * 64 * 4) * sizeof(double); }
+template <typename T>
+__global__ __launch_bounds__(WG) void k_rho_mom(RhoArgs a, ObsArgs ob, const double *__restrict__ PL, double *__restrict__ q,
+                                                int n_har, int nmom) {
+    extern __shared__ __align__(16) double lds[];  // rho_u [16][Nth | 1], then the partial tiles
+    const int inst = blockIdx.y;
+    if ((int)blockIdx.x >= nmom) return rho_block<T>(a, ob, (int)blockIdx.x - nmom, inst);
+    if (a.active && !a.active[inst]) return;  // idle serving slot (block-uniform)
+    const int ni = (a.N + 15) / 16;
+    const int i0 = (int)blockIdx.x % ni * 16, L0 = (int)blockIdx.x / ni * 16;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int kr = lane >> 4, lc = lane & 15;
+    const int kq = (((a.Nth + 3) / 4 + 3) / 4) * 4;  // quarter of N_theta, multiple of 4
+    const int kb = wave * kq, ke = min(a.Nth, kb + kq);
+    double av[MOM_U];  // loaded ahead of the sums
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int u = 0; u < MOM_U; ++u)
+            av[u] = PL[(size_t)min(k0 + 4 * u + kr, a.Nth - 1) * n_har + min(L0 + lc, n_har - 1)];
+    };
+    load(kb);
+    const int st = a.Nth | 1;
+    {
+        const int nn = min(16, a.N - i0), np = nn * a.Nth;
+        const size_t nd = (size_t)a.N * 2 * a.hq;
+        const T *db = reinterpret_cast<const T *>(a.dens) + (size_t)inst * a.n_orb * nd + (size_t)i0 * 2 * a.hq;
+        for (int p0 = threadIdx.x; p0 < np; p0 += WG * MOM_P) {
+            double ru[MOM_P];
+            int off[MOM_P], pi[MOM_P], pj[MOM_P];
+#pragma unroll
+            for (int e = 0; e < MOM_P; ++e) {
+                const int idx = min(p0 + e * WG, np - 1);
+                pi[e] = idx / a.Nth;
+                pj[e] = idx - pi[e] * a.Nth;
+                off[e] = pi[e] * 2 * a.hq + (pj[e] < a.h ? pj[e] : a.hq + a.Nth - 1 - pj[e]);
+                ru[e] = 0.0;
+            }
+            const T *dk = db;
+            int k = 0;
+            for (; k + MOM_K <= a.n_orb; k += MOM_K, dk += MOM_K * nd) {
+                T d[MOM_K][MOM_P];
+#pragma unroll
+                for (int b = 0; b < MOM_K; ++b)
+#pragma unroll
+                    for (int e = 0; e < MOM_P; ++e) d[b][e] = dk[b * nd + off[e]];
+#pragma unroll
+                for (int b = 0; b < MOM_K; ++b)
+#pragma unroll
+                    for (int e = 0; e < MOM_P; ++e) ru[e] += a.occ[k + b] * d[b][e];
+            }
+            for (; k < a.n_orb; ++k, dk += nd) {
+                T d[MOM_P];
+#pragma unroll
+                for (int e = 0; e < MOM_P; ++e) d[e] = dk[off[e]];
+#pragma unroll
+                for (int e = 0; e < MOM_P; ++e) ru[e] += a.occ[k] * d[e];
+            }
+#pragma unroll
+            for (int e = 0; e < MOM_P; ++e) {
+                if (a.rho_frozen) ru[e] += 0.5 * a.rho_frozen[i0 + pi[e]] * a.omega[pj[e]];
+                if (p0 + e * WG < np) lds[pi[e] * st + pj[e]] = ru[e];
+            }
+        }
+    }
+    __syncthreads();
+    d4_t acc = {0.0, 0.0, 0.0, 0.0};
+    const double *rl = lds + min(lc, a.N - 1 - i0) * st;  // nodes past N: results not stored
+    for (int k0 = kb; k0 < ke; k0 += 4 * MOM_U) {
+        if (k0 > kb) load(k0);
+#pragma unroll
+        for (int u = 0; u < MOM_U; ++u) {
+            const int j = k0 + 4 * u + kr;
+            const bool ok = j < ke;
+            const double b = ok ? rl[j] : 0.0;
+            if (k0 + 4 * u < ke) acc = mfma64(ok ? av[u] : 0.0, b, acc);
+        }
+    }
+    __syncthreads();
+    // partial tiles through LDS (wave 0's in the last slot); wave w finishes accumulator row r = w
+    typedef double part_t[64][4];
+    part_t *red = reinterpret_cast<part_t *>(lds);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wave > 0 ? wave - 1 : 3][lane][r] = acc[r];
+    __syncthreads();
+    const int r = wave, L = L0 + mfma_t<double>::row(kr, r);
+    const double v = ((red[3][lane][r] + red[0][lane][r]) + red[1][lane][r]) + red[2][lane][r];
+    if (L < n_har && i0 + lc < a.N) q[((size_t)inst * n_har + L) * a.N + i0 + lc] = v;
 }
 
 // One 16 x 16 tile of D = A B in FP64 on the matrix cores per work-group
@@ -4012,36 +4121,45 @@ static int launch_potential(ggb_ctx *ctx, const ObsArgs *ob = nullptr, MarkK mk 
         const unsigned nrho = (unsigned)(((size_t)N * Nth + WG - 1) / WG);
         const unsigned nobs = oa.obs ? (unsigned)((oa.C * 3 + WG / 64 - 1) / (WG / 64)) : 0u;
         const dim3 gr(nrho + nobs, p.n_inst);
-        if (p.precision)
-            k_rho<float><<<gr, WG, 0, st>>>(reinterpret_cast<const float *>(ctx->dens), ctx->occ, ctx->rho_frozen, ctx->r, ctx->wr,
-                                            ctx->omega, ctx->rho_u, ctx->vxc, N, Nth, ctx->ang.h, ctx->ang.hq, p.n_orb, oa,
-                                            ctx->active);
-        else
-            k_rho<double><<<gr, WG, 0, st>>>(ctx->dens, ctx->occ, ctx->rho_frozen, ctx->r, ctx->wr,
-                                             ctx->omega, ctx->rho_u, ctx->vxc, N, Nth, ctx->ang.h, ctx->ang.hq, p.n_orb, oa,
-                                             ctx->active);
-        GemmOperands gq;  // q[L][i] = sum_j PLT[L][j] rho_u[i][j]
-        gq.A = ctx->PLT;
-        gq.sam = Nth;
-        gq.sak = 1;
-        gq.saz = 0;
-        gq.B = ctx->rho_u;
-        gq.sbk = 1;
-        gq.sbn = Nth;
-        gq.sbz = (long)N * Nth;
-        gq.M = nh;
-        gq.active = ctx->active;
-        gq.N = N;
-        gq.K = Nth;
-        QmomEpi eq{ctx->q, N, nh};
-        if (p.n_inst >= TGW_MIN_INST) {
-            gq.A = ctx->PL;  // the same table as [j][L]: the 16 lanes of a K row read 16 consecutive L
-            gq.sam = 1;
-            gq.sak = nh;
-            const int ntl = (nh + 15) / 16;
-            k_tile_gemm_wide<QmomEpi, true><<<dim3((N + 15) / 16, (ntl + TGW_T - 1) / TGW_T, p.n_inst), WG, 0, st>>>(gq, eq);
+        const int ntl = (nh + 15) / 16;
+        const unsigned nmom = (unsigned)((N + 15) / 16 * ntl);
+        // moments in the same launch
+        const bool one = (double)N * Nth * p.n_orb * p.n_inst * ntl <= MOM_MAX_READS && (double)nmom * p.n_inst <= MOM_MAX_BLOCKS;
+        const RhoArgs ra{ctx->dens, ctx->occ, ctx->rho_frozen, ctx->r, ctx->wr, ctx->omega, one ? nullptr : ctx->rho_u, ctx->vxc,
+                         N, Nth, ctx->ang.h, ctx->ang.hq, p.n_orb, ctx->active};
+        if (one) {
+            const dim3 gm(nmom + gr.x, p.n_inst);
+            if (p.precision)
+                k_rho_mom<float><<<gm, WG, mom_lds(Nth), st>>>(ra, oa, ctx->PL, ctx->q, nh, (int)nmom);
+            else
+                k_rho_mom<double><<<gm, WG, mom_lds(Nth), st>>>(ra, oa, ctx->PL, ctx->q, nh, (int)nmom);
         } else {
-            k_tile_gemm<<<dim3((N + 15) / 16, (nh + 15) / 16, p.n_inst), WG, 0, st>>>(gq, eq);
+            if (p.precision)
+                k_rho<float><<<gr, WG, 0, st>>>(ra, oa);
+            else
+                k_rho<double><<<gr, WG, 0, st>>>(ra, oa);
+            GemmOperands gq;  // q[L][i] = sum_j PLT[L][j] rho_u[i][j]
+            gq.A = ctx->PLT;
+            gq.sam = Nth;
+            gq.sak = 1;
+            gq.saz = 0;
+            gq.B = ctx->rho_u;
+            gq.sbk = 1;
+            gq.sbn = Nth;
+            gq.sbz = (long)N * Nth;
+            gq.M = nh;
+            gq.active = ctx->active;
+            gq.N = N;
+            gq.K = Nth;
+            QmomEpi eq{ctx->q, N, nh};
+            if (p.n_inst >= TGW_MIN_INST) {
+                gq.A = ctx->PL;  // the same table as [j][L]: the 16 lanes of a K row read 16 consecutive L
+                gq.sam = 1;
+                gq.sak = nh;
+                k_tile_gemm_wide<QmomEpi, true><<<dim3((N + 15) / 16, (ntl + TGW_T - 1) / TGW_T, p.n_inst), WG, 0, st>>>(gq, eq);
+            } else {
+                k_tile_gemm<<<dim3((N + 15) / 16, ntl, p.n_inst), WG, 0, st>>>(gq, eq);
+            }
         }
         HIPCHK(ctx, mk(0));
         const int cs = (N + WG - 1) / WG;  // N <= 4096 (ggb_create): cs <= 16
