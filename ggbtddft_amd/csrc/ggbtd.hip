@@ -142,9 +142,17 @@ static __device__ __forceinline__ T kin_factor(double v, double vo, int p, doubl
 struct KinRef {
     const double *phi;   // [n_orb][N]
     const int32_t *l0;   // [n_orb]
-    const double4 *ab;   // [C]
+    const double *eps;   // [n_orb]
+    double4 *ab;         // [C]
     const int32_t *active;  // [n_inst] instances in use, or null (all)
+    double dt;
 };
+// (alpha, beta) of orbital k
+static __device__ __forceinline__ double4 kin_ref_ab(const KinRef &ref, int k, double ar, double ai) {
+    double sn, cs;
+    sincos(ref.eps[k] * ref.dt, &sn, &cs);
+    return make_double4(ar, ai, cs * ar + sn * ai, cs * ai - sn * ar);
+}
 
 // whether any instance with a column among real columns [n0, n0 + nreal) is
 // in use (work-group-uniform; idle serving slots skip their kinetic tiles)
@@ -156,16 +164,18 @@ static __device__ __forceinline__ bool kin_cols_active(const int32_t *active, in
         if (active[q]) return true;
     return false;
 }
-__global__ __launch_bounds__(WG) void k_kin_ref(const double *__restrict__ psi,
-                                                const double *__restrict__ phi,
-                                                const int32_t *__restrict__ l0,
-                                                const double *__restrict__ eps, double4 *ab,
-                                                int N, int C, int n_orb, double dt) {
+// PREP: and the FP32 copy of the column's ground-state block with alpha phi taken out, as
+// k_kin_prep writes it (one launch less where the angular kernel has written the others).
+// The narrow pass 1 forms alpha itself, with these sums.
+template <bool PREP>
+__global__ __launch_bounds__(WG) void k_kin_ref(const double2 *__restrict__ psi, KinRef ref, float2 *__restrict__ psi32, int N,
+                                                int C, int n_orb) {
     __shared__ double red[2][WG / 64];
     const int c = blockIdx.x, k = c % n_orb;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const double *ph = phi + (size_t)k * N;
-    const double2 *x = (const double2 *)psi + ((size_t)l0[k] * C + c) * N;
+    const double *ph = ref.phi + (size_t)k * N;
+    const size_t xo = ((size_t)ref.l0[k] * C + c) * N;
+    const double2 *x = psi + xo;
     double sr = 0.0, si = 0.0;
     for (int i = t; i < N; i += WG) {
         const double2 v = x[i];
@@ -181,29 +191,32 @@ __global__ __launch_bounds__(WG) void k_kin_ref(const double *__restrict__ psi,
         red[1][wave] = si;
     }
     __syncthreads();
-    if (t == 0) {
-        double ar = 0.0, ai = 0.0;
-        for (int w = 0; w < WG / 64; ++w) {
-            ar += red[0][w];
-            ai += red[1][w];
-        }
-        double sn, cs;
-        sincos(eps[k] * dt, &sn, &cs);
-        ab[c] = make_double4(ar, ai, cs * ar + sn * ai, cs * ai - sn * ar);
+    double ar = 0.0, ai = 0.0;
+    for (int w = 0; w < WG / 64; ++w) {
+        ar += red[0][w];
+        ai += red[1][w];
     }
+    if (t == 0) ref.ab[c] = kin_ref_ab(ref, k, ar, ai);
+    if (PREP)
+        for (int i = t; i < N; i += WG) {
+            double2 v = x[i];
+            const double f = ph[i];
+            v.x -= ar * f;
+            v.y -= ai * f;
+            psi32[xo + i] = make_float2((float)v.x, (float)v.y);
+        }
 }
 
 // FP32 copy of the state for the tiled pass 1, the ground-state component
 // alpha phi taken out (mixed form): psi32[l][c][i] = psi - [l = l0] alpha phi.
-// only_l0: just the ground-state block of each column (the other blocks were
-// written by the angular kernel's first half, which ends every step's input)
+// (In a step the angular kernel's first half writes the other blocks, and k_kin_ref<true> these.)
 __global__ __launch_bounds__(WG) void k_kin_prep(const double2 *__restrict__ psi, KinRef ref,
                                                  float2 *__restrict__ psi32, int N, int C,
-                                                 int n_orb, int only_l0) {
+                                                 int n_orb) {
     const int i = blockIdx.x * WG + threadIdx.x;
     const int c = blockIdx.y;
     const int k = c % n_orb;
-    const int l = only_l0 ? ref.l0[k] : blockIdx.z;
+    const int l = blockIdx.z;
     if (i >= N) return;
     const size_t o = ((size_t)l * C + c) * N + i;
     double2 v = psi[o];
@@ -272,6 +285,7 @@ __global__ __launch_bounds__(KIN_NARROW_WG) void k_kin_fwd(const float *__restri
     typedef float vta __attribute__((ext_vector_type(TA)));
     constexpr int NW = KIN_NW;
     __shared__ double red[NW][TA][64][4];
+    __shared__ double part[8][4][2];
     const tile3 tb = xcd_tile();  // (eigen panel, column tile, l): panels of one l share psi
     const int l = tb.z;
     const int nk = nkeep[l];
@@ -288,8 +302,47 @@ __global__ __launch_bounds__(KIN_NARROW_WG) void k_kin_fwd(const float *__restri
     const double *Xl = psi + ((size_t)l * C + (colok ? c : 0)) * N * 2 + p;
     const int kq = (((N + NW - 1) / NW + 3) / 4) * 4;  // K share of a wave, multiple of 4
     const int kb = wave * kq, ke = min(N, kb + kq);
+    // alpha of the tile's columns whose ground-state block this is, with the sums of k_kin_ref:
+    // part w of a column, its nodes i = 64 w + lane mod 256, is one wave's task.  Every panel of
+    // the block forms it (two rounds of loads more in these work-groups; as a launch of its
+    // own it took 3 us of a step), and the first one stores it for pass 2.
+    unsigned own = 0;  // columns of this block
+    if (ref.phi)
+        for (int q = 0; q < 8; ++q) {
+            const int cq = tb.y * 8 + q;
+            if (cq < C && ref.l0[cq % n_orb] == l) own |= 1u << q;
+        }
     double rc = 0.0;
-    const double *rrow = colok ? kin_ref_row(ref, l, c, p, N, n_orb, false, &rc) : nullptr;
+    const double *rrow = nullptr;
+    if (own) {
+        int task = wave;
+        for (unsigned left = own; left; left &= left - 1, task -= 4) {
+            for (; task >= 0 && task < 4; task += NW) {
+                const int q = __builtin_ctz(left), cq = tb.y * 8 + q;
+                const double *ph = ref.phi + (size_t)(cq % n_orb) * N;
+                const double2 *x = (const double2 *)psi + ((size_t)l * C + cq) * N;
+                double sr = 0.0, si = 0.0;
+                for (int i = 64 * task + lane; i < N; i += 256) {
+                    const double2 v = x[i];
+                    sr += ph[i] * v.x;
+                    si += ph[i] * v.y;
+                }
+                for (int off = 32; off > 0; off >>= 1) {
+                    sr += __shfl_down(sr, off);
+                    si += __shfl_down(si, off);
+                }
+                if (lane == 0) {
+                    part[q][task][0] = sr;
+                    part[q][task][1] = si;
+                }
+            }
+        }
+        __syncthreads();
+        if (own >> (lc >> 1) & 1) {
+            for (int w = 0; w < 4; ++w) rc += part[lc >> 1][w][p];
+            rrow = ref.phi + (size_t)(c % n_orb) * N;
+        }
+    }
     // wave w < 4 finishes accumulator row w of every tile: its phase factors
     // are loaded ahead of the products
     const int ar = mfma_t<float>::row(kr, wave & 3);
@@ -333,7 +386,17 @@ __global__ __launch_bounds__(KIN_NARROW_WG) void k_kin_fwd(const float *__restri
 #pragma unroll
         for (int r = 0; r < 4; ++r) red[wave > 0 ? wave - 1 : NW - 1][t][lane][r] = (double)acc[t][r];
     __syncthreads();
-    if (wave >= 4) return;
+    if (wave >= 4) {
+        if (wave == 4 && tb.x == 0 && lane < 8 && (own >> lane & 1)) {
+            double ar = 0.0, ai = 0.0;
+            for (int w = 0; w < 4; ++w) {
+                ar += part[lane][w][0];
+                ai += part[lane][w][1];
+            }
+            ref.ab[tb.y * 8 + lane] = kin_ref_ab(ref, (tb.y * 8 + lane) % n_orb, ar, ai);
+        }
+        return;
+    }
     const int r = wave;
 #pragma unroll
     for (int t = 0; t < TA; ++t) {
@@ -4311,12 +4374,18 @@ static void launch_kinetic_mixed(ggb_ctx *ctx, int pass, bool fresh, hipEvent_t 
     KinRef ref;
     ref.phi = ctx->have_ref ? ctx->phi_ref : nullptr;
     ref.l0 = ctx->l0;
+    ref.eps = ctx->eps;
     ref.ab = ctx->ab;
     ref.active = ctx->active;
-    if (pass == 0 && ref.phi)
-        k_kin_ref<<<ctx->C, WG, 0, ctx->stream>>>(ctx->psi, ctx->phi_ref, ctx->l0, ctx->eps, ctx->ab,
-                                                  p.n_r, ctx->C, p.n_orb, p.dt);
+    ref.dt = p.dt;
     const int var = kin_variant(ctx);
+    const bool tiled = var == GGB_KIN_TILED16 || var == GGB_KIN_TILED32;
+    if (pass == 0 && ref.phi && var != GGB_KIN_NARROW) {
+        if (tiled && fresh)
+            k_kin_ref<true><<<ctx->C, WG, 0, ctx->stream>>>((const double2 *)ctx->psi, ref, ctx->psi32, p.n_r, ctx->C, p.n_orb);
+        else
+            k_kin_ref<false><<<ctx->C, WG, 0, ctx->stream>>>((const double2 *)ctx->psi, ref, nullptr, p.n_r, ctx->C, p.n_orb);
+    }
     if (var == GGB_KIN_SPLIT16) {
         const int nct = (2 * ctx->C + TN - 1) / TN;
         const dim3 gf((p.nk_max + TM - 1) / TM, nct, p.n_l), gb((p.n_r + TM - 1) / TM, nct, p.n_l);
@@ -4340,9 +4409,9 @@ static void launch_kinetic_mixed(ggb_ctx *ctx, int pass, bool fresh, hipEvent_t 
     if (var >= GGB_KIN_TILED16) {
         const int nct = (2 * ctx->C + TN - 1) / TN;
         const dim3 gf((p.nk_max + TM - 1) / TM, nct, p.n_l), gb((p.n_r + TM - 1) / TM, nct, p.n_l);
-        if (pass == 0 && !(fresh && !ref.phi))
-            k_kin_prep<<<dim3((p.n_r + WG - 1) / WG, ctx->C, fresh ? 1 : p.n_l), WG, 0, ctx->stream>>>(
-                (const double2 *)ctx->psi, ref, ctx->psi32, p.n_r, ctx->C, p.n_orb, fresh ? 1 : 0);
+        if (pass == 0 && !fresh)
+            k_kin_prep<<<dim3((p.n_r + WG - 1) / WG, ctx->C, p.n_l), WG, 0, ctx->stream>>>((const double2 *)ctx->psi, ref,
+                                                                                         ctx->psi32, p.n_r, ctx->C, p.n_orb);
         if (var == GGB_KIN_TILED16 && ctx->C <= K32_MAX_C) return launch_kin32(ctx, pass, ref, e0, e1);
         const bool k32 = var == GGB_KIN_TILED32;
         const double2 *kph = ctx->kph;
