@@ -4348,10 +4348,24 @@ static void launch_kin32_t(ggb_ctx *ctx, int pass, const KinRef &ref, hipEvent_t
         kin_launch(k_kin32<0, TA, TB>, grid, WG, ctx->stream, e0, e1, g);
 }
 
-// TILED16 up to K32_MAX_C columns; beyond, the 64 x 128 tiles waste less than the half-width column
-// groups cost (argon, passes 0 / 1: 35 columns 42 / 40 against 52 / 60 us, 63 columns 64 / 60
-// against 53 / 61; krypton, 52 columns 151 / 137 against 130 / 144)
+// TILED16 up to K32_MAX_C columns always.  Beyond, the 64 x 128 tiles need fewer loads per
+// product, and win where they are full and there is one for every CU: k_kin32 is taken where a
+// pass has fewer than K32_MAX_WG of them, or where less than K32_FILL of them is output (up to
+// 4 for every CU).  Both passes, us, tiles / k_kin32: N_r = 96, 13 l, 100 columns (52 tiles) 37 / 20;
+// 256, 33 l, 100 columns (264 tiles, 0.63 full) 70 / 47, 400 columns (924, 0.72) 113 / 110, 1000
+// columns (0.79) 216 / 226; 384, 49 l, 64 columns (245, 0.95) 77 / 88; 512, 65 l, 84 columns
+// (910, 0.656) 201 / 163, 112 columns (910, 0.875) 203 / 210, 448 columns 544 / 643.
 #define K32_MAX_C 40
+#define K32_MAX_WG 240
+#define K32_FILL 0.66
+static bool kin32_better(const ggb_ctx *ctx) {
+    const ggb_problem &p = ctx->p;
+    if (ctx->C <= K32_MAX_C) return true;
+    const double rows = (p.nk_max + TM - 1) / TM, cols = (2 * ctx->C + TN - 1) / TN;
+    const double fill = (double)p.nk_max * 2 * ctx->C / (rows * TM * cols * TN), wg = rows * cols * p.n_l;
+    return wg < K32_MAX_WG || (fill < K32_FILL && wg <= 4 * 256);
+}
+
 // Shape by the number of 16 x 16 output tiles of a pass.  Up to about four waves per SIMD one tile per
 // wave (neon, 32 columns, 4116 tiles: 19 / 18 us; two rows of tiles 21 / 18, four 24 / 21); with more, operand
 // traffic counts: 2 x 2 tiles for one pair of column tiles (krypton, 13 columns, 7372 tiles: 53 / 56
@@ -4412,7 +4426,7 @@ static void launch_kinetic_mixed(ggb_ctx *ctx, int pass, bool fresh, hipEvent_t 
         if (pass == 0 && !fresh)
             k_kin_prep<<<dim3((p.n_r + WG - 1) / WG, ctx->C, p.n_l), WG, 0, ctx->stream>>>((const double2 *)ctx->psi, ref,
                                                                                          ctx->psi32, p.n_r, ctx->C, p.n_orb);
-        if (var == GGB_KIN_TILED16 && ctx->C <= K32_MAX_C) return launch_kin32(ctx, pass, ref, e0, e1);
+        if (var == GGB_KIN_TILED16 && kin32_better(ctx)) return launch_kin32(ctx, pass, ref, e0, e1);
         const bool k32 = var == GGB_KIN_TILED32;
         const double2 *kph = ctx->kph;
         const int32_t *nkeep = ctx->nkeep;

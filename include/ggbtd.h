@@ -227,8 +227,8 @@ void ggb_group_destroy(ggb_group *g);
  * form DEFAULT is NARROW up to 8 orbital columns, else TILED16.  NARROW: 16x16
  * tiles with the contraction split over the work-group's waves; TILED16 /
  * TILED32: sums in K chunks of 16 / 32 (TILED32 in the mixed form only), on 64x128
- * work-group tiles in LDS, or for TILED16 up to 40 orbital columns on tiles of 16
- * to 64 rows by 16 or 32 real columns per wave, with the same results. */
+ * work-group tiles in LDS, or for TILED16 with few columns or a small grid on tiles of
+ * 16 to 64 rows by 16 or 32 real columns per wave, with the same results. */
 #define GGB_KIN_DEFAULT 0
 #define GGB_KIN_NARROW 1
 #define GGB_KIN_TILED16 2

@@ -97,3 +97,17 @@ def test_mixed_passes_large_shapes():
     for inst in (10, 4, 3):
         got = run(inst)
         assert np.array_equal(got, wide[:, :4 * inst]), inst
+
+
+@pytest.mark.parametrize("N", [80, 75])
+def test_mixed_passes_many_columns(N):
+    """More than 40 columns: a pass with fewer than 240 tiles of 64 x 128 (448 columns and 33 l
+    here, or partly filled tiles) takes the small tiles, one with more full ones (512 columns) the large ones."""
+    print("case: mixed kinetic passes, many columns, N", N, flush=True)
+    S = AtomSystem("He", N, 30.0, 32, 0.05)
+    psi = _random_columns(S, 512)
+    wide = _mixed(S, psi, 512, "tiled16")
+    assert np.abs(wide - _kinetic(S, psi)).max() < 4 * (18 + N / 16) * 2.0 ** -24
+    for columns in (448, 300, 67, 41):
+        got = _mixed(S, psi[:, :columns].copy(), columns, "tiled16")
+        assert np.array_equal(got, wide[:, :columns]), columns
