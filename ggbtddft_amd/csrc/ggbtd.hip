@@ -702,6 +702,24 @@ __global__ __launch_bounds__(WG) void k_kin_transpose(const double *__restrict__
         if (a0 + y < nk_max && i0 + tx < np) Tl[(size_t)(a0 + y) * np + i0 + tx] = tile[tx][y];
 }
 
+// Tables of the mixed form from the FP64 one, at upload.  On the host the rounding and the scattered
+// stores of QT took 12 of the 14 ms of an upload at N_r = 384, 49 l (46 MB in FP64, which the copy
+// moves in 1.5 ms).
+__global__ __launch_bounds__(WG) void k_round32(const double2 *__restrict__ x, float2 *__restrict__ y, size_t n) {
+    const size_t k = (size_t)blockIdx.x * WG + threadIdx.x;
+    if (k >= n) return;
+    const double2 v = x[k];
+    y[k] = make_float2((float)v.x, (float)v.y);
+}
+// QT of the narrow pass 2 (kin_qt_index), four a of one node per thread
+__global__ __launch_bounds__(WG) void k_kin_pack_qt(const float *__restrict__ Q, float *__restrict__ QT, int N, int nk_max) {
+    const int i = blockIdx.x * 64 + (threadIdx.x & 63), a4 = blockIdx.y * (WG / 64) + (threadIdx.x >> 6);
+    const size_t l = blockIdx.z;
+    if (i >= N || 4 * a4 >= nk_max) return;
+    const float4 v = *reinterpret_cast<const float4 *>(Q + (l * N + i) * nk_max + 4 * a4);
+    *reinterpret_cast<float4 *>(QT + kin_qt_index(l, i, 4 * a4, N, nk_max)) = v;
+}
+
 // ---------------------------------------------------------------------------
 // Mixed form, tiled passes for many columns (instances sharing the tables).
 // Work-group tile 64 (M) x 128 (real columns); wave w owns the 32 x 64
@@ -3959,22 +3977,24 @@ extern "C" int ggb_upload_static(ggb_ctx *ctx, const ggb_static *s) {
             const int np = round16(p.n_r);
             k_kin_transpose<<<dim3((p.nk_max + 31) / 32, (np + 31) / 32, p.n_l), WG, 0, st>>>(ctx->Q, ctx->QT, p.n_r, p.nk_max, np);
             HIPCHK(ctx, hipGetLastError());
+        } else if (ctx->QT) {
+            // the FP64 table in two halves through QT's memory, then QT itself
+            float *Q32 = reinterpret_cast<float *>(ctx->Q), *QT = reinterpret_cast<float *>(ctx->QT);
+            for (size_t k0 = 0; k0 < nQ; k0 += nQ / 2) {  // nQ is a multiple of 16
+                HIPCHK(ctx, hipMemcpyAsync(QT, s->Q + k0, nQ / 2 * 8, hipMemcpyHostToDevice, st));
+                k_round32<<<(unsigned)((nQ / 4 + WG - 1) / WG), WG, 0, st>>>(reinterpret_cast<const double2 *>(QT),
+                                                                             reinterpret_cast<float2 *>(Q32 + k0), nQ / 4);
+                HIPCHK(ctx, hipGetLastError());
+            }
+            k_kin_pack_qt<<<dim3((unsigned)((N + 63) / 64), (unsigned)((nk / 4 + 3) / 4), p.n_l), WG, 0, st>>>(Q32, QT, p.n_r, p.nk_max);
+            HIPCHK(ctx, hipGetLastError());
         } else {
             std::vector<float> q32(nQ);
             for (size_t k = 0; k < nQ; ++k) q32[k] = (float)s->Q[k];
             HIPCHK(ctx, hipMemcpy(ctx->Q, q32.data(), nQ * 4, hipMemcpyHostToDevice));
-            if (ctx->QT) {
-                std::vector<float> qt(nQ);
-                for (size_t l = 0; l < Nl; ++l)
-                    for (size_t i = 0; i < N; ++i)
-                        for (size_t a = 0; a < nk; ++a) qt[kin_qt_index(l, i, a, N, nk)] = q32[(l * N + i) * nk + a];
-                HIPCHK(ctx, hipMemcpy(ctx->QT, qt.data(), nQ * 4, hipMemcpyHostToDevice));
-            }
-            if (ctx->Qlo) {  // low parts: Q - fl32(Q), rounded to FP32
-                std::vector<float> lo(nQ);
-                for (size_t k = 0; k < nQ; ++k) lo[k] = (float)(s->Q[k] - (double)q32[k]);
-                HIPCHK(ctx, hipMemcpy(ctx->Qlo, lo.data(), nQ * 4, hipMemcpyHostToDevice));
-            }
+            std::vector<float> lo(nQ);  // low parts: Q - fl32(Q), rounded to FP32
+            for (size_t k = 0; k < nQ; ++k) lo[k] = (float)(s->Q[k] - (double)q32[k]);
+            HIPCHK(ctx, hipMemcpy(ctx->Qlo, lo.data(), nQ * 4, hipMemcpyHostToDevice));
         }
     }
     {

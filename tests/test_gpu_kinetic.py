@@ -111,3 +111,15 @@ def test_mixed_passes_many_columns(N):
     for columns in (448, 300, 67, 41):
         got = _mixed(S, psi[:, :columns].copy(), columns, "tiled16")
         assert np.array_equal(got, wide[:, :columns]), columns
+
+
+# The tables that the upload rounds to FP32 and packs for the narrow pass 2, at sizes with partial blocks of
+# 64 nodes and of 16 eigenvalues.  A wave sums up to N / 8 products in FP32, eight waves' sums are added
+# in FP64: 2 + N / 8 roundings a pass at most.
+@pytest.mark.parametrize("N", [130, 96, 75, 21])
+def test_mixed_tables_packed_at_upload(N):
+    print("case: mixed tables, N", N, flush=True)
+    S = _system(N)
+    psi = _random_columns(S, 8)
+    got = _mixed(S, psi, 8, "narrow")
+    assert np.abs(got - _kinetic(S, psi)).max() < 4 * (18 + N / 8) * 2.0 ** -24
