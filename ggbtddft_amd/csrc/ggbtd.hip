@@ -18,7 +18,7 @@
 //   k_kin64<1>          psi = Q Y                        grid (N/32,  2C/32, n_l)
 //   (mixed form: k_kin_fwd / k_kin_bwd, 16-wide tiles, or k_kin_*_dma / _tiled, 64 x 128 tiles)
 //   k_angular<mode 1>   Lo, Le, Vh, |B psi|^2, observable partials
-//   k_rho               rho_u = sum occ |Psi|^2, v_xc; observable sums
+//   k_rho               rho_u = sum occ |Psi|^2, v_xc; observable sums, channel dipoles
 //   k_tile_gemm<Qmom>   multipole moments q_L = P_L^T rho_u (small contexts: both in k_rho_mom)
 //   k_hartree           V_L by prefix/suffix affine scans  grid (n_har, n_inst)
 //   k_tile_gemm<Dv>     dV = sum_L V_L P_L, v_xc - v_gs, phase factors of the next step
@@ -2725,8 +2725,8 @@ struct ChanArgs {
     const int *cur, *origin;     // graph replay: row = cur[0] - origin[0] + local
     int local;
 };
-__global__ __launch_bounds__(64) void k_chan_dip(ChanArgs a) {
-    const int l = blockIdx.x, c = blockIdx.y, lane = threadIdx.x;
+static __device__ void chan_pair(const ChanArgs &a, int l, int c) {
+    const int lane = threadIdx.x & 63;
     const int m = a.mcol[c % a.n_orb];
     const size_t row = a.cur ? (size_t)(a.cur[0] - a.origin[0] + a.local) : (size_t)a.local;
     double sr = 0.0, si = 0.0;
@@ -2751,6 +2751,8 @@ __global__ __launch_bounds__(64) void k_chan_dip(ChanArgs a) {
     }
     if (lane == 0) a.chan[(row * a.C + c) * a.Nl + l] = make_double2(sr, si);
 }
+// by itself where no density kernel follows (without interaction)
+__global__ __launch_bounds__(64) void k_chan_dip(ChanArgs a) { chan_pair(a, blockIdx.x, blockIdx.y); }
 
 // advances the replayed graph's step counter
 __global__ void k_bump(int *cur, int by) {
@@ -2800,14 +2802,22 @@ struct RhoArgs {
     int N, Nth, h, hq, n_orb;
     const int32_t *active;
 };
-// grid blocks `block` of nrho, then the observable sums of the step, one (column, observable)
-// pair per wave (instance 0's blocks); rho_u is stored where it is not null
+// grid blocks `block` of nrho, then the observable sums of the step and the instance's channel
+// dipoles (each a launch of 3 to 5 us by itself), one (orbital, observable or l) pair per wave;
+// rho_u is stored where it is not null
+static __host__ __device__ int rho_pair_blocks(int pairs) { return (pairs + WG / 64 - 1) / (WG / 64); }
 template <typename T>
-static __device__ __forceinline__ void rho_block(const RhoArgs &a, const ObsArgs &ob, int block, int inst) {
+static __device__ __forceinline__ void rho_block(const RhoArgs &a, const ObsArgs &ob, const ChanArgs &ch, int block, int inst) {
     const int nrho = (int)(((size_t)a.N * a.Nth + WG - 1) / WG);
     if (block >= nrho) {
-        const int pair = (block - nrho) * (WG / 64) + (threadIdx.x >> 6);
-        if (inst == 0 && ob.obs && pair < ob.C * 3) obs_reduce_pair(ob, pair);
+        const int no = ob.obs ? rho_pair_blocks(3 * a.n_orb) : 0;
+        const bool chan = block - nrho >= no;
+        const int pair = (block - nrho - (chan ? no : 0)) * (WG / 64) + (threadIdx.x >> 6);
+        if (chan) {
+            if (pair < a.n_orb * ch.Nl) chan_pair(ch, pair % ch.Nl, inst * a.n_orb + pair / ch.Nl);
+        } else if (pair < 3 * a.n_orb) {
+            obs_reduce_pair(ob, inst * a.n_orb * 3 + pair);
+        }
         return;
     }
     if (a.active && !a.active[inst]) return;  // idle serving slot (block-uniform)
@@ -2839,8 +2849,8 @@ static __device__ __forceinline__ void rho_block(const RhoArgs &a, const ObsArgs
     a.vxc[o] = (double)lda_vxc<T>((T)rho);
 }
 template <typename T>
-__global__ __launch_bounds__(WG) void k_rho(RhoArgs a, ObsArgs ob) {
-    rho_block<T>(a, ob, blockIdx.x, blockIdx.y);
+__global__ __launch_bounds__(WG) void k_rho(RhoArgs a, ObsArgs ob, ChanArgs ch) {
+    rho_block<T>(a, ob, ch, blockIdx.x, blockIdx.y);
 }
 
 // k_rho and the multipole moments q_L(i) = sum_j P_L(chi_j) rho_u(i, j) in one launch, for small
@@ -2861,11 +2871,11 @@ __global__ __launch_bounds__(WG) void k_rho(RhoArgs a, ObsArgs ob) {
 #define MOM_U 9  // theta values of a lane per round: a quarter of N_theta = 129
 static size_t mom_lds(int Nth) { return std::max<size_t>((size_t)16 * (Nth | 1), 4 * 64 * 4) * sizeof(double); }
 template <typename T>
-__global__ __launch_bounds__(WG) void k_rho_mom(RhoArgs a, ObsArgs ob, const double *__restrict__ PL, double *__restrict__ q,
+__global__ __launch_bounds__(WG) void k_rho_mom(RhoArgs a, ObsArgs ob, ChanArgs ch, const double *__restrict__ PL, double *__restrict__ q,
                                                 int n_har, int nmom) {
     extern __shared__ __align__(16) double lds[];  // rho_u [16][Nth | 1], then the partial tiles
     const int inst = blockIdx.y;
-    if ((int)blockIdx.x >= nmom) return rho_block<T>(a, ob, (int)blockIdx.x - nmom, inst);
+    if ((int)blockIdx.x >= nmom) return rho_block<T>(a, ob, ch, (int)blockIdx.x - nmom, inst);
     if (a.active && !a.active[inst]) return;  // idle serving slot (block-uniform)
     const int ni = (a.N + 15) / 16;
     const int i0 = (int)blockIdx.x % ni * 16, L0 = (int)blockIdx.x / ni * 16;
@@ -4192,7 +4202,7 @@ static hipError_t no_mark_k(int) { return hipSuccess; }
 
 // mk(0) after the density kernel, mk(1) after the Hartree scans (timing events)
 template <typename MarkK = hipError_t (*)(int)>
-static int launch_potential(ggb_ctx *ctx, const ObsArgs *ob = nullptr, MarkK mk = no_mark_k) {
+static int launch_potential(ggb_ctx *ctx, const ObsArgs *ob = nullptr, MarkK mk = no_mark_k, const ChanArgs *chan = nullptr) {
     const ggb_problem &p = ctx->p;
     hipStream_t st = ctx->stream;
     const int N = p.n_r, Nth = p.n_theta, nh = p.n_har;
@@ -4202,8 +4212,10 @@ static int launch_potential(ggb_ctx *ctx, const ObsArgs *ob = nullptr, MarkK mk 
     if (oa.obs && !p.interacting) k_obs_reduce<<<oa.C * 3, 64, 0, st>>>(oa);
     if (p.interacting) {
         const unsigned nrho = (unsigned)(((size_t)N * Nth + WG - 1) / WG);
-        const unsigned nobs = oa.obs ? (unsigned)((oa.C * 3 + WG / 64 - 1) / (WG / 64)) : 0u;
-        const dim3 gr(nrho + nobs, p.n_inst);
+        ChanArgs ch = ChanArgs();
+        if (chan) ch = *chan;
+        const unsigned nobs = oa.obs ? rho_pair_blocks(3 * p.n_orb) : 0, nchan = chan ? rho_pair_blocks(p.n_orb * p.n_l) : 0;
+        const dim3 gr(nrho + nobs + nchan, p.n_inst);
         const int ntl = (nh + 15) / 16;
         const unsigned nmom = (unsigned)((N + 15) / 16 * ntl);
         // moments in the same launch
@@ -4213,14 +4225,14 @@ static int launch_potential(ggb_ctx *ctx, const ObsArgs *ob = nullptr, MarkK mk 
         if (one) {
             const dim3 gm(nmom + gr.x, p.n_inst);
             if (p.precision)
-                k_rho_mom<float><<<gm, WG, mom_lds(Nth), st>>>(ra, oa, ctx->PL, ctx->q, nh, (int)nmom);
+                k_rho_mom<float><<<gm, WG, mom_lds(Nth), st>>>(ra, oa, ch, ctx->PL, ctx->q, nh, (int)nmom);
             else
-                k_rho_mom<double><<<gm, WG, mom_lds(Nth), st>>>(ra, oa, ctx->PL, ctx->q, nh, (int)nmom);
+                k_rho_mom<double><<<gm, WG, mom_lds(Nth), st>>>(ra, oa, ch, ctx->PL, ctx->q, nh, (int)nmom);
         } else {
             if (p.precision)
-                k_rho<float><<<gr, WG, 0, st>>>(ra, oa);
+                k_rho<float><<<gr, WG, 0, st>>>(ra, oa, ch);
             else
-                k_rho<double><<<gr, WG, 0, st>>>(ra, oa);
+                k_rho<double><<<gr, WG, 0, st>>>(ra, oa, ch);
             GemmOperands gq;  // q[L][i] = sum_j PLT[L][j] rho_u[i][j]
             gq.A = ctx->PLT;
             gq.sam = Nth;
@@ -4509,7 +4521,7 @@ static hipError_t no_mark() { return hipSuccess; }
 
 // channel dipoles of the state after the step into dst (row 0, or the
 // replay row cur[0] - cur[1] + step)
-static void launch_channels(ggb_ctx *ctx, int step, double2 *dst, const int *cur) {
+static ChanArgs chan_args(ggb_ctx *ctx, int step, double2 *dst, const int *cur) {
     ChanArgs a;
     a.psi = ctx->psi;
     a.r = ctx->r;
@@ -4523,7 +4535,7 @@ static void launch_channels(ggb_ctx *ctx, int step, double2 *dst, const int *cur
     a.cur = cur;
     a.origin = cur ? cur + 1 : nullptr;
     a.local = cur ? step : 0;
-    k_chan_dip<<<dim3(ctx->p.n_l, ctx->C), 64, 0, ctx->stream>>>(a);
+    return a;
 }
 
 template <typename Mark = hipError_t (*)(), typename MarkK = hipError_t (*)(int)>
@@ -4532,7 +4544,10 @@ static int launch_second_half(ggb_ctx *ctx, int step, double *obs_dst, const int
                               MarkK mk = no_mark_k) {
     launch_angular<1>(ctx, step, cur);
     HIPCHK(ctx, hipGetLastError());
-    if (chan_dst) launch_channels(ctx, step, chan_dst, cur);
+    ChanArgs ch;
+    if (chan_dst) ch = chan_args(ctx, step, chan_dst, cur);
+    const bool own = chan_dst && !ctx->p.interacting;  // else with the density
+    if (own) k_chan_dip<<<dim3(ctx->p.n_l, ctx->C), 64, 0, ctx->stream>>>(ch);
     HIPCHK(ctx, between());  // timing event between the angular half and the rebuild
     ObsArgs ob;
     ob.part = ctx->obs_part;
@@ -4542,7 +4557,7 @@ static int launch_second_half(ggb_ctx *ctx, int step, double *obs_dst, const int
     ob.cur = cur;
     ob.origin = cur ? cur + 1 : nullptr;
     ob.local = step;
-    return launch_potential(ctx, &ob, mk);
+    return launch_potential(ctx, &ob, mk, chan_dst && !own ? &ch : nullptr);
 }
 
 extern "C" int ggb_upload_orbitals(ggb_ctx *ctx, const double *psi) {

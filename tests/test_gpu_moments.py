@@ -38,3 +38,42 @@ def test_one_launch_equals_two(atom, N, lmax, n_theta, few, many, precision):
     assert np.abs(one).max() > 1e-3
     assert all(np.array_equal(v, one[0]) for v in one)
     assert all(np.array_equal(v, one[0]) for v in two)
+
+
+@pytest.mark.parametrize("atom, N, lmax, n", [("Ar", 75, 40, 1), ("Ar", 75, 40, 9), ("Ne", 203, 48, 6), ("H", 50, 11, 3)])
+def test_channel_dipoles_with_the_density(atom, N, lmax, n):
+    """Channel dipoles from the launch of the density (one launch, two, and by itself without
+    interaction), against numpy on the orbitals after the step; idle instances hold zero.  A sum of
+    4 N products: 8 N eps of the sum of their sizes."""
+    from ggbtddft_amd.engine import Propagator
+    print("case: channel dipoles,", atom, N, lmax, n, flush=True)
+    S = AtomSystem(atom, N, 40.0, lmax, 0.05, ground_state="device", tables="device")
+    rng = np.random.default_rng(n)
+    E = 0.3 * rng.standard_normal((n, 3))
+    active = np.ones(n, dtype=bool)
+    active[1:n - 1:3] = False
+    with Propagator(S, n_inst=n) as prop:
+        prop.set_field(E)
+        prop.set_active(active)
+        got = prop.run(0, 2, channels=True)["chan"][-1].reshape(n, S.n_orb, S.n_l)
+        psi = prop.download_orbitals().reshape(S.n_l, n, S.n_orb, S.N)
+    r = S.grid.r
+    for k in range(S.n_orb):
+        m = S.m[k]
+        for l in range(S.n_l):
+            if l < m:
+                assert not got[:, k, l].any()
+                continue
+
+            def c(a):
+                return np.sqrt(((a + 1) ** 2 - m * m) / ((2 * a + 1) * (2 * a + 3)))
+            z = np.zeros((n, S.N), dtype=complex)
+            size = np.zeros((n, S.N))
+            for f, b in ((c(l), l + 1), (c(l - 1) if l > m else 0.0, l - 1)):
+                if f and m <= b < S.n_l:
+                    z += f * r * psi[b, :, k]
+                    size += 2 * f * r * np.abs(psi[b, :, k])
+            ref = (psi[l, :, k].conj() * z).sum(axis=1)
+            tol = 8 * N * 2.0 ** -53 * (np.abs(psi[l, :, k]) * size).sum(axis=1)
+            assert (np.abs(got[:, k, l] - ref)[active] <= tol[active]).all(), (k, l)
+            assert not got[~active, k, l].any()
