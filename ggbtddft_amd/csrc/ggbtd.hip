@@ -2848,8 +2848,17 @@ static __device__ __forceinline__ void rho_block(const RhoArgs &a, const ObsArgs
     if (a.rho_u) a.rho_u[o] = ru;
     a.vxc[o] = (double)lda_vxc<T>((T)rho);
 }
+// The pointers once more as kernel arguments, which can be declared free of aliases: scalar loads of the
+// tables (64 argon instances: 107 us for density and moments, 110 without).
+#define RHO_PTRS                                                                                                  \
+    const T *__restrict__ dens, const double *__restrict__ occ, const double *__restrict__ rho_frozen,            \
+        const double *__restrict__ r, const double *__restrict__ wr, const double *__restrict__ omega,            \
+        double *__restrict__ rho_u, double *__restrict__ vxc
+#define RHO_PTRS_OF(T, a) reinterpret_cast<const T *>((a).dens), (a).occ, (a).rho_frozen, (a).r, (a).wr, (a).omega, (a).rho_u, (a).vxc
+#define RHO_ARGS(a) RhoArgs{dens, occ, rho_frozen, r, wr, omega, rho_u, vxc, (a).N, (a).Nth, (a).h, (a).hq, (a).n_orb, (a).active}
 template <typename T>
-__global__ __launch_bounds__(WG) void k_rho(RhoArgs a, ObsArgs ob, ChanArgs ch) {
+__global__ __launch_bounds__(WG) void k_rho(RHO_PTRS, RhoArgs g, ObsArgs ob, ChanArgs ch) {
+    const RhoArgs a = RHO_ARGS(g);
     rho_block<T>(a, ob, ch, blockIdx.x, blockIdx.y);
 }
 
@@ -2871,9 +2880,10 @@ __global__ __launch_bounds__(WG) void k_rho(RhoArgs a, ObsArgs ob, ChanArgs ch) 
 #define MOM_U 9  // theta values of a lane per round: a quarter of N_theta = 129
 static size_t mom_lds(int Nth) { return std::max<size_t>((size_t)16 * (Nth | 1), 4 * 64 * 4) * sizeof(double); }
 template <typename T>
-__global__ __launch_bounds__(WG) void k_rho_mom(RhoArgs a, ObsArgs ob, ChanArgs ch, const double *__restrict__ PL, double *__restrict__ q,
+__global__ __launch_bounds__(WG) void k_rho_mom(RHO_PTRS, RhoArgs g, ObsArgs ob, ChanArgs ch, const double *__restrict__ PL, double *__restrict__ q,
                                                 int n_har, int nmom) {
     extern __shared__ __align__(16) double lds[];  // rho_u [16][Nth | 1], then the partial tiles
+    const RhoArgs a = RHO_ARGS(g);
     const int inst = blockIdx.y;
     if ((int)blockIdx.x >= nmom) return rho_block<T>(a, ob, ch, (int)blockIdx.x - nmom, inst);
     if (a.active && !a.active[inst]) return;  // idle serving slot (block-uniform)
@@ -2953,8 +2963,8 @@ __global__ __launch_bounds__(WG) void k_rho_mom(RhoArgs a, ObsArgs ob, ChanArgs 
 #pragma unroll
     for (int r = 0; r < 4; ++r) red[wave > 0 ? wave - 1 : 3][lane][r] = acc[r];
     __syncthreads();
-    const int r = wave, L = L0 + mfma_t<double>::row(kr, r);
-    const double v = ((red[3][lane][r] + red[0][lane][r]) + red[1][lane][r]) + red[2][lane][r];
+    const int L = L0 + mfma_t<double>::row(kr, wave);  // accumulator row `wave`
+    const double v = ((red[3][lane][wave] + red[0][lane][wave]) + red[1][lane][wave]) + red[2][lane][wave];
     if (L < n_har && i0 + lc < a.N) q[((size_t)inst * n_har + L) * a.N + i0 + lc] = v;
 }
 
@@ -4225,14 +4235,14 @@ static int launch_potential(ggb_ctx *ctx, const ObsArgs *ob = nullptr, MarkK mk 
         if (one) {
             const dim3 gm(nmom + gr.x, p.n_inst);
             if (p.precision)
-                k_rho_mom<float><<<gm, WG, mom_lds(Nth), st>>>(ra, oa, ch, ctx->PL, ctx->q, nh, (int)nmom);
+                k_rho_mom<float><<<gm, WG, mom_lds(Nth), st>>>(RHO_PTRS_OF(float, ra), ra, oa, ch, ctx->PL, ctx->q, nh, (int)nmom);
             else
-                k_rho_mom<double><<<gm, WG, mom_lds(Nth), st>>>(ra, oa, ch, ctx->PL, ctx->q, nh, (int)nmom);
+                k_rho_mom<double><<<gm, WG, mom_lds(Nth), st>>>(RHO_PTRS_OF(double, ra), ra, oa, ch, ctx->PL, ctx->q, nh, (int)nmom);
         } else {
             if (p.precision)
-                k_rho<float><<<gr, WG, 0, st>>>(ra, oa, ch);
+                k_rho<float><<<gr, WG, 0, st>>>(RHO_PTRS_OF(float, ra), ra, oa, ch);
             else
-                k_rho<double><<<gr, WG, 0, st>>>(ra, oa, ch);
+                k_rho<double><<<gr, WG, 0, st>>>(RHO_PTRS_OF(double, ra), ra, oa, ch);
             GemmOperands gq;  // q[L][i] = sum_j PLT[L][j] rho_u[i][j]
             gq.A = ctx->PLT;
             gq.sam = Nth;
