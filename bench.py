@@ -596,7 +596,7 @@ def main():
         "fp64_ratio_denominator": {"value": fp64_ref, "steps": ref_steps,
                                    "ms_per_step": 1e3 * ref_el / ref_steps},
         "kinetic_variant": tuned[0], "autotuner_ms_per_kinetic_step": tuned[1],
-        "roofline": {"kernel": "k_kin_fwd (kinetic propagator, Q^T pass)", "bound": "hbm",
+        "roofline": {"kernel": "k_kin64<0> (kinetic propagator, Q^T pass)", "bound": "hbm",
                      "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
                      "traffic": traffic["hbm_bytes_per_launch"] if traffic else None,
