@@ -517,9 +517,9 @@ __global__ __launch_bounds__(KIN_NARROW_WG) void k_kin_bwd(const float *__restri
 //    covers whole 128-byte lines; component-wise loads touched each line twice.
 // What bounds it: HBM up to about 16 columns (the table is read once), the FP64
 // matrix pipe beyond.  At argon size (N = 512, 65 l) passes 0 / 1 take, against the
-// LDS-tiled kernels that ran from 9 columns on: 14 columns 28 / 26 us (91 / 122),
-// 28 columns 45 / 43 us (94 / 124), 224 columns 237 / 234 us (369 / 349, 53 TFLOP/s);
-// krypton (N = 768, 97 l, 13 columns) 91 / 88 us (258 / 293).
+// LDS-tiled kernels that ran from 9 columns on: 14 columns 26 / 27 us (91 / 122),
+// 28 columns 44 / 45 us (94 / 124), 224 columns 237 / 234 us (369 / 349, 53 TFLOP/s);
+// krypton (N = 768, 97 l, 13 columns) 87 / 84 us (258 / 293).
 // ---------------------------------------------------------------------------
 #define K64_NW 4
 #define K64_WG (64 * K64_NW)
@@ -664,7 +664,8 @@ static __device__ __forceinline__ void kin64_tiles(const Kin64Args &g, int l, in
                 if (m < g.N) Dc[m] = make_double2(re, im);
             } else if (m < nk8) {  // pass 1 reads Y up to nk8
                 const double2 f = kp[t];
-                Dc[m] = m < nk ? make_double2(f.x * re + f.y * im, f.x * im - f.y * re) : make_double2(0.0, 0.0);
+                // contracted the same way in every shape
+                Dc[m] = m < nk ? make_double2(fma(f.x, re, f.y * im), fma(f.x, im, -(f.y * re))) : make_double2(0.0, 0.0);
             }
         }
     }
@@ -4349,18 +4350,27 @@ static void launch_kin64_t(ggb_ctx *ctx, int pass, hipEvent_t e0, hipEvent_t e1)
         kin_launch(k_kin64<0, TA, TB>, grid, K64_WG, ctx->stream, e0, e1, g);
 }
 
-// Shape of the FP64 passes.  NARROW: one tile of 16 real columns per work-group
-// (idle instances are skipped 8 columns at a time), and the only one up to 8
-// columns.  Otherwise two tiles, which read the table half as often; panels of
-// 32 rows up to 32 columns, where the work-groups are few, of 64 beyond
-// (argon size, passes 0 / 1: 28 columns 45 / 43 us with 32 rows, 47 / 45 with 64;
-// 63 columns 80 / 77 against 81 / 77, 224 columns 249 / 245 against 237 / 234).
-// Every element is formed by the same products in the same order in all of them.
+// Shape of the FP64 passes by the 16 x 16 output tiles of a pass.  NARROW, one column tile, and up to
+// 2000 tiles: panels of 32 rows by one tile of 16 real columns, the most work-groups.  Up to 7200
+// tiles: 64 rows by one tile.  Beyond, or where the table is larger than what the last-level cache
+// keeps for a second column tile: 64 rows by two, which read the table half as often.  Both passes,
+// us, 32 x 1 / 64 x 1 / 64 x 2: helium N = 96, 40 columns (390 tiles) 13 / 15 / 18; neon N = 256, 16
+// columns (858) 20 / 22 / 25; neon N = 384, 16 columns (1862) 33 / 32 / 36; argon N = 300, 35 columns (3485)
+// 43 / 41 / 46; argon N = 512, 21 columns (5460) 86 / 78 / 90, 28 columns (7280) 111 / 99 / 94, 63 columns
+// 205 / 178 / 169; krypton N = 768, 97 l, 13 columns (7566, 391 MB of table) 213 / 202 / 177.  (32 x 2
+// is never the fastest by more than 2 %.)  Every element is formed by the same products in the same
+// order in all of them.
+#define K64_TILES_32 2000
+#define K64_TILES_64 7200
+#define K64_TABLE_BYTES 200e6
 static void launch_kin64(ggb_ctx *ctx, int pass, hipEvent_t e0, hipEvent_t e1) {
-    if (ctx->kin_variant == GGB_KIN_NARROW || ctx->C <= 8)
+    const ggb_problem &p = ctx->p;
+    const int nct = (2 * ctx->C + 15) / 16, rows = pass ? p.n_r : p.nk_max;
+    const double tiles = (double)((rows + 15) / 16) * nct * p.n_l;
+    if (ctx->kin_variant == GGB_KIN_NARROW || nct == 1 || tiles < K64_TILES_32)
         launch_kin64_t<2, 1>(ctx, pass, e0, e1);
-    else if (ctx->C <= 32)
-        launch_kin64_t<2, 2>(ctx, pass, e0, e1);
+    else if (tiles < K64_TILES_64 && 8.0 * p.n_l * p.n_r * p.nk_max < K64_TABLE_BYTES)
+        launch_kin64_t<4, 1>(ctx, pass, e0, e1);
     else
         launch_kin64_t<4, 2>(ctx, pass, e0, e1);
 }

@@ -136,8 +136,8 @@ int ggb_upload_columns(ggb_ctx *ctx, int32_t c0, int32_t nc, const double *psi);
  * at creation).  The angular, density and potential kernels skip idle
  * instances (their columns keep stale values), and the kinetic products skip
  * every tile of orbital columns that all belong to idle instances (8
- * columns in the narrow kernels, 16 in the other FP64 ones, 8 or 16 in the tiled
- * mixed ones up to 40 columns, else 64), so a serving lane with free slots does less work.  A
+ * columns in the narrow kernels, 8 or 16 in the other FP64 ones, 8 to 64 in the tiled
+ * mixed ones), so a serving lane with free slots does less work.  A
  * slot being seated must be marked in use before ggb_rebuild_potential.  No
  * counterpart in the reference, which runs its scans one after another. */
 int ggb_set_active(ggb_ctx *ctx, const int32_t *active);
@@ -223,7 +223,7 @@ void ggb_group_destroy(ggb_group *g);
 
 /* Kinetic-pass kernel variants (tile shapes).  In FP64 every variant forms the
  * same sums in the same order: NARROW takes 16 real columns (8 orbital columns)
- * per work-group, DEFAULT and TILED16 from 9 orbital columns on 32.  In the mixed
+ * per work-group, DEFAULT and TILED16 16 or 32 by the size of the pass.  In the mixed
  * form DEFAULT is NARROW up to 8 orbital columns, else TILED16.  NARROW: 16x16
  * tiles with the contraction split over the work-group's waves; TILED16 /
  * TILED32: sums in K chunks of 16 / 32 (TILED32 in the mixed form only), on 64x128

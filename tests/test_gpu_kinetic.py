@@ -123,3 +123,27 @@ def test_mixed_tables_packed_at_upload(N):
     psi = _random_columns(S, 8)
     got = _mixed(S, psi, 8, "narrow")
     assert np.abs(got - _kinetic(S, psi)).max() < 4 * (18 + N / 8) * 2.0 ** -24
+
+
+# 65 l and 70 to 300 columns: passes of 2000 to 7200 output tiles (64 rows by one column tile) and
+# beyond (by two, the last group whole or with one tile left), with rows that end inside a panel
+@pytest.mark.parametrize("N", [96, 75])
+@pytest.mark.parametrize("columns", [71, 72, 240, 249])
+def test_fp64_passes_larger_shapes(N, columns):
+    print("case: FP64 kinetic passes, 65 l, N", N, "columns", columns, flush=True)
+    from ggbtddft_amd.engine import Propagator
+    if ("l", N) not in _systems:
+        _systems["l", N] = AtomSystem("He", N, 30.0, 64, 0.05)
+    S = _systems["l", N]
+    psi = _random_columns(S, columns)
+    ref = _kinetic(S, psi)
+    got = {}
+    for variant in ("default", "narrow"):
+        with Propagator(S, n_inst=columns) as prop:
+            prop.set_field(np.zeros(1))
+            prop.set_kinetic_variant(variant)
+            prop.upload_orbitals(psi)
+            prop.substep(1)
+            got[variant] = prop.download_orbitals()
+    assert np.array_equal(got["default"], got["narrow"])
+    assert np.abs(got["default"] - ref).max() < 4 * N * 2.0 ** -53
