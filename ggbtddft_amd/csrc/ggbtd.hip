@@ -4401,36 +4401,43 @@ static void launch_kin32_t(ggb_ctx *ctx, int pass, const KinRef &ref, hipEvent_t
 }
 
 // TILED16 up to K32_MAX_C columns always.  Beyond, the 64 x 128 tiles need fewer loads per
-// product, and win where they are full and there is one for every CU: k_kin32 is taken where a
-// pass has fewer than K32_MAX_WG of them, or where less than K32_FILL of them is output (up to
-// 4 for every CU).  Both passes, us, tiles / k_kin32: N_r = 96, 13 l, 100 columns (52 tiles) 37 / 20;
-// 256, 33 l, 100 columns (264 tiles, 0.63 full) 70 / 47, 400 columns (924, 0.72) 113 / 110, 1000
-// columns (0.79) 216 / 226; 384, 49 l, 64 columns (245, 0.95) 77 / 88; 512, 65 l, 84 columns
-// (910, 0.656) 201 / 163, 112 columns (910, 0.875) 203 / 210, 448 columns 544 / 643.
+// product, and win where they are full and there are several for every CU: k_kin32 is taken where a
+// pass has at most one for each CU, up to K32_MAX_WG where they are not nearly full, and up to 4
+// for every CU where less than two thirds of them is output.  Both passes, us, tiles / k_kin32: N_r = 96,
+// 13 l, 100 columns (52 tiles) 37 / 20; 384, 49 l, 48 columns (245) 74 / 59, 64 columns 77 / 71; 400, 49 l,
+// 52 columns (294, 0.74 full) 92 / 78; 512, 65 l, 56 columns (455, 0.88) 128 / 118, 63 columns (0.98) 122 / 131,
+// 84 columns (910, 0.656) 201 / 163, 112 columns (910, 0.875) 203 / 210, 448 columns 544 / 643; 256, 33 l,
+// 1000 columns (0.79) 216 / 226.
 #define K32_MAX_C 40
-#define K32_MAX_WG 240
-#define K32_FILL 0.66
+#define K32_MAX_WG 460
 static bool kin32_better(const ggb_ctx *ctx) {
     const ggb_problem &p = ctx->p;
     if (ctx->C <= K32_MAX_C) return true;
     const double rows = (p.nk_max + TM - 1) / TM, cols = (2 * ctx->C + TN - 1) / TN;
     const double fill = (double)p.nk_max * 2 * ctx->C / (rows * TM * cols * TN), wg = rows * cols * p.n_l;
-    return wg < K32_MAX_WG || (fill < K32_FILL && wg <= 4 * 256);
+    return wg <= 256 || (wg <= K32_MAX_WG && fill < 0.95) || (wg <= 4 * 256 && fill < 0.66);
 }
 
 // Shape by the number of 16 x 16 output tiles of a pass.  Up to about four waves per SIMD one tile per
-// wave (neon, 32 columns, 4116 tiles: 19 / 18 us; two rows of tiles 21 / 18, four 24 / 21); with more, operand
-// traffic counts: 2 x 2 tiles for one pair of column tiles (krypton, 13 columns, 7372 tiles: 53 / 56
-// against 73 / 59), 4 x 1 for more columns (argon, 35 columns, 8775 tiles: 42 / 40 against 45 / 45).
+// wave (neon, 32 columns, 3724 tiles: 25 / 22 us; two rows of tiles 27 / 21, four 31 / 25); with more,
+// operand traffic counts: 2 x 2 tiles for one pair of column tiles (krypton, 13 columns, 7372 tiles:
+// 53 / 56 against 73 / 59), else rows of tiles for one column tile, as many as fit: a panel is 4 waves
+// of 1, 2 or 4 tiles, and its last one is partly empty.  Against 4 tiles, 2 cost 1.1 to 1.2 times as much
+// per tile and 1 up to half as much again, so argon N = 512 (28 row tiles of 32) takes 4 (84 columns 168 us, 2: 187, 1: 206)
+// and N = 300 (17 of 32, or of 24) takes 2 (140 columns 87 us, 4: 108, 1: 94).
 static void launch_kin32(ggb_ctx *ctx, int pass, const KinRef &ref, hipEvent_t e0, hipEvent_t e1) {
-    const int nct = (2 * ctx->C + 15) / 16;
+    const int nct = (2 * ctx->C + 15) / 16, rt = ((pass ? ctx->p.n_r : ctx->p.nk_max) + 15) / 16;
     const long tiles = (long)(ctx->p.nk_max / 16) * nct * ctx->p.n_l;
-    if (tiles <= 5000)
-        launch_kin32_t<1, 1>(ctx, pass, ref, e0, e1);
-    else if (nct <= 2)
-        launch_kin32_t<2, 2>(ctx, pass, ref, e0, e1);
-    else
+    if (tiles <= 4500) return launch_kin32_t<1, 1>(ctx, pass, ref, e0, e1);
+    if (nct <= 2) return launch_kin32_t<2, 2>(ctx, pass, ref, e0, e1);
+    // row tiles computed, with the cost of each
+    const double c4 = (rt + 15) / 16 * 16, c2 = 1.2 * ((rt + 7) / 8 * 8), c1 = 1.45 * ((rt + 3) / 4 * 4);
+    if (c4 <= c2 && c4 <= c1)
         launch_kin32_t<4, 1>(ctx, pass, ref, e0, e1);
+    else if (c2 <= c1)
+        launch_kin32_t<2, 1>(ctx, pass, ref, e0, e1);
+    else
+        launch_kin32_t<1, 1>(ctx, pass, ref, e0, e1);
 }
 
 static void launch_kinetic_mixed(ggb_ctx *ctx, int pass, bool fresh, hipEvent_t e0, hipEvent_t e1) {

@@ -147,3 +147,19 @@ def test_fp64_passes_larger_shapes(N, columns):
             got[variant] = prop.download_orbitals()
     assert np.array_equal(got["default"], got["narrow"])
     assert np.abs(got["default"] - ref).max() < 4 * N * 2.0 ** -53
+
+
+@pytest.mark.parametrize("lmax", [64, 95])
+def test_mixed_passes_panel_shapes(lmax):
+    """Small-tile passes of more than 4500 output tiles, with 1, 2 or 4 row tiles per wave by how
+    full the last panel is (N = 150: 6 row tiles of 16 eigenvalues and 10 of nodes; N = 270: 11 and 17),
+    against the large tiles of the same sums (more columns)."""
+    print("case: mixed kinetic passes, panel shapes, l_max", lmax, flush=True)
+    for N, few, many in ((150, 230, 512), (270, 60, 320)):
+        S = AtomSystem("He", N, 60.0, lmax, 0.05, ground_state="device", tables="device")
+        psi = _random_columns(S, many)
+        wide = _mixed(S, psi, many, "tiled16")
+        assert np.abs(wide - _kinetic(S, psi)).max() < 4 * (18 + N / 16) * 2.0 ** -24
+        for columns in (few, few - 7, 34):
+            got = _mixed(S, psi[:, :columns].copy(), columns, "tiled16")
+            assert np.array_equal(got, wide[:, :columns]), (N, columns)
