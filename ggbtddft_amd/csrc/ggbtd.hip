@@ -56,6 +56,7 @@ typedef double d4_t __attribute__((ext_vector_type(4)));
 #ifndef ANG_NT_MIXED
 #define ANG_NT_MIXED 2  // angular column tiles per work-group in the mixed form (1, 2 or 4)
 #endif
+#define ANG_NT_WAVES 4600  // waves (of one-tile work-groups) of a context from which it takes them
 #define RHO_MIN 1e-40 // v_xc = 0 at or below this density
 #define KIN_NARROW_MAX_C 8  // up to 8 complex columns: one 16-wide MFMA column tile
 #define TIMING_STRIDE 16    // timing mode 1 samples every 16th step
@@ -3653,10 +3654,15 @@ static ang_geom ang_geometry(const ggb_problem *p) {
     // mixed form: the folded sums S/D (FP32) fit in the FP64 l-space tile's
     // space whenever hq <= N_l + 6; the kernel parks the old tile values it
     // needs in registers meanwhile (one work-group less of LDS per CU)
-    // mixed form (many columns): two column tiles per work-group, each table
-    // value then feeds two products and the per-work-group work is shared by
-    // twice the radial nodes
-    a.nt = p->precision ? ANG_NT_MIXED : 1;
+    // mixed form: two column tiles per work-group, each table value then feeds two products and the
+    // per-work-group work is shared by twice the radial nodes; one in contexts whose waves do not
+    // fill the device, where a work-group of one tile is done sooner (same sums for every state
+    // value).  Both phases, us, one tile / two: helium N = 256 20 / 25 (96 waves), neon N = 384 23 / 28
+    // (768), argon N = 512 30 / 34 (2240), neon N = 384, 4 instances 30 / 35 (3072), argon, 2 instances
+    // 42.0 / 42.9 (4480); krypton N = 400, 2 instances 42 / 41 (5200), neon, 8 instances 44 / 42
+    // (6144), argon, 3 instances 56 / 52 (6720), 32 instances 376 / 327.
+    const double ang_waves = (double)((p->n_r + RT - 1) / RT) * p->n_orb * p->n_inst * a.waves;
+    a.nt = p->precision && ang_waves > ANG_NT_WAVES ? ANG_NT_MIXED : 1;
     static_assert(ANG_NT_MIXED == 1 || ANG_NT_MIXED == 2 || ANG_NT_MIXED == 4, "column tiles: 1, 2 or 4");
     a.ntiles = (p->n_r + RT * a.nt - 1) / (RT * a.nt);
     const size_t xbytes = (size_t)(p->n_l + 6) * 16 * a.nt * sizeof(double);

@@ -81,3 +81,28 @@ def test_wave_tiles_idle_slots_and_graph():
     assert np.array_equal(got_g, got)
     for key in obs:
         assert np.array_equal(obs_g[key], obs[key]), key
+
+
+@pytest.mark.parametrize("N, lmax, n_theta", [(75, 40, 81), (72, 40, 82), (77, 64, 129), (50, 12, 25)])
+def test_mixed_one_and_two_tiles_per_workgroup(N, lmax, n_theta):
+    """Mixed form: a context of few waves takes one angular tile per work-group, a larger one two.  The
+    state and potential are the same bit for bit; observables are the same terms added in another
+    order: 2 N eps of their weights each way at most."""
+    from ggbtddft_amd.engine import Propagator
+    print("case: mixed angular tiles, N", N, "l_max", lmax, flush=True)
+    S = AtomSystem("Ar", N, 30.0, lmax, 0.05, n_theta=n_theta, ground_state="device", tables="device")
+    E = 0.2 * np.random.default_rng(N).standard_normal(STEPS + 1)
+
+    def run(n):
+        with Propagator(S, n_inst=n, precision=1) as prop:
+            prop.set_kinetic_variant("narrow")
+            prop.set_field(np.tile(E, (n, 1)))
+            obs = prop.run(0, STEPS)
+            return obs, prop.download_orbitals(), prop.download_potential()
+    few, many = run(1), run(50)
+    assert np.array_equal(few[1], many[1][:, :S.n_orb])
+    assert np.array_equal(few[2][0], many[2][0])
+    scale = {"dip": 30.0, "acc": 1 / S.grid.r.min() ** 2, "norm": 1.0}
+    for key, w in scale.items():
+        d = np.abs(few[0][key].reshape(STEPS, 1, -1) - many[0][key].reshape(STEPS, 50, -1)).max()
+        assert d <= 4 * N * 2.0 ** -53 * w, (key, d)
