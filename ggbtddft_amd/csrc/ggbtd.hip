@@ -3050,9 +3050,18 @@ __global__ __launch_bounds__(WG) void k_tile_gemm(GemmOperands g, Epi epi) {
 #ifndef TGW_G
 #define TGW_G 3   // tiles per reduction round through LDS
 #endif
-#ifndef TGW_MIN_INST
-#define TGW_MIN_INST 8  // instances from which the potential products use the panel form
-#endif
+// 16 x 16 tiles of a product from which it takes the panel form.  Moments (with the density kernel),
+// us, tiles / panels: argon N = 512, 3 instances (864 tiles) 17.4 / 16.8, 7 (2016) 27.4 / 25.3, 32 72 / 60;
+// neon N = 384, 4 instances (672) 13.8 / 14.7, 8 (1344) 18.5 / 18.8, 12 (2016) 23.5 / 22.7.  The potential,
+// whose last group of tiles may hold only one: argon (9 theta tiles), 7 instances 14.1 / 14.8, 10 (2880)
+// 16.8 / 16.6, 32 38.5 / 35.4; krypton (13), 6 instances (3744) 26.1 / 28.6, 8 (4992) 32.4 / 31.7; neon (7), 45
+// instances (7560) 31.2 / 34.2, so not where more than a sixth of the groups' tiles is empty.
+#define TGW_MIN_MOM 1200
+#define TGW_MIN_DV 2300
+static bool dv_panels(double row_tiles, int theta_tiles) {
+    const double waste = (double)((theta_tiles + TGW_T - 1) / TGW_T * TGW_T) / theta_tiles;
+    return waste < 1.2 && row_tiles * theta_tiles >= TGW_MIN_DV * (waste > 1.1 ? 2 : 1);
+}
 template <class Epi, bool WIDE_M>
 __global__ __launch_bounds__(WG) void k_tile_gemm_wide(GemmOperands g, Epi epi) {
     __shared__ double red[4][TGW_G][64][4];
@@ -4264,7 +4273,7 @@ static int launch_potential(ggb_ctx *ctx, const ObsArgs *ob = nullptr, MarkK mk 
             gq.N = N;
             gq.K = Nth;
             QmomEpi eq{ctx->q, N, nh};
-            if (p.n_inst >= TGW_MIN_INST) {
+            if ((double)nmom * p.n_inst >= TGW_MIN_MOM) {
                 gq.A = ctx->PL;  // the same table as [j][L]: the 16 lanes of a K row read 16 consecutive L
                 gq.sam = 1;
                 gq.sak = nh;
@@ -4296,8 +4305,8 @@ static int launch_potential(ggb_ctx *ctx, const ObsArgs *ob = nullptr, MarkK mk 
     gv.N = Nth;
     gv.K = p.interacting ? nh : 0;
     DvEpi ev{ctx->vxc, ctx->v_gs, ctx->mask, ctx->dv, ctx->phase, N, Nth, p.interacting, p.precision, p.dt};
-    if (p.n_inst >= TGW_MIN_INST) {
-        const int ntj = (Nth + 15) / 16;
+    const int ntj = (Nth + 15) / 16;
+    if (dv_panels((double)((N + 15) / 16) * p.n_inst, ntj)) {
         k_tile_gemm_wide<DvEpi, false><<<dim3((N + 15) / 16, (ntj + TGW_T - 1) / TGW_T, p.n_inst), WG, 0, st>>>(gv, ev);
     } else {
         k_tile_gemm<<<dim3((Nth + 15) / 16, (N + 15) / 16, p.n_inst), WG, 0, st>>>(gv, ev);

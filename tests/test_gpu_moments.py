@@ -77,3 +77,20 @@ def test_channel_dipoles_with_the_density(atom, N, lmax, n):
             tol = 8 * N * 2.0 ** -53 * (np.abs(psi[l, :, k]) * size).sum(axis=1)
             assert (np.abs(got[:, k, l] - ref)[active] <= tol[active]).all(), (k, l)
             assert not got[~active, k, l].any()
+
+
+# panel and 16 x 16 forms of the two potential products, each against the other: instances below and
+# beyond the tile counts at which either product changes (N_theta with 9, 7 and 13 tiles of 16)
+@pytest.mark.parametrize("N, lmax, n_theta, counts", [(203, 64, 129, (2, 9, 11, 30)), (203, 48, 97, (5, 14, 30)),
+                                                      (100, 96, 193, (1, 9, 30, 60))])
+def test_potential_products_by_tiles(N, lmax, n_theta, counts):
+    print("case: potential products, N", N, "l_max", lmax, "N_theta", n_theta, flush=True)
+    S = AtomSystem("Ne", N, 40.0, lmax, 0.05, n_theta=n_theta, ground_state="device", tables="device")
+    psi = S.psi0.copy()
+    psi[1:4] += 0.1 * np.random.default_rng(N).standard_normal(psi[1:4].shape) * np.exp(-S.grid.r)
+    for k in range(S.n_orb):
+        psi[:S.m[k], k] = 0.0
+    ref = _run(S, psi, counts[0], 0)[0]
+    for n in counts[1:]:
+        dv = _run(S, psi, n, 0)
+        assert all(np.array_equal(v, ref) for v in dv), n
