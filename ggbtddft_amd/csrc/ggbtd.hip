@@ -506,7 +506,7 @@ __global__ __launch_bounds__(KIN_NARROW_WG) void k_kin_bwd(const float *__restri
 //           of 16 (k = eigen index, m = radial node), B = Y, D = psi.
 // A work-group takes a panel of 16 TA rows m (as TA tiles with interleaved rows:
 // row 4 r + kr of tile t is m0 + TA (4 r + kr) + t) by TB tiles of 16 real columns
-// (8 complex ones); its K64_NW waves take equal shares of k and add their
+// (8 complex ones); its NW waves take equal shares of k and add their
 // partial tiles in fixed order through LDS.  No tile is staged: every wave loads
 // its operands straight into registers, one block of 8 k ahead of the products
 // on the block before.
@@ -522,8 +522,6 @@ __global__ __launch_bounds__(KIN_NARROW_WG) void k_kin_bwd(const float *__restri
 // 28 columns 44 / 45 us (94 / 124), 224 columns 237 / 234 us (369 / 349, 53 TFLOP/s);
 // krypton (N = 768, 97 l, 13 columns) 87 / 84 us (258 / 293).
 // ---------------------------------------------------------------------------
-#define K64_NW 4
-#define K64_WG (64 * K64_NW)
 typedef double d2_t __attribute__((ext_vector_type(2)));
 struct Kin64Args {
     const double *A;       // PASS 0: Q [l][N][nk_max], PASS 1: QT [l][nk_max][np]
@@ -535,10 +533,9 @@ struct Kin64Args {
     int N, nk_max, np, C, n_orb;
 };
 
-template <int PASS, int TA, int TB>
+template <int PASS, int TA, int TB, int NW>
 static __device__ __forceinline__ void kin64_tiles(const Kin64Args &g, int l, int nk, int m0, int n0,
                                                    double (*red)[TA][64][4]) {
-    constexpr int NW = K64_NW;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int kr = lane >> 4, lc = lane & 15, p = lc & 1;
     const int C = g.C;
@@ -672,9 +669,9 @@ static __device__ __forceinline__ void kin64_tiles(const Kin64Args &g, int l, in
     }
 }
 
-template <int PASS, int TA, int TB>
-__global__ __launch_bounds__(K64_WG) void k_kin64(Kin64Args g) {
-    __shared__ double red[K64_NW][TA][64][4];
+template <int PASS, int TA, int TB, int NW>
+__global__ __launch_bounds__(64 * NW) void k_kin64(Kin64Args g) {
+    __shared__ double red[NW][TA][64][4];
     const tile3 tb = xcd_tile();  // (row panel, column group, l): panels of one l share B
     const int l = tb.z;
     const int nk = g.nkeep[l];
@@ -683,9 +680,9 @@ __global__ __launch_bounds__(K64_WG) void k_kin64(Kin64Args g) {
     const int n0 = tb.y * 16 * TB;
     if (!kin_cols_active(g.active, n0, 16 * TB, g.C, g.n_orb)) return;  // idle instances only
     if (TB > 1 && n0 + 16 >= 2 * g.C)  // last group with one tile left
-        kin64_tiles<PASS, TA, 1>(g, l, nk, m0, n0, red);
+        kin64_tiles<PASS, TA, 1, NW>(g, l, nk, m0, n0, red);
     else
-        kin64_tiles<PASS, TA, TB>(g, l, nk, m0, n0, red);
+        kin64_tiles<PASS, TA, TB, NW>(g, l, nk, m0, n0, red);
 }
 
 // QT[l][a][i] = Q[l][i][a], rows of np >= N values (zero from N on), through LDS
@@ -4342,7 +4339,7 @@ static void kin_launch(void (*k)(KArgs...), dim3 g, int threads, hipStream_t st,
         k<<<g, threads, 0, st>>>(args...);
 }
 
-template <int TA, int TB>
+template <int TA, int TB, int NW = 4>
 static void launch_kin64_t(ggb_ctx *ctx, int pass, hipEvent_t e0, hipEvent_t e1) {
     const ggb_problem &p = ctx->p;
     Kin64Args g;
@@ -4360,9 +4357,9 @@ static void launch_kin64_t(ggb_ctx *ctx, int pass, hipEvent_t e0, hipEvent_t e1)
     const int rows = pass ? p.n_r : p.nk_max;
     const dim3 grid((rows + 16 * TA - 1) / (16 * TA), (2 * g.C + 16 * TB - 1) / (16 * TB), p.n_l);
     if (pass)
-        kin_launch(k_kin64<1, TA, TB>, grid, K64_WG, ctx->stream, e0, e1, g);
+        kin_launch(k_kin64<1, TA, TB, NW>, grid, 64 * NW, ctx->stream, e0, e1, g);
     else
-        kin_launch(k_kin64<0, TA, TB>, grid, K64_WG, ctx->stream, e0, e1, g);
+        kin_launch(k_kin64<0, TA, TB, NW>, grid, 64 * NW, ctx->stream, e0, e1, g);
 }
 
 // Shape of the FP64 passes by the 16 x 16 output tiles of a pass.  NARROW, one column tile, and up to
@@ -4375,6 +4372,10 @@ static void launch_kin64_t(ggb_ctx *ctx, int pass, hipEvent_t e0, hipEvent_t e1)
 // 205 / 178 / 169; krypton N = 768, 97 l, 13 columns (7566, 391 MB of table) 213 / 202 / 177.  (32 x 2
 // is never the fastest by more than 2 %.)  Every element is formed by the same products in the same
 // order in all of them.
+//   Pass 0 on one column tile and long rows: k split over eight waves instead of four, with more of the
+// table's rows in flight (argon N = 512, 7 columns 23.8 -> 23.2 us, neon N = 768 67.0 -> 65.3; shorter rows
+// lose: N = 384 12.3 -> 12.7, N = 300 10.5 -> 11.1).
+#define K64_EIGHT_N 448
 #define K64_TILES_32 2000
 #define K64_TILES_64 7200
 #define K64_TABLE_BYTES 200e6
@@ -4382,7 +4383,9 @@ static void launch_kin64(ggb_ctx *ctx, int pass, hipEvent_t e0, hipEvent_t e1) {
     const ggb_problem &p = ctx->p;
     const int nct = (2 * ctx->C + 15) / 16, rows = pass ? p.n_r : p.nk_max;
     const double tiles = (double)((rows + 15) / 16) * nct * p.n_l;
-    if (ctx->kin_variant == GGB_KIN_NARROW || nct == 1 || tiles < K64_TILES_32)
+    if (pass == 0 && nct == 1 && p.n_r >= K64_EIGHT_N)
+        launch_kin64_t<2, 1, 8>(ctx, pass, e0, e1);
+    else if (ctx->kin_variant == GGB_KIN_NARROW || nct == 1 || tiles < K64_TILES_32)
         launch_kin64_t<2, 1>(ctx, pass, e0, e1);
     else if (tiles < K64_TILES_64 && 8.0 * p.n_l * p.n_r * p.nk_max < K64_TABLE_BYTES)
         launch_kin64_t<4, 1>(ctx, pass, e0, e1);

@@ -222,7 +222,7 @@ const char *ggb_group_last_error(const ggb_group *g);
 void ggb_group_destroy(ggb_group *g);
 
 /* Kinetic-pass kernel variants (tile shapes).  In FP64 every variant forms the
- * same sums in the same order: NARROW takes 16 real columns (8 orbital columns)
+ * same sums in the same order (up to 8 orbital columns all are one): NARROW takes 16 real columns (8 orbital columns)
  * per work-group, DEFAULT and TILED16 16 or 32 by the size of the pass.  In the mixed
  * form DEFAULT is NARROW up to 8 orbital columns, else TILED16.  NARROW: 16x16
  * tiles with the contraction split over the work-group's waves; TILED16 /

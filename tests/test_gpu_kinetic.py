@@ -163,3 +163,19 @@ def test_mixed_passes_panel_shapes(lmax):
         for columns in (few, few - 7, 34):
             got = _mixed(S, psi[:, :columns].copy(), columns, "tiled16")
             assert np.array_equal(got, wide[:, :columns]), (N, columns)
+
+
+@pytest.mark.parametrize("N", [448, 453])
+@pytest.mark.parametrize("columns", [1, 8])
+def test_fp64_long_rows(N, columns):
+    """One column tile on 448 rows and more: eight waves share the contraction of pass 0."""
+    print("case: FP64 kinetic passes, long rows, N", N, "columns", columns, flush=True)
+    from ggbtddft_amd.engine import Propagator
+    S = AtomSystem("He", N, 100.0, 4, 0.05, ground_state="device", tables="device")
+    psi = _random_columns(S, columns)
+    with Propagator(S, n_inst=columns) as prop:
+        prop.set_field(np.zeros(1))
+        prop.upload_orbitals(psi)
+        prop.substep(1)
+        got = prop.download_orbitals()
+    assert np.abs(got - _kinetic(S, psi)).max() < 4 * N * 2.0 ** -53
