@@ -3983,6 +3983,11 @@ extern "C" int ggb_upload_static(ggb_ctx *ctx, const ggb_static *s) {
     drop_graph(ctx);
     const size_t N = p.n_r, Nl = p.n_l, Nth = p.n_theta;
     hipStream_t st = ctx->stream;
+    // a refusal after copies from the caller's tables have been queued waits for them
+    auto refuse = [&](const char *msg) {
+        (void)hipStreamSynchronize(st);
+        return fail(ctx, GGB_E_ARG, msg);
+    };
     HIPCHK(ctx, hipMemcpyAsync(ctx->r, s->r, N * 8, hipMemcpyHostToDevice, st));
     {
         // the Hartree scans' ratio powers as exp(n log(r_{a-1}/r_a)) (no overflow
@@ -4052,7 +4057,7 @@ extern "C" int ggb_upload_static(ggb_ctx *ctx, const ggb_static *s) {
         for (size_t j = 0; j < Nth; ++j)
             if (std::fabs(s->chi[j] + s->chi[Nth - 1 - j]) > 1e-13 ||
                 std::fabs(s->omega[j] - s->omega[Nth - 1 - j]) > 1e-13 * std::fabs(s->omega[j]))
-                return fail(ctx, GGB_E_ARG, "ggb_upload_static: theta grid must be symmetric (Gauss-Legendre)");
+                return refuse("ggb_upload_static: theta grid must be symmetric (Gauss-Legendre)");
         for (int mm = 0; mm < p.n_m; ++mm)
             for (size_t j = 0; j < Nth; ++j)
                 for (size_t l = 0; l < Nl; ++l) {
@@ -4060,9 +4065,8 @@ extern "C" int ggb_upload_static(ggb_ctx *ctx, const ggb_static *s) {
                     const double a = s->B[((size_t)mm * Nth + j) * Nl + l];
                     const double b = s->B[((size_t)mm * Nth + Nth - 1 - j) * Nl + l];
                     if (std::fabs(a - sg * b) > tol || ((int)l < mm && a != 0.0))
-                        return fail(ctx, GGB_E_ARG,
-                                    "ggb_upload_static: B must satisfy B[m][N_theta-1-j][l] = (-1)^(l-m) B[m][j][l]"
-                                    " and vanish for l < m");
+                        return refuse("ggb_upload_static: B must satisfy B[m][N_theta-1-j][l] = (-1)^(l-m) B[m][j][l]"
+                                      " and vanish for l < m");
                 }
         std::vector<double> bh((size_t)p.n_m * ag.nblk, 0.0);
         for (int mm = 0; mm < p.n_m; ++mm) {
@@ -4096,7 +4100,7 @@ extern "C" int ggb_upload_static(ggb_ctx *ctx, const ggb_static *s) {
     if (p.precision && s->phi && s->l0 && s->eps) {
         for (int k = 0; k < p.n_orb; ++k)
             if (s->l0[k] < s->m[k] || s->l0[k] >= p.n_l)
-                return fail(ctx, GGB_E_ARG, "ggb_upload_static: reference l0 out of range");
+                return refuse("ggb_upload_static: reference l0 out of range");
         HIPCHK(ctx, hipMemcpy(ctx->phi_ref, s->phi, (size_t)p.n_orb * N * 8, hipMemcpyHostToDevice));
         HIPCHK(ctx, hipMemcpy(ctx->eps, s->eps, (size_t)p.n_orb * 8, hipMemcpyHostToDevice));
         HIPCHK(ctx, hipMemcpy(ctx->l0, s->l0, (size_t)p.n_orb * 4, hipMemcpyHostToDevice));
