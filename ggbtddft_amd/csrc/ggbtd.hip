@@ -874,14 +874,19 @@ __global__ __launch_bounds__(WG) void k_kin_fwd_tiled(const float *__restrict__ 
 //     (k, k+1) x (re, im); slot q = k/2 sits at position (q + c) & 7.
 // Rows a >= nk_max and columns beyond C load a valid in-range element instead
 // of zeros; they only reach outputs that are not stored.  Needs N % 16 == 0.
+// The bound of four waves per SIMD (here, in k_kin_bwd_dma and in k_kin32)
+// keeps the accumulators out of the accumulation registers, from which every
+// chunk's results would be copied back.  Both passes, argon at N = 512: 64
+// instances 573 -> 551 us, 12 instances 170 -> 165.  k_kin32 there at 2 and 3
+// instances 57.4 -> 56.1 and 70.0 -> 68.2; equal on the smallest contexts.
 typedef __attribute__((address_space(3))) void lds_void_t;
 #define KD_WAIT(n) __builtin_amdgcn_s_waitcnt(0xF70 | (n))  // vmcnt(n), other counters untouched
-__global__ __launch_bounds__(WG) void k_kin_fwd_dma(const float *__restrict__ Q,
-                                                    const double2 *__restrict__ kph,
-                                                    const int32_t *__restrict__ nkeep,
-                                                    const float2 *__restrict__ psi32, KinRef ref,
-                                                    float *__restrict__ Y, int N, int nk_max, int C,
-                                                    int n_orb) {
+__global__ __launch_bounds__(WG, 4) void k_kin_fwd_dma(const float *__restrict__ Q,
+                                                       const double2 *__restrict__ kph,
+                                                       const int32_t *__restrict__ nkeep,
+                                                       const float2 *__restrict__ psi32, KinRef ref,
+                                                       float *__restrict__ Y, int N, int nk_max, int C,
+                                                       int n_orb) {
     typedef mfma_t<float>::v4 v4;
     // three buffers of (A chunk: 1024 floats, B chunk: 2048 floats)
     __shared__ __align__(16) float lds[3 * 3072];
@@ -1105,11 +1110,11 @@ __global__ __launch_bounds__(WG) void k_kin_bwd_tiled(const float *__restrict__ 
 // 16 different 64-byte rows: a 2-way bank conflict that no rotation within a
 // row removes.  Rows i >= N and columns beyond C load row/column 0 and are
 // not stored.
-__global__ __launch_bounds__(WG) void k_kin_bwd_dma(const float *__restrict__ Q,
-                                                    const int32_t *__restrict__ nkeep,
-                                                    const float *__restrict__ Y, KinRef ref,
-                                                    double *__restrict__ psi, int N, int nk_max,
-                                                    int C, int n_orb) {
+__global__ __launch_bounds__(WG, 4) void k_kin_bwd_dma(const float *__restrict__ Q,
+                                                       const int32_t *__restrict__ nkeep,
+                                                       const float *__restrict__ Y, KinRef ref,
+                                                       double *__restrict__ psi, int N, int nk_max,
+                                                       int C, int n_orb) {
     typedef mfma_t<float>::v4 v4;
     __shared__ __align__(16) float lds[3 * 3072];  // three buffers of (A: 64 x 16, B: 128 x 16)
     const tile3 tb = xcd_tile();  // (radial tile, column tile, l)
@@ -1282,7 +1287,7 @@ static __device__ __forceinline__ void rows_transpose(float (&x)[4]) {
 }
 
 template <int PASS, int TA, int TB>
-__global__ __launch_bounds__(WG) void k_kin32(Kin32Args g) {
+__global__ __launch_bounds__(WG, 4) void k_kin32(Kin32Args g) {
     typedef float vta __attribute__((ext_vector_type(TA)));
     const tile3 tb = xcd_tile();  // (group of 4 row panels, column group, l): they share the columns
     const int l = tb.z;
@@ -3059,8 +3064,14 @@ static bool dv_panels(double row_tiles, int theta_tiles) {
     const double waste = (double)((theta_tiles + TGW_T - 1) / TGW_T * TGW_T) / theta_tiles;
     return waste < 1.2 && row_tiles * theta_tiles >= TGW_MIN_DV * (waste > 1.1 ? 2 : 1);
 }
+
+// The bound of five waves per SIMD keeps the accumulators in the ordinary
+// registers.  Without it they go to the accumulation registers, and each
+// chunk's results are copied back to be added in FP64.  64 argon instances:
+// density product 107.4 -> 104.9 us, potential product 62.8 -> 58.0.  A bound
+// of six spills (potential 70).
 template <class Epi, bool WIDE_M>
-__global__ __launch_bounds__(WG) void k_tile_gemm_wide(GemmOperands g, Epi epi) {
+__global__ __launch_bounds__(WG, 5) void k_tile_gemm_wide(GemmOperands g, Epi epi) {
     __shared__ double red[4][TGW_G][64][4];
     const int z = blockIdx.z;
     if (g.active && !g.active[z]) return;  // block-uniform
