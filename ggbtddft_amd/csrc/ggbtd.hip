@@ -876,9 +876,10 @@ __global__ __launch_bounds__(WG) void k_kin_fwd_tiled(const float *__restrict__ 
 // of zeros; they only reach outputs that are not stored.  Needs N % 16 == 0.
 // The bound of four waves per SIMD (here, in k_kin_bwd_dma and in k_kin32)
 // keeps the accumulators out of the accumulation registers, from which every
-// chunk's results would be copied back.  Both passes, argon at N = 512: 64
-// instances 573 -> 551 us, 12 instances 170 -> 165.  k_kin32 there at 2 and 3
-// instances 57.4 -> 56.1 and 70.0 -> 68.2; equal on the smallest contexts.
+// chunk's results would be copied back.  Both passes, argon at N = 512, 64
+// instances: 554 -> 533 us (12 instances 159 on both sides).  k_kin32 there at
+// 2 and 3 instances 57.4 -> 56.1 and 70.0 -> 68.2; equal on the smallest
+// contexts.
 typedef __attribute__((address_space(3))) void lds_void_t;
 #define KD_WAIT(n) __builtin_amdgcn_s_waitcnt(0xF70 | (n))  // vmcnt(n), other counters untouched
 __global__ __launch_bounds__(WG, 4) void k_kin_fwd_dma(const float *__restrict__ Q,
@@ -1504,13 +1505,17 @@ static __device__ __forceinline__ void kin_split_step(const float (*Ah)[TMP], co
     }
 }
 
-__global__ __launch_bounds__(WG) void k_kin_fwd_split(const float *__restrict__ Qh,
-                                                      const float *__restrict__ Ql,
-                                                      const double2 *__restrict__ kph,
-                                                      const int32_t *__restrict__ nkeep,
-                                                      const double *__restrict__ psi, KinRef ref,
-                                                      float *__restrict__ Yh, float *__restrict__ Yl,
-                                                      int N, int nk_max, int C, int n_orb) {
+// The bound of two waves per SIMD (what the LDS allows; here and in
+// k_kin_bwd_split) keeps the accumulators out of the accumulation registers:
+// argon at N = 512, 64 instances, 1081 + 1428 -> 1047 + 1422 us; 8 instances
+// 184 + 281 -> 181 + 279.
+__global__ __launch_bounds__(WG, 2) void k_kin_fwd_split(const float *__restrict__ Qh,
+                                                         const float *__restrict__ Ql,
+                                                         const double2 *__restrict__ kph,
+                                                         const int32_t *__restrict__ nkeep,
+                                                         const double *__restrict__ psi, KinRef ref,
+                                                         float *__restrict__ Yh, float *__restrict__ Yl,
+                                                         int N, int nk_max, int C, int n_orb) {
     constexpr int AV = SPK * TM / WG;  // A values per thread (consecutive a)
     constexpr int BV = SPK * 64 / WG;  // complex B values per thread (consecutive i)
     __shared__ float Ash[2][SPK][TMP], Asl[2][SPK][TMP];  // [k = i][m = a]
@@ -1631,13 +1636,13 @@ __global__ __launch_bounds__(WG) void k_kin_fwd_split(const float *__restrict__ 
     }
 }
 
-__global__ __launch_bounds__(WG) void k_kin_bwd_split(const float *__restrict__ Qh,
-                                                      const float *__restrict__ Ql,
-                                                      const int32_t *__restrict__ nkeep,
-                                                      const float *__restrict__ Yh,
-                                                      const float *__restrict__ Yl, KinRef ref,
-                                                      double *__restrict__ psi, int N, int nk_max,
-                                                      int C, int n_orb) {
+__global__ __launch_bounds__(WG, 2) void k_kin_bwd_split(const float *__restrict__ Qh,
+                                                         const float *__restrict__ Ql,
+                                                         const int32_t *__restrict__ nkeep,
+                                                         const float *__restrict__ Yh,
+                                                         const float *__restrict__ Yl, KinRef ref,
+                                                         double *__restrict__ psi, int N, int nk_max,
+                                                         int C, int n_orb) {
     constexpr int AV = SPK * TM / WG;  // A values per thread (consecutive a of one row i)
     constexpr int BV = SPK * TN / WG;  // B values per thread (consecutive a of one column)
     __shared__ float Ash[2][SPK][TMP], Asl[2][SPK][TMP];  // [k = a][m = i]
