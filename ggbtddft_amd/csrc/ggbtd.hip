@@ -5721,6 +5721,7 @@ struct GsArgs {
     int32_t *ticket;     // work-groups of the sweep started so far
     int team, rows;      // work-groups per group, rows of a product of each
     int redo;            // only the groups with res[1 + g] < 0, whose team gave up waiting
+    int expire;          // phase of a team whose wait counts as run out (-1: none; ggb_debug_ground_state)
     int N, n_shell, n_group, sweeps, interacting, first, final_;
     double Z, mix, gamma;
 };
@@ -5956,6 +5957,7 @@ static __device__ __forceinline__ void gs_matvec(const GsArgs &a, GsTeam &tm, co
     // the whole vector, as its rows arrive
     const long long empty = __double_as_longlong(gs_empty());
     const long long t0 = wall_clock64();
+    if (tm.phase == a.expire) tm.ok = false;
     for (int i = t; i < N; i += GS_WG) {
         double v = __hip_atomic_load(slot + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         while (__double_as_longlong(v) == empty && tm.ok) {
@@ -6026,12 +6028,14 @@ static __device__ void gs_deflate(const GsArgs &a, const double *u, int j, doubl
 // over the group's shells with the potential a.v; eps and the group's
 // largest eps change into a.res[1 + g].  Every work-group keeps all vectors and
 // does the same vector work in the same order, so all hold the same bits; the orbitals
-// are kept in LDS until the last sweep, when the team's first work-group stores them.
+// and their energies are kept in LDS until the last shell of the last sweep is done, when the
+// team's first work-group stores them all: a team that gives up leaves a.u and a.eps as they were.
 template <bool TEAM, bool LDSU>
 __global__ __launch_bounds__(GS_WG) void k_gs_sweep(GsArgs a) {
     extern __shared__ double gsm[];
     __shared__ double red[GS_WG / 64];
     __shared__ double scr[GS_WG];
+    __shared__ double es[GS_MAX_K];  // orbital energies after the last sweep
     __shared__ int ticket;
     if (TEAM) {
         if (threadIdx.x == 0) ticket = atomicAdd(a.ticket, 1);
@@ -6103,22 +6107,23 @@ __global__ __launch_bounds__(GS_WG) void k_gs_sweep(GsArgs a) {
                 // unchanged) and the largest change (+inf at the first iteration)
                 const double e = gs_dot(x, hx, N, red);
                 dmax = fmax(dmax, fabs(e - a.eps[sh[j]]));
-                __syncthreads();
-                if (tm.me == 0 && tm.ok) {
-                    if (threadIdx.x == 0) a.eps[sh[j]] = e;
-                    for (int i = threadIdx.x; i < N; i += blockDim.x) a.u[(size_t)sh[j] * N + i] = us[i];
-                }
+                if (threadIdx.x == 0) es[j] = e;
             }
         }
     }
-    if (tm.me == 0 && threadIdx.x == 0) a.res[1 + g] = tm.ok ? dmax : -1.0;
+    if (tm.me != 0) return;
+    if (tm.ok)
+        for (int j = 0; j < k; ++j) {
+            if (threadIdx.x == 0) a.eps[sh[j]] = es[j];
+            for (int i = threadIdx.x; i < N; i += blockDim.x) a.u[(size_t)sh[j] * N + i] = u[(size_t)j * N + i];
+        }
+    if (threadIdx.x == 0) a.res[1 + g] = tm.ok ? dmax : -1.0;
 }
 
-extern "C" int ggb_ground_state(const ggb_gs_problem *p, const int32_t *shell_l, const double *occ,
-                                const double *r, const double *wr, const double *T,
-                                const double *Q0, const double *lam0, double *u, double *eps,
-                                double *v_gs, double *rho_u, int32_t *iterations,
-                                int32_t *converged) {
+static int ground_state(const ggb_gs_problem *p, const int32_t *shell_l, const double *occ,
+                        const double *r, const double *wr, const double *T, const double *Q0,
+                        const double *lam0, double *u, double *eps, double *v_gs, double *rho_u,
+                        int32_t *iterations, int32_t *converged, int expire) {
     auto bad = [](const char *msg) {
         g_create_err = std::string("ggb_ground_state: ") + msg;
         return GGB_E_ARG;
@@ -6225,7 +6230,7 @@ extern "C" int ggb_ground_state(const ggb_gs_problem *p, const int32_t *shell_l,
         a.N = N, a.n_shell = ns, a.n_group = G, a.sweeps = p->sweeps, a.interacting = p->interacting ? 1 : 0;
         a.Z = p->Z, a.mix = p->mix, a.gamma = p->gamma;
         a.final_ = 0;
-        a.ex = dex, a.priv = dpriv, a.ticket = dticket, a.team = team, a.rows = rows;
+        a.ex = dex, a.priv = dpriv, a.ticket = dticket, a.team = team, a.rows = rows, a.expire = expire;
         std::vector<double> res(1 + G);
         for (it = 1; it <= p->max_iter; ++it) {
             a.first = it == 1;
@@ -6283,4 +6288,21 @@ extern "C" int ggb_ground_state(const ggb_gs_problem *p, const int32_t *shell_l,
     *iterations = it;
     *converged = conv ? 1 : 0;
     return rc;
+}
+
+extern "C" int ggb_ground_state(const ggb_gs_problem *p, const int32_t *shell_l, const double *occ,
+                                const double *r, const double *wr, const double *T,
+                                const double *Q0, const double *lam0, double *u, double *eps,
+                                double *v_gs, double *rho_u, int32_t *iterations,
+                                int32_t *converged) {
+    return ground_state(p, shell_l, occ, r, wr, T, Q0, lam0, u, eps, v_gs, rho_u, iterations, converged, -1);
+}
+
+extern "C" int ggb_debug_ground_state(const ggb_gs_problem *p, const int32_t *shell_l, const double *occ,
+                                      const double *r, const double *wr, const double *T,
+                                      const double *Q0, const double *lam0, double *u, double *eps,
+                                      double *v_gs, double *rho_u, int32_t *iterations,
+                                      int32_t *converged, int32_t expire) {
+    return ground_state(p, shell_l, occ, r, wr, T, Q0, lam0, u, eps, v_gs, rho_u, iterations, converged,
+                        std::max(expire, -1));
 }

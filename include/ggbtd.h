@@ -338,6 +338,17 @@ int ggb_ground_state(const ggb_gs_problem *p, const int32_t *shell_l, const doub
                      const double *lam0, double *u, double *eps, double *v_gs, double *rho_u,
                      int32_t *iterations, int32_t *converged);
 
+/* ggb_ground_state with every wait of phase `expire` (counted from 0 in each
+ * iteration; four phases a shell and sweep) among the work-groups that share a
+ * group of shells taken as run out, in every iteration: the groups whose sweeps
+ * have such a phase are done again from the same start by one work-group each,
+ * and the results are the same bit for bit.  -1: no such phase.  For checks;
+ * grids below 144 nodes have no waits. */
+int ggb_debug_ground_state(const ggb_gs_problem *p, const int32_t *shell_l, const double *occ,
+                           const double *r, const double *wr, const double *T, const double *Q0,
+                           const double *lam0, double *u, double *eps, double *v_gs, double *rho_u,
+                           int32_t *iterations, int32_t *converged, int32_t expire);
+
 /* Kinetic propagator tables on the device.  For l = 0..n_l-1 the radial
  * Hamiltonian H_l = -T/2 + diag(l(l+1)/(2 r^2) + v) (T [n_r][n_r] symmetric,
  * v = -Z/r + v_gs) is formed on the device and all n_l are diagonalised by
