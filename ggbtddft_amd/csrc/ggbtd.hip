@@ -261,8 +261,9 @@ static __device__ __forceinline__ const double *kin_ref_row(const KinRef &kr, in
 #ifndef KIN_NW
 #define KIN_NW 8
 #endif
-// waves 0..3 finish accumulator rows 0..3 of every tile after the K split
-static_assert(KIN_NW >= 4 && KIN_NW <= 16, "4 to 16 waves per narrow work-group");
+// waves 0..3 finish accumulator rows 0..3 of every tile after the K split, and wave 4 stores
+// (alpha, beta) meanwhile
+static_assert(KIN_NW >= 5 && KIN_NW <= 16, "5 to 16 waves per narrow work-group");
 #define KIN_NARROW_WG (64 * KIN_NW)
 // Panel form: one work-group takes the 16 TA eigen rows a0 .. a0 + 16 TA - 1 as
 // TA tiles with interleaved rows (row ar of tile t is a = a0 + TA ar + t).  A
