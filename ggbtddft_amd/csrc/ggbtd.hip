@@ -422,7 +422,7 @@ static __host__ __device__ __forceinline__ size_t kin_qt_index(size_t l, size_t 
 // pass 1.  Within a wave the K order is permuted (lane kr of MFMA j in chunk u
 // takes a = k0 + 16u + 4kr + j) so that each lane reads 4 consecutive a of Q
 // and of planar Y as one vector.  Q and Y are zero beyond nkeep up to nk_max
-// (host padding, zeroed Y), so the loop runs to nkeep rounded up to 16
+// (host padding; Y from ggb_create or set_variant), so the loop runs to nkeep rounded up to 16
 // without per-element guards; rows i >= N and columns c >= C read row/column
 // 0 and are not stored.
 #ifndef KIN_KU2
@@ -1034,8 +1034,8 @@ __global__ __launch_bounds__(WG) void k_kin_bwd_tiled(const float *__restrict__ 
     const int ia = i0 + am;
     const int colb = n0 + bn;
     const bool bok = (colb >> 1) < C;
-    // the tables and Y are zero from nkeep up to nk_max: runs of AV, BV (<= 16,
-    // dividing 16) are wholly inside or outside [0, nk_max)
+    // the tables and Y are zero from nkeep up to nk_max (Y from ggb_create or set_variant): runs of AV, BV
+    // (<= 16, dividing 16) are wholly inside or outside [0, nk_max)
     float ra[AV], rb[BV];
     auto load = [&](int k0) {
         const bool oka = ia < N && k0 + ak < nk_max;
@@ -5446,6 +5446,27 @@ extern "C" int ggb_spectrum_noalloc(int32_t device, const double *signal, int32_
                        power, intensity, "ggb_spectrum_noalloc");
 }
 
+// k_kin32 keeps Y as [l][c][a] complex, the other mixed passes as [l][c][re, im][a].  The latter read Y's
+// padding (a >= nkeep) and never store it: after k_kin32 it holds values of earlier orbitals, and
+// an infinity or NaN among them would outlive an upload of new ones, so it is cleared.
+static bool kin_y_complex(const ggb_ctx *ctx) {
+    return ctx->p.precision == 1 && kin_variant(ctx) == GGB_KIN_TILED16 && kin32_better(ctx);
+}
+__global__ __launch_bounds__(WG) void k_clear(float4 *x, size_t n) {
+    const size_t k = (size_t)blockIdx.x * WG + threadIdx.x;
+    if (k < n) x[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+static int set_variant(ggb_ctx *ctx, int variant) {
+    const bool was = kin_y_complex(ctx);
+    ctx->kin_variant = variant;
+    if (!was || kin_y_complex(ctx)) return GGB_OK;
+    const size_t n = (size_t)ctx->p.n_l * ctx->C * ctx->p.nk_max / 2;  // nk_max is a multiple of 16
+    HIPCHK(ctx, hipSetDevice(ctx->p.device));
+    k_clear<<<(unsigned)((n + WG - 1) / WG), WG, 0, ctx->stream>>>(reinterpret_cast<float4 *>(ctx->Y), n);
+    HIPCHK(ctx, hipGetLastError());
+    return GGB_OK;
+}
+
 extern "C" int ggb_set_kinetic_variant(ggb_ctx *ctx, int32_t variant) {
     if (!ctx) return GGB_E_ARG;
     const bool split = ctx->p.precision == 2;
@@ -5455,8 +5476,7 @@ extern "C" int ggb_set_kinetic_variant(ggb_ctx *ctx, int32_t variant) {
         (!split && variant == GGB_KIN_SPLIT16))
         return fail(ctx, GGB_E_ARG, "ggb_set_kinetic_variant: unknown or unsupported variant");
     if (variant != ctx->kin_variant) drop_graph(ctx);
-    ctx->kin_variant = variant;
-    return GGB_OK;
+    return set_variant(ctx, variant);
 }
 
 extern "C" int ggb_autotune(ggb_ctx *ctx, int32_t reps, int32_t *chosen, double *ms) {
@@ -5479,8 +5499,8 @@ extern "C" int ggb_autotune(ggb_ctx *ctx, int32_t reps, int32_t *chosen, double 
     const int first = ctx->p.precision == 2 ? GGB_KIN_SPLIT16 : GGB_KIN_NARROW;
     const int last = ctx->p.precision == 2 ? GGB_KIN_SPLIT16 : ctx->p.precision ? GGB_KIN_TILED32 : GGB_KIN_TILED16;
     for (int v = first; v <= last && e == hipSuccess && rc == GGB_OK; ++v) {
-        ctx->kin_variant = v;
-        rc = launch_kinetic(ctx);  // warm-up
+        rc = set_variant(ctx, v);
+        if (rc == GGB_OK) rc = launch_kinetic(ctx);  // warm-up
         if (rc == GGB_OK) e = hipEventRecord(e0, ctx->stream);
         for (int r = 0; r < reps && rc == GGB_OK && e == hipSuccess; ++r) rc = launch_kinetic(ctx);
         if (rc == GGB_OK && e == hipSuccess) e = hipEventRecord(e1, ctx->stream);
@@ -5499,7 +5519,8 @@ extern "C" int ggb_autotune(ggb_ctx *ctx, int32_t reps, int32_t *chosen, double 
     if (e1) (void)hipEventDestroy(e1);
     (void)hipFree(saved);
     if (rc == GGB_OK && e != hipSuccess) rc = fail(ctx, GGB_E_HIP, std::string("ggb_autotune: ") + hipGetErrorString(e));
-    ctx->kin_variant = (rc == GGB_OK) ? best : prev;
+    const int rv = set_variant(ctx, rc == GGB_OK ? best : prev);
+    if (rc == GGB_OK) rc = rv;
     if (rc == GGB_OK && chosen) *chosen = best;
     if (rc == GGB_OK && ms)
         for (int v = 0; v < GGB_KIN_NVARIANT; ++v) ms[v] = t[v];
