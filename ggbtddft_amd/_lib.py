@@ -23,7 +23,7 @@ EXPORTS = ("ggb_abi_version", "ggb_create", "ggb_upload_static", "ggb_upload_orb
            "ggb_spectrum", "ggb_set_kinetic_variant", "ggb_autotune", "ggb_ground_state",
            "ggb_set_channels", "ggb_get_channels", "ggb_spectrum_noalloc", "ggb_group_create",
            "ggb_group_run", "ggb_group_last_error", "ggb_group_destroy", "ggb_propagator_tables",
-           "ggb_debug_ground_state", "ggb_last_error", "ggb_destroy")
+           "ggb_debug_ground_state", "ggb_debug_forms", "ggb_last_error", "ggb_destroy")
 KIN_VARIANTS = ("default", "narrow", "tiled16", "tiled32", "split16")
 NPHASE = 7
 PHASES = ("half_potential_laser", "kinetic_qt", "kinetic_q", "laser_half_potential_obs",
@@ -93,6 +93,8 @@ def load():
     lib.ggb_download_potential.argtypes = [vp, _dp]
     lib.ggb_debug_substep.restype = ctypes.c_int
     lib.ggb_debug_substep.argtypes = [vp, ctypes.c_int32, ctypes.c_int32]
+    lib.ggb_debug_forms.restype = ctypes.c_int
+    lib.ggb_debug_forms.argtypes = [vp, _ip]
     lib.ggb_set_timing.restype = ctypes.c_int
     lib.ggb_set_timing.argtypes = [vp, ctypes.c_int32]
     lib.ggb_get_timing.restype = ctypes.c_int

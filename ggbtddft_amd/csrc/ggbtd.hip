@@ -4244,6 +4244,20 @@ static void launch_angular(ggb_ctx *ctx, int step, const int *cur = nullptr) {
 // launched on its own
 static hipError_t no_mark_k(int) { return hipSuccess; }
 
+// forms of the two potential products (ggb_debug_forms)
+enum { POT_ONE = 1, POT_TILES = 2, POT_PANELS = 3 };  // moments in the density's launch, 16 x 16 tiles, panels
+static int moment_form(const ggb_ctx *ctx) {
+    const ggb_problem &p = ctx->p;
+    const int ntl = (p.n_har + 15) / 16;
+    const double nmom = (double)((p.n_r + 15) / 16) * ntl * p.n_inst;
+    if ((double)p.n_r * p.n_theta * p.n_orb * p.n_inst * ntl <= MOM_MAX_READS && nmom <= MOM_MAX_BLOCKS) return POT_ONE;
+    return nmom >= TGW_MIN_MOM ? POT_PANELS : POT_TILES;
+}
+static int dv_form(const ggb_ctx *ctx) {
+    const ggb_problem &p = ctx->p;
+    return dv_panels((double)((p.n_r + 15) / 16) * p.n_inst, (p.n_theta + 15) / 16) ? POT_PANELS : POT_TILES;
+}
+
 // mk(0) after the density kernel, mk(1) after the Hartree scans (timing events)
 template <typename MarkK = hipError_t (*)(int)>
 static int launch_potential(ggb_ctx *ctx, const ObsArgs *ob = nullptr, MarkK mk = no_mark_k, const ChanArgs *chan = nullptr) {
@@ -4262,8 +4276,8 @@ static int launch_potential(ggb_ctx *ctx, const ObsArgs *ob = nullptr, MarkK mk 
         const dim3 gr(nrho + nobs + nchan, p.n_inst);
         const int ntl = (nh + 15) / 16;
         const unsigned nmom = (unsigned)((N + 15) / 16 * ntl);
-        // moments in the same launch
-        const bool one = (double)N * Nth * p.n_orb * p.n_inst * ntl <= MOM_MAX_READS && (double)nmom * p.n_inst <= MOM_MAX_BLOCKS;
+        const int form = moment_form(ctx);
+        const bool one = form == POT_ONE;
         const RhoArgs ra{ctx->dens, ctx->occ, ctx->rho_frozen, ctx->r, ctx->wr, ctx->omega, one ? nullptr : ctx->rho_u, ctx->vxc,
                          N, Nth, ctx->ang.h, ctx->ang.hq, p.n_orb, ctx->active};
         if (one) {
@@ -4291,7 +4305,7 @@ static int launch_potential(ggb_ctx *ctx, const ObsArgs *ob = nullptr, MarkK mk 
             gq.N = N;
             gq.K = Nth;
             QmomEpi eq{ctx->q, N, nh};
-            if ((double)nmom * p.n_inst >= TGW_MIN_MOM) {
+            if (form == POT_PANELS) {
                 gq.A = ctx->PL;  // the same table as [j][L]: the 16 lanes of a K row read 16 consecutive L
                 gq.sam = 1;
                 gq.sak = nh;
@@ -4324,7 +4338,7 @@ static int launch_potential(ggb_ctx *ctx, const ObsArgs *ob = nullptr, MarkK mk 
     gv.K = p.interacting ? nh : 0;
     DvEpi ev{ctx->vxc, ctx->v_gs, ctx->mask, ctx->dv, ctx->phase, N, Nth, p.interacting, p.precision, p.dt};
     const int ntj = (Nth + 15) / 16;
-    if (dv_panels((double)((N + 15) / 16) * p.n_inst, ntj)) {
+    if (dv_form(ctx) == POT_PANELS) {
         k_tile_gemm_wide<DvEpi, false><<<dim3((N + 15) / 16, (ntj + TGW_T - 1) / TGW_T, p.n_inst), WG, 0, st>>>(gv, ev);
     } else {
         k_tile_gemm<<<dim3((Nth + 15) / 16, (N + 15) / 16, p.n_inst), WG, 0, st>>>(gv, ev);
@@ -4377,10 +4391,9 @@ static void launch_kin64_t(ggb_ctx *ctx, int pass, hipEvent_t e0, hipEvent_t e1)
     g.n_orb = p.n_orb;
     const int rows = pass ? p.n_r : p.nk_max;
     const dim3 grid((rows + 16 * TA - 1) / (16 * TA), (2 * g.C + 16 * TB - 1) / (16 * TB), p.n_l);
-    if (pass)
-        kin_launch(k_kin64<1, TA, TB, NW>, grid, 64 * NW, ctx->stream, e0, e1, g);
-    else
-        kin_launch(k_kin64<0, TA, TB, NW>, grid, 64 * NW, ctx->stream, e0, e1, g);
+    if constexpr (NW == 4)  // eight waves: pass 0 only (kin64_shape)
+        if (pass) return kin_launch(k_kin64<1, TA, TB, NW>, grid, 64 * NW, ctx->stream, e0, e1, g);
+    kin_launch(k_kin64<0, TA, TB, NW>, grid, 64 * NW, ctx->stream, e0, e1, g);
 }
 
 // Shape of the FP64 passes by the 16 x 16 output tiles of a pass.  NARROW, one column tile, and up to
@@ -4395,23 +4408,31 @@ static void launch_kin64_t(ggb_ctx *ctx, int pass, hipEvent_t e0, hipEvent_t e1)
 // order in all of them.
 //   Pass 0 on one column tile and long rows: k split over eight waves instead of four, with more of the
 // table's rows in flight (argon N = 512, 7 columns 23.8 -> 23.2 us, neon N = 768 67.0 -> 65.3; shorter rows
-// lose: N = 384 12.3 -> 12.7, N = 300 10.5 -> 11.1).
+// lose: N = 384 12.3 -> 12.7, N = 300 10.5 -> 11.1; three lanes side by side, helium N = 512, 5 columns among
+// them, 25.85 -> 25.73 ms for 120 steps).  There a sum is of eight parts instead of four: up to 8 columns
+// and from 9 on differ in rounding.
 #define K64_EIGHT_N 448
 #define K64_TILES_32 2000
 #define K64_TILES_64 7200
 #define K64_TABLE_BYTES 200e6
-static void launch_kin64(ggb_ctx *ctx, int pass, hipEvent_t e0, hipEvent_t e1) {
+struct KinShape {
+    int ta, tb, nw;  // 16 ta rows by 16 tb real columns, waves per work-group
+};
+static KinShape kin64_shape(const ggb_ctx *ctx, int pass) {
     const ggb_problem &p = ctx->p;
     const int nct = (2 * ctx->C + 15) / 16, rows = pass ? p.n_r : p.nk_max;
     const double tiles = (double)((rows + 15) / 16) * nct * p.n_l;
-    if (pass == 0 && nct == 1 && p.n_r >= K64_EIGHT_N)
-        launch_kin64_t<2, 1, 8>(ctx, pass, e0, e1);
-    else if (ctx->kin_variant == GGB_KIN_NARROW || nct == 1 || tiles < K64_TILES_32)
-        launch_kin64_t<2, 1>(ctx, pass, e0, e1);
-    else if (tiles < K64_TILES_64 && 8.0 * p.n_l * p.n_r * p.nk_max < K64_TABLE_BYTES)
-        launch_kin64_t<4, 1>(ctx, pass, e0, e1);
-    else
-        launch_kin64_t<4, 2>(ctx, pass, e0, e1);
+    if (pass == 0 && nct == 1 && p.n_r >= K64_EIGHT_N) return {2, 1, 8};
+    if (ctx->kin_variant == GGB_KIN_NARROW || nct == 1 || tiles < K64_TILES_32) return {2, 1, 4};
+    if (tiles < K64_TILES_64 && 8.0 * p.n_l * p.n_r * p.nk_max < K64_TABLE_BYTES) return {4, 1, 4};
+    return {4, 2, 4};
+}
+static void launch_kin64(ggb_ctx *ctx, int pass, hipEvent_t e0, hipEvent_t e1) {
+    const KinShape s = kin64_shape(ctx, pass);
+    if (s.nw == 8) return launch_kin64_t<2, 1, 8>(ctx, pass, e0, e1);
+    if (s.ta == 2) return launch_kin64_t<2, 1>(ctx, pass, e0, e1);
+    if (s.tb == 1) return launch_kin64_t<4, 1>(ctx, pass, e0, e1);
+    launch_kin64_t<4, 2>(ctx, pass, e0, e1);
 }
 
 // e0/e1 (optional): events stamped with the start and end of the pass's
@@ -4457,6 +4478,11 @@ static bool kin32_better(const ggb_ctx *ctx) {
     return wg <= 256 || (wg <= K32_MAX_WG && fill < 0.95) || (wg <= 4 * 256 && fill < 0.66);
 }
 
+// whether k_kin32 runs (its Y is laid out differently: set_variant)
+static bool kin_y_complex(const ggb_ctx *ctx) {
+    return ctx->p.precision == 1 && kin_variant(ctx) == GGB_KIN_TILED16 && kin32_better(ctx);
+}
+
 // Shape by the number of 16 x 16 output tiles of a pass.  Up to about four waves per SIMD one tile per
 // wave (neon, 32 columns, 3724 tiles: 25 / 22 us; two rows of tiles 27 / 21, four 31 / 25); with more,
 // operand traffic counts: 2 x 2 tiles for one pair of column tiles (krypton, 13 columns, 7372 tiles:
@@ -4464,19 +4490,23 @@ static bool kin32_better(const ggb_ctx *ctx) {
 // of 1, 2 or 4 tiles, and its last one is partly empty.  Against 4 tiles, 2 cost 1.1 to 1.2 times as much
 // per tile and 1 up to half as much again, so argon N = 512 (28 row tiles of 32) takes 4 (84 columns 168 us, 2: 187, 1: 206)
 // and N = 300 (17 of 32, or of 24) takes 2 (140 columns 87 us, 4: 108, 1: 94).
-static void launch_kin32(ggb_ctx *ctx, int pass, const KinRef &ref, hipEvent_t e0, hipEvent_t e1) {
+static KinShape kin32_shape(const ggb_ctx *ctx, int pass) {
     const int nct = (2 * ctx->C + 15) / 16, rt = ((pass ? ctx->p.n_r : ctx->p.nk_max) + 15) / 16;
     const long tiles = (long)(ctx->p.nk_max / 16) * nct * ctx->p.n_l;
-    if (tiles <= 4500) return launch_kin32_t<1, 1>(ctx, pass, ref, e0, e1);
-    if (nct <= 2) return launch_kin32_t<2, 2>(ctx, pass, ref, e0, e1);
+    if (tiles <= 4500) return {1, 1, 4};
+    if (nct <= 2) return {2, 2, 4};
     // row tiles computed, with the cost of each
     const double c4 = (rt + 15) / 16 * 16, c2 = 1.2 * ((rt + 7) / 8 * 8), c1 = 1.45 * ((rt + 3) / 4 * 4);
-    if (c4 <= c2 && c4 <= c1)
-        launch_kin32_t<4, 1>(ctx, pass, ref, e0, e1);
-    else if (c2 <= c1)
-        launch_kin32_t<2, 1>(ctx, pass, ref, e0, e1);
-    else
-        launch_kin32_t<1, 1>(ctx, pass, ref, e0, e1);
+    if (c4 <= c2 && c4 <= c1) return {4, 1, 4};
+    if (c2 <= c1) return {2, 1, 4};
+    return {1, 1, 4};
+}
+static void launch_kin32(ggb_ctx *ctx, int pass, const KinRef &ref, hipEvent_t e0, hipEvent_t e1) {
+    const KinShape s = kin32_shape(ctx, pass);
+    if (s.ta == 1) return launch_kin32_t<1, 1>(ctx, pass, ref, e0, e1);
+    if (s.ta == 4) return launch_kin32_t<4, 1>(ctx, pass, ref, e0, e1);
+    if (s.tb == 1) return launch_kin32_t<2, 1>(ctx, pass, ref, e0, e1);
+    launch_kin32_t<2, 2>(ctx, pass, ref, e0, e1);
 }
 
 static void launch_kinetic_mixed(ggb_ctx *ctx, int pass, bool fresh, hipEvent_t e0, hipEvent_t e1) {
@@ -5222,6 +5252,25 @@ extern "C" int ggb_selftest_mfma(int32_t device, double *out) {
     return e == hipSuccess ? GGB_OK : GGB_E_HIP;
 }
 
+extern "C" int ggb_debug_forms(ggb_ctx *ctx, int32_t *forms) {
+    if (!ctx) return GGB_E_ARG;
+    if (!forms) return fail(ctx, GGB_E_ARG, "ggb_debug_forms: null argument");
+    const int var = kin_variant(ctx);
+    for (int pass = 0; pass < 2; ++pass) {
+        int kind = var == GGB_KIN_SPLIT16 ? 4 : var == GGB_KIN_NARROW ? 1 : 2;
+        KinShape s{0, 0, 0};
+        if (ctx->p.precision == 0)
+            kind = 0, s = kin64_shape(ctx, pass);
+        else if (kin_y_complex(ctx))
+            kind = 3, s = kin32_shape(ctx, pass);
+        forms[pass] = 1000 * kind + 100 * s.nw + 10 * s.ta + s.tb;
+    }
+    forms[2] = ctx->p.interacting ? moment_form(ctx) : 0;
+    forms[3] = dv_form(ctx);
+    forms[4] = ctx->ang.wave ? 0 : ctx->ang.nt;
+    return GGB_OK;
+}
+
 extern "C" int ggb_set_timing(ggb_ctx *ctx, int32_t mode) {
     if (!ctx) return GGB_E_ARG;
     if (mode < 0 || mode > 2) return fail(ctx, GGB_E_ARG, "ggb_set_timing: mode must be 0, 1 or 2");
@@ -5449,9 +5498,6 @@ extern "C" int ggb_spectrum_noalloc(int32_t device, const double *signal, int32_
 // k_kin32 keeps Y as [l][c][a] complex, the other mixed passes as [l][c][re, im][a].  The latter read Y's
 // padding (a >= nkeep) and never store it: after k_kin32 it holds values of earlier orbitals, and
 // an infinity or NaN among them would outlive an upload of new ones, so it is cleared.
-static bool kin_y_complex(const ggb_ctx *ctx) {
-    return ctx->p.precision == 1 && kin_variant(ctx) == GGB_KIN_TILED16 && kin32_better(ctx);
-}
 __global__ __launch_bounds__(WG) void k_clear(float4 *x, size_t n) {
     const size_t k = (size_t)blockIdx.x * WG + threadIdx.x;
     if (k < n) x[k] = make_float4(0.f, 0.f, 0.f, 0.f);

@@ -183,6 +183,16 @@ int ggb_download_potential(ggb_ctx *ctx, double *dv);
  * current state.  `step` selects the field sample. */
 int ggb_debug_substep(ggb_ctx *ctx, int32_t which, int32_t step);
 
+/* The forms of the kernels that this context's steps launch, for checks that
+ * mean to compare two of them.  forms[0], forms[1]: kinetic passes 0 and 1, as
+ * 1000 kind + 100 waves + 10 TA + TB (panels of 16 TA rows by 16 TB real
+ * columns), kind 0 the FP64 kernel, 1 the narrow mixed ones, 2 the 64 x 128
+ * mixed tiles, 3 the few-column mixed kernel, 4 the split form (kinds 1, 2, 4:
+ * no shape).  forms[2]: moments, 0 none, 1 in the density's launch, 2 tiles, 3
+ * panels; forms[3]: potential, 2 tiles, 3 panels; forms[4]: angular kernel, 0 a
+ * wave per tile, else column tiles per work-group. */
+int ggb_debug_forms(ggb_ctx *ctx, int32_t forms[5]);
+
 /* Replay the step loop of ggb_run from a hipGraph of `steps` steps (0 =
  * plain stream launches, the default).  The graph is captured on the next
  * ggb_run and re-captured after any call that may move a buffer; runs with
