@@ -6304,9 +6304,9 @@ static int ground_state(const ggb_gs_problem *p, const int32_t *shell_l, const d
         for (it = 1; it <= p->max_iter; ++it) {
             a.first = it == 1;
             k_gs_potential<<<1, GS_WG, 0, st>>>(a);
-            // one set of teams of this process on the device at a time
-            static std::mutex teams;
-            std::unique_lock<std::mutex> alone(teams, std::defer_lock);
+            // one set of teams of this process on a device at a time
+            static std::mutex teams[64];
+            std::unique_lock<std::mutex> alone(teams[p->device & 63], std::defer_lock);
             if (team > 1) alone.lock();
             auto sweeps = [&](bool in_team) {
                 const size_t lds = in_lds ? ldsu : lds5;
