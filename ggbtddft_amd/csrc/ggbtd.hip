@@ -14,9 +14,11 @@
 //
 // Kernels, launch order per step:
 //   k_angular<mode 0>   Vh, Le, Lo                       grid (N / 8 NT, C)
-//   k_kin64<0>          Y = e^{-i lam dt} Q^T psi (FP64) grid (nk/32, 2C/32, n_l)
-//   k_kin64<1>          psi = Q Y                        grid (N/32,  2C/32, n_l)
-//   (mixed form: k_kin_fwd / k_kin_bwd, 16-wide tiles, or k_kin_*_dma / _tiled, 64 x 128 tiles)
+//                       (FP64, many tiles: k_angular_wave, grid (N / 32, C))
+//   k_kin64<0>          Y = e^{-i lam dt} Q^T psi (FP64) grid (nk / 16 TA, 2C / 16 TB, n_l), (TA, TB) by size
+//   k_kin64<1>          psi = Q Y                        grid (N / 16 TA,  2C / 16 TB, n_l)
+//   (mixed form: k_kin_fwd / k_kin_bwd, 16-wide tiles; k_kin32, small tiles per wave; or
+//   k_kin_*_dma / _tiled, 64 x 128 tiles)
 //   k_angular<mode 1>   Lo, Le, Vh, |B psi|^2, observable partials
 //   k_rho               rho_u = sum occ |Psi|^2, v_xc; observable sums, channel dipoles
 //   k_tile_gemm<Qmom>   multipole moments q_L = P_L^T rho_u (small contexts: both in k_rho_mom)
@@ -519,9 +521,9 @@ __global__ __launch_bounds__(KIN_NARROW_WG) void k_kin_bwd(const float *__restri
 //    covers whole 128-byte lines; component-wise loads touched each line twice.
 // What bounds it: HBM up to about 16 columns (the table is read once), the FP64
 // matrix pipe beyond.  At argon size (N = 512, 65 l) passes 0 / 1 take, against the
-// LDS-tiled kernels that ran from 9 columns on: 14 columns 26 / 27 us (91 / 122),
-// 28 columns 44 / 45 us (94 / 124), 224 columns 237 / 234 us (369 / 349, 53 TFLOP/s);
-// krypton (N = 768, 97 l, 13 columns) 87 / 84 us (258 / 293).
+// LDS-tiled kernels that ran from 9 columns on: 14 columns 27 / 27 us (91 / 122),
+// 28 columns 45 / 47 us (94 / 124), 224 columns 233 / 234 us (369 / 349, 54 TFLOP/s);
+// krypton (N = 768, 97 l, 13 columns) 91 / 81 us (258 / 293).
 // ---------------------------------------------------------------------------
 typedef double d2_t __attribute__((ext_vector_type(2)));
 struct Kin64Args {
@@ -3406,7 +3408,7 @@ __global__ __launch_bounds__(WG) void k_spec_fd8(const double *__restrict__ x,
 }
 
 #define SF_W 8       // columns of a tile (128-byte runs of a strided pass)
-#define SF_RMAX 9    // bits of a pass at most: 512 x 9 complex values are 74 KB of LDS
+#define SF_RMAX 9    // bits of a pass at most: 512 x 9 complex values and 512 roots are 80 KB of LDS
 #define SF_EPT 16    // values per thread at most: 512 x 8 / 256
 struct SpecFft {
     double2 *buf;         // transforms of length 2^m
@@ -5955,11 +5957,11 @@ static __device__ void gs_colsum(const TE *M, const double *x, int N, double *ou
 // read all of T, Q0 and Q0^T through one CU: 99 us a pass at N = 512, 2.4 ms an
 // iteration.  Now a team of work-groups shares the rows of each product, 16 rows a
 // work-group where the device holds all teams, and only product rows are exchanged.
-// An argon iteration at N = 512 takes 0.59 ms (2.38), a krypton one at N = 768 0.94 ms
+// The sweeps of an argon iteration at N = 512 take 0.56 ms (2.38), of a krypton one at N = 768 1.09 ms
 // (7.37); every sum keeps its terms and their order, so the results are the same bit
 // for bit.  What bounds it is the latency of a phase (a product of 16 rows, a
-// store and a load across the device), not its bytes.  Below N = 128 one work-group alone
-// is as fast (He, N = 96: 11.2 against 15.8 ms in a team) and keeps gs_colsum.
+// store and a load across the device), not its bytes.  Below N = 144
+// (GS_TEAM_MIN_N) a group stays in one work-group (He, N = 96: 11.2 against 15.8 ms in a team) and keeps gs_colsum.
 //   A phase: each work-group writes its rows to one of three exchange slots, and
 // every thread polls the values it needs until none is empty: there are no flags and
 // no barrier over the team.  The slot of phase n - 1 is emptied again, each
